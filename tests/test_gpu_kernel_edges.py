@@ -1,0 +1,40 @@
+"""Kernels at the sizes where their work splits: waves and tiles that are
+exactly full, one over and one short, and loads that gather in one place."""
+import numpy as np
+import pytest
+
+from demso_amd import api
+from demso_amd import scene as sc
+from helpers import dev
+
+pytestmark = pytest.mark.gpu
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 257, 5000])
+def test_image_of_discs_past_its_end(gpu_ctx, oracle, n):
+    """Discs above and right of the image clamp to its last pixel, which the
+    highest index among them owns (some discs lie inside, some across)."""
+    s = sc.settling(seed=n, side=71)
+    s.pos, s.type, s.radius = s.pos[:n].copy(), s.type[:n], s.radius[:n].copy()
+    rng = np.random.default_rng(n)
+    lx, ly = s.instances[0].box
+    s.pos[:, 0] = rng.uniform(0.0, 1.3 * lx, n)
+    s.pos[:, 1] = rng.uniform(0.8 * ly, 3.0 * ly, n)
+    s.pos[n // 2] = (lx * (1 - 1e-3), ly * (1 - 1e-3))
+    zero = np.zeros(n, np.float32)
+    gpu_ctx.load_scene(s)
+    rp = api.render_params(s, image_height=300, view_rotations=False)
+    import torch
+
+    img = torch.zeros((rp["image_dim"][1], rp["image_dim"][0], 4), dtype=torch.uint8, device="cuda")
+    api.plotParticles(gpu_ctx, img, dev(s.pos), dev(zero), dev(s.type), n, rp, dev(zero), radius=dev(s.radius))
+    want = oracle.plot(s, rp, s.pos, zero, s.type, zero, radius=s.radius)
+    assert np.array_equal(img.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("n", [1, 255, 1023, 1025, 65537])
+def test_pressure_scale_blocks(gpu_ctx, n):
+    v = np.random.default_rng(n).normal(size=n).astype(np.float32)
+    for at in (0, n // 2, n - 1):
+        w = v.copy()
+        w[at] = 9.5
+        assert api.updatePressureScale(gpu_ctx, dev(w), n) == 9.5
