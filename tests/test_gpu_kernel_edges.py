@@ -5,9 +5,12 @@ import pytest
 
 from demso_amd import api
 from demso_amd import scene as sc
-from helpers import dev
+from helpers import bits_equal, dev
 
 pytestmark = pytest.mark.gpu
+
+FIELDS = ("hash", "index", "cellStart", "cellEnd", "id", "type", "loc", "pos", "vel", "theta", "omega", "acc",
+          "alpha", "pressure")
 
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 257, 5000])
 def test_image_of_discs_past_its_end(gpu_ctx, oracle, n):
@@ -38,3 +41,37 @@ def test_pressure_scale_blocks(gpu_ctx, n):
         w = v.copy()
         w[at] = 9.5
         assert api.updatePressureScale(gpu_ctx, dev(w), n) == 9.5
+
+
+def swept_row(n, seed=2):
+    """n discs over two wide cell rows, a few of which hop between them every
+    step, so that each hop shifts the slots of all the discs between."""
+    s = sc.column_collapse(seed=seed, cols=n, n=n, box=(n * 0.012, 0.05), pitch=0.0115, jitter=0.0, dt=1e-4)
+    s.pos[:, 1] = np.where(np.arange(n) % 2 == 0, 0.008, 0.025).astype(np.float32)
+    rng = np.random.default_rng(seed)
+    hop = rng.choice(n, max(2, n // 500), replace=False)
+    s.vel[hop, 1] = np.where(s.pos[hop, 1] < 0.011, 100.0, -100.0)
+    return s
+
+
+@pytest.mark.parametrize("n", [64, 2047, 2048, 2049, 4097, 12289])
+def test_long_lists_equal_radix(gpu_ctx, n):
+    """Few movers that shift whole tiles of stayers: the in-place re-sort's
+    lists against the radix sort."""
+    s = swept_row(n)
+    a, b = api.Simulation(gpu_ctx, s), api.Simulation(gpu_ctx, s)
+    a.set_sort_mode(1)
+    b.set_sort_mode(2)
+    try:
+        listed = []
+        for _ in range(4):
+            a.step(2)
+            b.step(2)
+            listed.append(b.resort_counts()["listed"])
+            da, db = a.download(), b.download()
+            for k in FIELDS:
+                assert bits_equal(da[k], db[k]), k
+        assert max(listed) > n // 8
+    finally:
+        a.close()
+        b.close()
