@@ -10,6 +10,8 @@
 
 #include <math.h>
 
+#include <type_traits>
+
 #pragma clang fp contract(off)
 
 namespace dem {
@@ -536,6 +538,54 @@ constexpr int kBatchN = 1;
 // instance with several rows, or an ensemble of instances.
 constexpr int kOneMat = 0, kManyMat = 1, kInstances = 2;
 
+// The radii of the contact-list walk's marks are taken this much longer.
+constexpr float kReach = 1.0f + 0x1p-18f;
+
+// w[y] = 2 w[y] + !(x[y] > limit) for the three rows: each comparison's carry
+// is added with the shift (the compiler takes a select and a shift-or).  A
+// lane mask that a vector instruction wrote may be read by another only two
+// instructions later on gfx950, so the three comparisons come first.
+__device__ __forceinline__ void shift_in(uint32_t (&w)[3], const float (&x)[3], float limit) {
+  uint64_t m0, m1, m2;
+  asm("v_cmp_ngt_f32_e64 %3, %6, %9\n\t"
+      "v_cmp_ngt_f32_e64 %4, %7, %9\n\t"
+      "v_cmp_ngt_f32_e64 %5, %8, %9\n\t"
+      "v_addc_co_u32_e64 %0, vcc, %0, %0, %3\n\t"
+      "v_addc_co_u32_e64 %1, vcc, %1, %1, %4\n\t"
+      "v_addc_co_u32_e64 %2, vcc, %2, %2, %5"
+      : "+&v"(w[0]), "+&v"(w[1]), "+&v"(w[2]), "=&s"(m0), "=&s"(m1), "=&s"(m2)
+      : "v"(x[0]), "v"(x[1]), "v"(x[2]), "s"(limit)
+      : "vcc");
+}
+
+// The contact-list walk's windows, one set a wave in LDS: the positions and
+// radii of the sorted particles [w0, w1) that hold the candidates of all the
+// wave's lanes in a neighbour row (the lanes' ranges follow each other in
+// sorted order, so a row's window is a little longer than a wave).  Loaded
+// once, coalesced; each lane then walks its candidates in LDS.  The vector
+// cache looks up one line a cycle, and walking the candidates through it
+// (585 lookups a wave at 4M settling discs, where it was busy 93% of the
+// kernel's time) bound the kernel.  With the windows and the shorter marks
+// it takes 49.9 us there (58.7), 150 us on the 4M dense pack (172), 136 us on
+// the 8.2M-disc ensemble (149).  Entries: three rows of kWindow, then
+// kWindowSlack more, as a lane with few candidates reads on past its row's.
+// Eight waves a SIMD fit (32 x 4,864 bytes of 160 KB).
+constexpr uint32_t kWindow = 128, kWindowSlack = 64;
+struct WaveWindow {
+  float2 pos[3 * kWindow];
+  float r[3 * kWindow + kWindowSlack];  // (reads of pos past its end land here)
+};
+static_assert(sizeof(WaveWindow) == 4864, "eight waves a SIMD");
+
+// This wave's windows in the block's dynamic LDS (window_bytes(block)).
+extern __shared__ __attribute__((aligned(16))) unsigned char dem_windows[];
+__device__ __forceinline__ WaveWindow* wave_window() {
+  return reinterpret_cast<WaveWindow*>(dem_windows) + threadIdx.x / (uint32_t)kWave;
+}
+inline size_t window_bytes(int mode, int block) {
+  return mode == kList ? sizeof(WaveWindow) * (size_t)((block + kWave - 1) / kWave) : 0;
+}
+
 // kUni: every lane of the wave has material row t_uni (a wave-uniform value,
 // so the material row and the instance geometry are scalar loads and the
 // grid arithmetic scalar); the ensemble kernels take this path for every
@@ -547,7 +597,8 @@ __device__ __forceinline__ void collide_particle(const StepConst& c, uint32_t i,
                                                  const uint32_t* __restrict__ cell_start,
                                                  const uint32_t* __restrict__ cell_end, uint32_t n, Own& own,
                                                  const ControlOut& ctl, float& fx_out, float& fy_out,
-                                                 float& moment_out, float& pres_out, uint32_t t_uni = 0) {
+                                                 float& moment_out, float& pres_out, uint32_t t_uni = 0,
+                                                 WaveWindow* win = nullptr) {
   constexpr bool kMulti = kMat == kInstances, kOne = kMat == kOneMat;
   PairCtx q;
   own.t = kOne ? 0u : (kUni ? t_uni : clamp_idx(type[i], c.num_types));
@@ -638,53 +689,162 @@ __device__ __forceinline__ void collide_particle(const StepConst& c, uint32_t i,
           candidate_load<kRadius, kOne, false, kO>(c, j < re[y] ? j : 0u, pos, type, radius, d, cb[y][k]);
         }
     }
-    if (kMode == kList && !c.attract && re[0] - rs[0] <= 64u && re[1] - rs[1] <= 64u && re[2] - rs[2] <= 64u) {
+    if (kMode == kList && (!c.attract || q.den > 0.0) && re[0] - rs[0] <= 64u && re[1] - rs[1] <= 64u &&
+        re[2] - rs[2] <= 64u) {
       // Rows of at most 64 candidates: first one bit per candidate that may
-      // touch (the pair law's own prefilter, from position and radius), then
-      // the law over the set bits of all three rows in row order, so a wave
-      // runs the law as often as its busiest lane has contacts.  Candidates
-      // that exert no force add +0, so skipping them leaves every sum
-      // unchanged; a row's partial sum is flushed when the walk moves on to
-      // a later row.  (With attraction every candidate within reach pulls,
-      // so the rows are walked one candidate at a time instead.)
-      // The three rows are walked together, the k-th candidate of each
-      // loaded at once (three loads in flight; a row already walked
-      // re-reads the particle's own slot, which is never marked).
-      // (the marks are kept as 32-bit halves: bit k of a row's mask is the
-      // same bit for every lane, so setting it is one select and one or)
-      uint32_t hlo[3] = {0u, 0u, 0u}, hhi[3] = {0u, 0u, 0u};
-      const uint32_t len0 = re[0] - rs[0], len1 = re[1] - rs[1], len2 = re[2] - rs[2];
-      const uint32_t L = max(len0, max(len1, len2));
-      // positions k of the rows' k-th candidates, in [k0, k1), marking into
-      // word w (bit k - 32 w)
-      auto mark = [&](uint32_t k0, uint32_t k1, uint32_t (&w)[3], uint32_t wbase) {
-        for (uint32_t k = k0; k < k1; ++k) {
-          Cand b[3];
-          const uint32_t j0 = k < len0 ? rs[0] + k : i, j1 = k < len1 ? rs[1] + k : i, j2 = k < len2 ? rs[2] + k : i;
-          candidate_load<kRadius, kOne, false, kO>(c, j0, pos, type, radius, d, b[0]);
-          candidate_load<kRadius, kOne, false, kO>(c, j1, pos, type, radius, d, b[1]);
-          candidate_load<kRadius, kOne, false, kO>(c, j2, pos, type, radius, d, b[2]);
-          const uint32_t jy[3] = {j0, j1, j2};
-          const uint32_t bit = 1u << (k - wbase);
+      // exert a force (from position and radius), then the law over the set
+      // bits of all three rows in row order, so a wave runs the law as often
+      // as its busiest lane has contacts.  Candidates that exert no force add
+      // +0, so skipping them leaves every sum unchanged; a row's partial sum
+      // is flushed when the walk moves on to a later row.  (An attracting
+      // candidate out of reach adds +0 / den to the pressure: +0 for den > 0;
+      // the 16,290-disc pile's fused step takes 15.7 us this way, 42 one
+      // candidate at a time.)
+      // The three rows are walked together, from the wave's windows in LDS
+      // (WaveWindow) or from global memory.  The walk is most of the kernel's
+      // instructions on sparse states, so each candidate costs as few as
+      // possible: a mark is one comparison shifted into the row's word
+      // (candidate k at bit 31 - k), and the particle itself and the places
+      // past the row's end are cleared afterwards.  A mark may be set without
+      // a contact, never the other way round: where a contact is, the law's
+      // d2 < R^2; d2 here (one rounding less) is within 2^-22 of it, and R
+      // here is R (1 + 2^-18) within 2^-23, so d2 - R^2 rounds to a negative
+      // number, or to at most 2^-125 where the squares underflow; NaN is
+      // marked.
+      // A row's places: its length, and where its second and third cells
+      // start, 8 bits each (an empty cell starts where the next one does, a
+      // flush of an empty sum changes nothing).
+      uint32_t first[3], cut[3];
 #pragma unroll
-          for (int y = 0; y < 3; ++y) {
-            const float rx = b[y].p.x - q.p.x, ry = b[y].p.y - q.p.y;
-            const float d2 = rx * rx + ry * ry;
-            const float R = q.rA + b[y].r;
-            const bool maybe = !(d2 > (R * R) * 1.00000095367431640625f) || R < 1.0842022e-19f;
-            w[y] |= maybe && jy[y] != i ? bit : 0u;
+      for (int y = 0; y < 3; ++y) {
+        const uint32_t c0 = b0[y] == kNoBoundary ? 0u : min(b0[y] - rs[y], 64u);
+        const uint32_t c1 = b1[y] == kNoBoundary ? c0 : min(b1[y] - rs[y], 64u);
+        first[y] = rs[y];
+        cut[y] = (re[y] - rs[y]) | c0 << 8 | c1 << 16;
+      }
+      auto length = [&](int y) { return cut[y] & 0xFFu; };
+      const uint32_t L = max(length(0), max(length(1), length(2)));
+      // At most 2^-125 where a candidate at p with radius r may exert a force.
+      const float reach = q.rA * kReach;
+      auto beyond = [&](auto attract, float2 p, float r) {
+        const float rx = p.x - q.p.x, ry = p.y - q.p.y;
+        const float d2 = __builtin_fmaf(ry, ry, rx * rx);
+        float R = __builtin_fmaf(r, kReach, reach);
+        // (attractSpheres reaches 2.4 times either radius)
+        if constexpr (attract) R = fmaxf(R, (2.4f * kReach) * fmaxf(q.rA, r));
+        return __builtin_fmaf(-R, R, d2);
+      };
+      // The windows, where the whole wave is here and every lane's ranges
+      // lie in them (rows far apart, as around wide empty spaces, do not fit
+      // and are walked in global memory).
+      uint32_t w0[3] = {0u, 0u, 0u}, w1[3] = {0u, 0u, 0u};
+      bool in_win = win && __ballot(true) == ~0ull;
+#pragma unroll
+      for (int y = 0; y < 3; ++y) {
+        const uint64_t some = __ballot(length(y) != 0u);
+        if (some) {
+          const uint32_t end = first[y] + length(y);
+          w0[y] = (uint32_t)__builtin_amdgcn_readlane((int)first[y], __builtin_ctzll(some));
+          w1[y] = (uint32_t)__builtin_amdgcn_readlane((int)end, 63 - __builtin_clzll(some));
+          in_win = in_win && w1[y] - w0[y] <= kWindow &&
+                   __ballot(length(y) && (first[y] < w0[y] || end > w1[y])) == 0;
+        }
+      }
+      if (in_win) {
+        const uint32_t lane = __lane_id();
+        auto stage = [&](uint32_t e) {
+          Cand b[3];
+#pragma unroll
+          for (int y = 0; y < 3; ++y)
+            if (w0[y] + e < w1[y]) candidate_load<kRadius, kOne, false, kO>(c, w0[y] + e, pos, type, radius, d, b[y]);
+#pragma unroll
+          for (int y = 0; y < 3; ++y)
+            if (w0[y] + e < w1[y]) {
+              win->pos[(uint32_t)y * kWindow + e] = b[y].p;
+              win->r[(uint32_t)y * kWindow + e] = b[y].r;
+            }
+        };
+        stage(lane);
+        // what is left of the three windows: usually a few places each, taken
+        // by a third of the wave a row
+        constexpr uint32_t kThird = (uint32_t)kWave / 3u;
+        const uint32_t longest = max(w1[0] - w0[0], max(w1[1] - w0[1], w1[2] - w0[2]));
+        if (longest > (uint32_t)kWave + kThird) {
+          stage((uint32_t)kWave + lane);
+        } else if (longest > (uint32_t)kWave) {
+          const uint32_t y = lane / kThird, e = (uint32_t)kWave + lane % kThird;
+          const uint32_t a = y == 0u ? w0[0] : (y == 1u ? w0[1] : w0[2]), z = y == 0u ? w1[0] : (y == 1u ? w1[1] : w1[2]);
+          if (y < 3u && a + e < z) {
+            Cand b;
+            candidate_load<kRadius, kOne, false, kO>(c, a + e, pos, type, radius, d, b);
+            win->pos[y * kWindow + e] = b.p;
+            win->r[y * kWindow + e] = b.r;
           }
         }
+        // (one wave's LDS instructions execute in order; this keeps the
+        // compiler's order)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int y = 0; y < 3; ++y) first[y] = length(y) ? first[y] : w0[y];  // an entry of the window for each lane
+      }
+      // the window entry of candidate j of row y
+      auto entry = [&](int y, uint32_t j) { return j - w0[y] + (uint32_t)y * kWindow; };
+      // the rows' candidates [k0, k1), marked into w
+      auto mark = [&](auto attract, uint32_t k0, uint32_t k1, uint32_t (&w)[3]) {
+        uint32_t walked = 0;
+        if (in_win) {
+          // two candidates a row at a time
+          for (uint32_t k = k0; k < k1; k += 2u, walked += 2u) {
+            Cand b[3][2];
+#pragma unroll
+            for (int y = 0; y < 3; ++y)
+#pragma unroll
+              for (uint32_t u = 0; u < 2u; ++u) {
+                b[y][u].p = win->pos[entry(y, first[y]) + k + u];
+                b[y][u].r = win->r[entry(y, first[y]) + k + u];
+              }
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+              const float x[3] = {beyond(attract, b[0][u].p, b[0][u].r), beyond(attract, b[1][u].p, b[1][u].r),
+                                  beyond(attract, b[2][u].p, b[2][u].r)};
+              shift_in(w, x, 0x1p-125f);
+            }
+          }
+        } else {
+          // a row already walked re-reads its last candidate
+          for (uint32_t k = k0; k < k1; ++k, ++walked) {
+            Cand b[3];
+#pragma unroll
+            for (int y = 0; y < 3; ++y)
+              candidate_load<kRadius, kOne, false, kO>(c, first[y] + min(k, max(length(y), 1u) - 1u), pos, type,
+                                                       radius, d, b[y]);
+            const float x[3] = {beyond(attract, b[0].p, b[0].r), beyond(attract, b[1].p, b[1].r),
+                                beyond(attract, b[2].p, b[2].r)};
+            shift_in(w, x, 0x1p-125f);
+          }
+        }
+        // left-aligned: the first candidate at bit 31 (none walked: 0)
+#pragma unroll
+        for (int y = 0; y < 3; ++y) w[y] = walked ? w[y] << (32u - walked) : 0u;
       };
-      mark(0u, min(L, 32u), hlo, 0u);
-      if (L > 32u) mark(32u, L, hhi, 32u);
+      uint32_t hlo[3] = {0u, 0u, 0u}, hhi[3] = {0u, 0u, 0u};
+      auto mark_all = [&](auto attract) {
+        mark(attract, 0u, min(L, 32u), hlo);
+        if (L > 32u) mark(attract, 32u, L, hhi);
+      };
+      if (c.attract) mark_all(std::true_type{});
+      else mark_all(std::false_type{});
       uint64_t h[3];
 #pragma unroll
-      for (int y = 0; y < 3; ++y) h[y] = ((uint64_t)hhi[y] << 32) | hlo[y];
+      for (int y = 0; y < 3; ++y) {
+        h[y] = ((uint64_t)hlo[y] << 32) | hhi[y];
+        if (length(y) < 64u) h[y] &= ~(~0ull >> length(y));           // past the row's end
+        const uint32_t own_k = i - first[y];
+        if (own_k < length(y)) h[y] &= ~(1ull << (63u - own_k));  // the particle itself
+      }
       RowSum rsum;
-      rsum.b0 = b0[0];
-      rsum.b1 = b1[0];
-      int row = 0;
+      rsum.b0 = rsum.b1 = kNoBoundary;
+      int row = -1;
       // the particle's velocity, spin and the pressure terms' reciprocal,
       // only where a candidate may touch
       if (h[0] | h[1] | h[2]) {
@@ -695,20 +855,34 @@ __device__ __forceinline__ void collide_particle(const StepConst& c, uint32_t i,
         const bool in0 = h[0] != 0, in1 = !in0 && h[1] != 0;
         const int y = in0 ? 0 : (in1 ? 1 : 2);
         const uint64_t hy = in0 ? h[0] : (in1 ? h[1] : h[2]);
-        const uint32_t j = (in0 ? rs[0] : (in1 ? rs[1] : rs[2])) + (uint32_t)__builtin_ctzll(hy);
-        const uint64_t rest = hy & (hy - 1u);
+        const uint32_t k = (uint32_t)__builtin_clzll(hy), f = in0 ? first[0] : (in1 ? first[1] : first[2]);
+        const uint32_t j = f + k;
+        const uint64_t rest = hy & (~0ull >> 1 >> k);
         h[0] = in0 ? rest : h[0];
         h[1] = in1 ? rest : h[1];
         h[2] = (!in0 && !in1) ? rest : h[2];
         if (y != row) {
           fx += rsum.cfx;
           fy += rsum.cfy;
+          const uint32_t ct = in0 ? cut[0] : (in1 ? cut[1] : cut[2]);
           rsum = RowSum{};
-          rsum.b0 = in0 ? b0[0] : (in1 ? b0[1] : b0[2]);
-          rsum.b1 = in0 ? b1[0] : (in1 ? b1[1] : b1[2]);
+          rsum.b0 = f + (ct >> 8 & 0xFFu);
+          rsum.b1 = f + (ct >> 16);
           row = y;
         }
-        candidate<kRadius, kOne, true, kO, true>(c, q, j, false, pos, d, type, radius, rsum, fx, fy, moment, pres);
+        Cand b;
+        if (in_win) {
+          const uint32_t e = in0 ? entry(0, j) : (in1 ? entry(1, j) : entry(2, j));
+          b.p = win->pos[e];
+          b.r = win->r[e];
+          b.t = kOne ? 0u : clamp_idx(ld<kO>(type, j), c.num_types);
+          const uint32_t jv = d.at<kO>(j);
+          b.v = ld<kO>(d.vel, jv);
+          b.w = ld<kO>(d.omega, jv);
+        } else {
+          candidate_load<kRadius, kOne, true, kO>(c, j, pos, type, radius, d, b);
+        }
+        candidate_at<kRadius, kOne, true, kO, true>(c, q, j, false, b, d, type, rsum, fx, fy, moment, pres);
       }
       fx += rsum.cfx;
       fy += rsum.cfy;
@@ -800,6 +974,7 @@ __device__ __forceinline__ void collide_kernel_body(DEM_COLLIDE_PARAMS) {
   Own own;
   float fx, fy, moment, pres;
   const Dyn d{vel, omega, gat};
+  WaveWindow* win = kMode == kList ? wave_window() : nullptr;
   bool done = false;
   if constexpr (kMat == kInstances) {
     // waves inside one instance (all but the few that straddle a boundary)
@@ -807,13 +982,14 @@ __device__ __forceinline__ void collide_kernel_body(DEM_COLLIDE_PARAMS) {
     const uint32_t t0 = __builtin_amdgcn_readfirstlane(t);
     if (__ballot(t != t0) == 0) {
       collide_particle<kRadius, kMat, kMode, kControl, kO, true>(c, i, pos, d, type, radius, cell_start, cell_end, n,
-                                                                 own, ctl, fx, fy, moment, pres, t0);
+                                                                 own, ctl, fx, fy, moment, pres, t0, win);
       done = true;
     }
   }
   if (!done)
     collide_particle<kRadius, kMat, kMode, kControl, kO>(c, i, pos, d, type, radius, cell_start, cell_end, n, own,
-                                                         ctl, fx, fy, moment, pres);
+                                                         ctl, fx, fy, moment, pres, 0u,
+                                                         kMat == kInstances ? nullptr : win);
   // A wave whose discs all feel no force stores zeros without the three
   // divisions: the sums start at +0 and are never -0, so fx, fy and moment
   // are +0 exactly when nothing acted, and +0 over a positive finite mass or
@@ -1168,7 +1344,7 @@ hipError_t launch_reorder(hipStream_t s, int block, uint32_t* cell_start, uint32
 }
 
 // Kernel variant dispatch: kRadius x material layout x (candidate mode,
-// control), where the controlled particle always uses the plain mode.
+// control), where the controlled particle uses the plain or the list mode.
 inline int mat_kind(const StepConst& c) {
   return c.num_instances > 1 ? kInstances : (c.num_types == 1 ? kOneMat : kManyMat);
 }
@@ -1187,7 +1363,8 @@ inline int mat_kind(const StepConst& c) {
   } while (0)
 #define DEM_DISPATCH(MACRO)                                              \
   do {                                                                   \
-    if (ctl) DEM_DISPATCH_RM(MACRO, kPlain, true);                       \
+    if (ctl && mode == kList) DEM_DISPATCH_RM(MACRO, kList, true);       \
+    else if (ctl) DEM_DISPATCH_RM(MACRO, kPlain, true);                  \
     else if (mode == kPrefetch) DEM_DISPATCH_RM(MACRO, kPrefetch, false);\
     else if (mode == kBatch) DEM_DISPATCH_RM(MACRO, kBatch, false);      \
     else if (mode == kList) DEM_DISPATCH_RM(MACRO, kList, false);        \
@@ -1209,7 +1386,8 @@ hipError_t launch_collide(const StepConst& c, hipStream_t s, int block, const fl
 #define DEM_COLLIDE(R, M, P, X)                                                                             \
   do {                                                                                                      \
     if (o32)                                                                                                \
-      hipLaunchKernelGGL((collide_kernel<R, M, P, X, true>()), grid_for(n, block), dim3(block), 0, s, c, pos, \
+      hipLaunchKernelGGL((collide_kernel<R, M, P, X, true>()), grid_for(n, block), dim3(block),                 \
+                         window_bytes(P, block), s, c, pos,                                                      \
                          vel, acc, omega, alpha, type, radius, cell_start, cell_end, pressure, co, gat, quiet, n); \
     else                                                                                                    \
       hipLaunchKernelGGL((collide_kernel<R, M, P, X, false>()), grid_for(n, block), dim3(block), 0, s, c,     \
@@ -1236,7 +1414,8 @@ hipError_t launch_collide_integrate(const StepConst& c, hipStream_t s, int block
                      vel_out, omega_out, theta_out, next, co, n)
   // the fused kernel has no batched mode: with integrate's registers on top
   // of the batch it spills heavily; it loads one candidate at a time instead
-  if (ctl) DEM_DISPATCH_RM(DEM_CI, kPlain, true);
+  if (ctl && mode == kList) DEM_DISPATCH_RM(DEM_CI, kList, true);
+  else if (ctl) DEM_DISPATCH_RM(DEM_CI, kPlain, true);
   else if (mode == kPrefetch) DEM_DISPATCH_RM(DEM_CI, kPrefetch, false);
   else if (mode == kList) DEM_DISPATCH_RM(DEM_CI, kList, false);
   else DEM_DISPATCH_RM(DEM_CI, kPlain, false);

@@ -75,3 +75,40 @@ def test_long_lists_equal_radix(gpu_ctx, n):
     finally:
         a.close()
         b.close()
+
+
+def packed_rows(n, seed, attract=0.0):
+    """n discs in a few rows of overlapping neighbours, a wide empty gap in
+    the middle (the wave across it has rows far apart) and, at its right
+    end, a heap of discs in one cell (rows of more than 64 candidates)."""
+    s = sc.column_collapse(seed=seed, cols=max(1, n // 4), n=n, box=(n * 0.012 + 6.0, 0.4), pitch=0.0098,
+                           jitter=0.0009)
+    s.pos[n // 2:, 0] += 4.0
+    heap = slice(n - n // 5, n)
+    rng = np.random.default_rng(seed)
+    s.pos[heap] = s.pos[heap][:1] + rng.uniform(-0.004, 0.004, s.pos[heap].shape).astype(np.float32)
+    s.vel[:] = (rng.normal(size=s.vel.shape) * 0.2).astype(np.float32)
+    s.omega[:] = (rng.normal(size=n) * 30.0).astype(np.float32)
+    s.materials[0].attract = attract
+    return s
+
+
+@pytest.mark.parametrize("attract", [0.0, 3.0])
+@pytest.mark.parametrize("n", [5, 63, 64, 65, 129, 700])
+def test_contact_lists_across_windows(gpu_ctx, oracle, n, attract):
+    """The contact-list walk where a wave's rows fit its windows, where they
+    do not, where a wave is not full and where a row has over 64 candidates,
+    with and without attraction, against the oracle."""
+    s = packed_rows(n, seed=n, attract=attract)
+    gpu_ctx.set_step_variant(contact_lists=True)
+    sim, ref = api.Simulation(gpu_ctx, s), oracle.Sim(s, "f32")
+    try:
+        for _ in range(3):
+            sim.step(1)
+            ref.step(1)
+            got, want = sim.download(), ref.state()
+            for k in ("hash", "index", "pos", "vel", "omega", "acc", "alpha", "pressure"):
+                assert bits_equal(got[k], want[k]), k
+    finally:
+        sim.close()
+        ref.close()
