@@ -225,7 +225,7 @@ struct SortScratch {
   uint32_t* row_totals = nullptr;    // 256
   uint32_t capacity = 0;             // max keys
 };
-// Keys per tile of the radix sort (its per-tile digit counts are 256 words).
+// Keys per tile of the radix sort's largest sorts (its per-tile digit counts are 256 words).
 constexpr uint32_t kSortTile = 8192;
 int sort_passes(uint32_t key_bits);
 uint32_t sort_tiles(uint32_t n);

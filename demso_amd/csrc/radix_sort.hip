@@ -8,7 +8,9 @@
 //   downsweep : stable tile ranking, a scatter into LDS in sorted order, then
 //               ordered writes so that consecutive lanes write consecutive
 //               addresses of a digit run.
-// Tiles are 4096 keys.  Inside a tile, each wave owns a run of consecutive
+// Tiles are 8,192 keys, or 2,048 up to a million keys (kSmallTileMax); up to
+// 8,192 keys one workgroup does every pass in LDS (k_sort_tile).
+// Inside a tile, each wave owns a run of consecutive
 // keys and visits them 64 at a time in input order, and the waves' counts are
 // combined in wave order, so ranks follow input order: the sort is stable.
 //
@@ -20,6 +22,8 @@
 // A group whose lanes all share one digit (the high digits of nearly sorted
 // keys) skips the LDS round trip.  The counting and ranking cost a few
 // instructions a key, so the passes stream at close to the memory rate.
+#include <algorithm>
+
 #include "dem_internal.h"
 
 namespace dem {
@@ -27,15 +31,20 @@ namespace {
 
 constexpr int kThreads = 256;  // the row scan
 constexpr int kWaves = kThreads / kWave;
-constexpr uint32_t kTile = kSortTile;
 constexpr int kUThreads = 512;  // the upsweep
 constexpr int kUWaves = kUThreads / kWave;
-constexpr int kItems = (int)kTile / kUThreads;
-static_assert(kItems * kUThreads == (int)kTile && kItems % 4 == 0, "upsweep threads cover a tile, 4 keys a load");
+// Keys a thread of the upsweep and the downsweep takes, and with it the tile.
+// 16 (8,192 keys) moves the most a block; but few such tiles leave most of
+// the chip idle while each ranks its keys in 16 dependent rounds, so smaller
+// sorts take 4 (2,048 keys): 317,811 keys ran 39 tiles at 13.5 us a
+// downsweep, and run 156 in 7.2 us.  At kSmallTileMax the small tiles are as
+// many (512, two blocks a CU) as the large ones are at four times the keys.
+constexpr int kLargeItems = 16, kSmallItems = 4;
+constexpr uint32_t kSmallTile = kUThreads * kSmallItems, kSmallTileMax = 512u * kSmallTile;
+static_assert(kUThreads * kLargeItems == (int)kSortTile, "tiles of kSortTile keys");
 constexpr int kBits = 8;
 constexpr int kRadix = 1 << kBits;
 static_assert(kRadix == kThreads, "one thread per digit in the per-digit phases");
-static_assert(kWaves * kRadix <= (int)kTile, "the peer masks fit in the tile's LDS staging");
 
 __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t x) {
   const uint32_t lane = __lane_id();
@@ -108,10 +117,11 @@ __device__ __forceinline__ uint32_t word(const uint4& v, int j) { return j == 0 
 
 // Per-tile digit counts.  The order of the keys does not matter here, so
 // each lane counts 4 consecutive keys at a time.
-template <bool kVec>
+template <bool kVec, int kItems>
 __global__ __launch_bounds__(kUThreads) void k_upsweep(const uint32_t* __restrict__ keys, uint32_t n,
                                                        uint32_t shift, uint32_t* __restrict__ block_counts,
                                                        uint32_t num_tiles) {
+  constexpr uint32_t kTile = kUThreads * kItems;
   __shared__ uint32_t cnt[kUWaves][kRadix];
   for (int k = threadIdx.x; k < kUWaves * kRadix; k += kUThreads) (&cnt[0][0])[k] = 0;
   __syncthreads();
@@ -174,12 +184,10 @@ __global__ __launch_bounds__(kThreads) void k_scan_rows(uint32_t* __restrict__ b
 // current tile's write-out.
 constexpr int kDThreads = 512;
 constexpr int kDWaves = kDThreads / kWave;
-constexpr int kDItems = (int)kTile / kDThreads;
-constexpr int kDQuads = kDItems / 4;
-static_assert(kDItems * kDThreads == (int)kTile && kDItems % 4 == 0, "downsweep tiles are the upsweep's tiles");
-static_assert(kDWaves * kRadix * 2 <= (int)kTile, "the peer masks fit in the keys' half of the LDS staging");
+static_assert(kDThreads == kUThreads && kLargeItems % 4 == 0 && kSmallItems % 4 == 0,
+              "downsweep tiles are the upsweep's tiles, 4 keys a load");
 
-template <bool kVec>
+template <bool kVec, int kDQuads>
 __device__ __forceinline__ void load_tile(const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ vals_in,
                                           uint32_t base, uint32_t n, uint4* kq, uint4* vq) {
   const uint32_t lane = __lane_id();
@@ -192,17 +200,22 @@ __device__ __forceinline__ void load_tile(const uint32_t* __restrict__ keys_in, 
 }
 
 // (two blocks a CU: at most 128 VGPRs)
-template <bool kVec>
+template <bool kVec, int kDItems>
 __global__ __launch_bounds__(kDThreads, 4) void k_downsweep(
     const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ vals_in,
     uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out, uint32_t n, uint32_t shift,
     const uint32_t* __restrict__ block_offsets, const uint32_t* __restrict__ row_totals,
     uint32_t num_tiles) {
+  constexpr uint32_t kTile = kDThreads * kDItems;
+  constexpr int kDQuads = kDItems / 4;
   // the tile's keys and values: in load order (keys in the first half,
-  // values in the second), then, after the ranking (for which its first
-  // kDWaves * kRadix * 8 bytes hold the waves' peer masks), in sorted order
-  // as (value << 32 | key)
+  // values in the second), then, after the ranking, in sorted order as
+  // (value << 32 | key).  The waves' peer masks lie in the keys' half while
+  // the keys are ranked, or on their own where they do not fit there.
+  constexpr bool kOwnMasks = kDWaves * kRadix * 2 > (int)kTile;
   __shared__ uint64_t stage[kTile];
+  __shared__ uint64_t own_masks[kOwnMasks ? kDWaves * kRadix : 1];
+  uint64_t* masks = kOwnMasks ? own_masks : stage;
   __shared__ uint32_t cnt[kDWaves][kRadix];
   __shared__ uint32_t g_start[kRadix];
   __shared__ uint32_t wsum[kDWaves];
@@ -211,7 +224,7 @@ __global__ __launch_bounds__(kDThreads, 4) void k_downsweep(
   uint32_t* s_vals = s_keys + kTile;
 
   const uint32_t tid = threadIdx.x, lane = __lane_id(), w = tid / kWave;
-  uint64_t* tab = stage + w * kRadix;
+  uint64_t* tab = masks + w * kRadix;
   uint32_t* wk = s_keys + w * (kWave * kDItems);
   uint32_t* wv = s_vals + w * (kWave * kDItems);
   // Start of each digit's run in the output: exclusive scan of the digit
@@ -233,7 +246,7 @@ __global__ __launch_bounds__(kDThreads, 4) void k_downsweep(
   uint4 kq[kDQuads], vq[kDQuads];
   uint32_t key[kDItems], val[kDItems], rank[kDItems];
   uint32_t tile = blockIdx.x;
-  if (tile < num_tiles) load_tile<kVec>(keys_in, vals_in, tile * kTile + w * (kWave * kDItems), n, kq, vq);
+  if (tile < num_tiles) load_tile<kVec, kDQuads>(keys_in, vals_in, tile * kTile + w * (kWave * kDItems), n, kq, vq);
   for (; tile < num_tiles; tile += gridDim.x) {
     const uint32_t base = tile * kTile + w * (kWave * kDItems);
     __syncthreads();  // the previous tile's write-out has read the staging
@@ -250,7 +263,7 @@ __global__ __launch_bounds__(kDThreads, 4) void k_downsweep(
     __syncthreads();  // every wave has read its keys before the peer masks are cleared
     for (int k = tid; k < kDWaves * kRadix; k += kDThreads) {
       (&cnt[0][0])[k] = 0;
-      stage[k] = 0ull;
+      masks[k] = 0ull;
     }
     __syncthreads();
 #pragma unroll
@@ -312,7 +325,7 @@ __global__ __launch_bounds__(kDThreads, 4) void k_downsweep(
     __syncthreads();
     // the next tile's loads go out before this tile's writes
     const uint32_t next = tile + gridDim.x;
-    if (next < num_tiles) load_tile<kVec>(keys_in, vals_in, next * kTile + w * (kWave * kDItems), n, kq, vq);
+    if (next < num_tiles) load_tile<kVec, kDQuads>(keys_in, vals_in, next * kTile + w * (kWave * kDItems), n, kq, vq);
     const uint32_t tile_n = min(kTile, n - tile * kTile);
     for (uint32_t s = tid; s < tile_n; s += kDThreads) {
       const uint64_t kv = stage[s];
@@ -322,6 +335,97 @@ __global__ __launch_bounds__(kDThreads, 4) void k_downsweep(
         keys_out[g] = k;
         vals_out[g] = (uint32_t)(kv >> 32);
       }
+    }
+  }
+}
+
+// Up to 8,192 keys: one workgroup of 1,024 threads does every pass, the pairs
+// in registers between them and in LDS to change places.  The three kernels a
+// pass cost their launches and a chip-wide round trip each (4,096 keys, two
+// passes: 34 us; this 9.0 us).  A wave owns kItems * 64 consecutive
+// pairs and ranks them as the downsweep does.
+constexpr int kOneThreads = 1024, kOneWaves = kOneThreads / kWave;
+constexpr uint32_t kOneMax = kOneThreads * 8;
+
+template <int kItems>
+__global__ __launch_bounds__(kOneThreads) void k_sort_tile(const uint32_t* keys_in, const uint32_t* vals_in,
+                                                           uint32_t* keys_out, uint32_t* vals_out, uint32_t n,
+                                                           int passes) {
+  __shared__ uint64_t stage[kOneThreads * kItems];
+  __shared__ uint64_t masks[kOneWaves * kRadix];
+  __shared__ uint32_t cnt[kOneWaves][kRadix];
+  __shared__ uint32_t wsum[kOneWaves];
+  const uint32_t tid = threadIdx.x, lane = __lane_id(), w = tid / kWave;
+  const uint32_t base = w * (kWave * kItems) + lane;
+  uint64_t* tab = masks + w * kRadix;
+  const uint64_t lt = (1ull << lane) - 1ull;
+  uint32_t key[kItems], val[kItems], rank[kItems];
+#pragma unroll
+  for (int it = 0; it < kItems; ++it) {
+    const uint32_t i = base + it * kWave;
+    key[it] = i < n ? keys_in[i] : 0u;
+    val[it] = i < n ? vals_in[i] : 0u;
+  }
+  for (int k = tid; k < kOneWaves * kRadix; k += kOneThreads) masks[k] = 0ull;  // peer_mask leaves them zero
+  for (int pass = 0; pass < passes; ++pass) {
+    const uint32_t shift = (uint32_t)(pass * kBits);
+    for (int k = tid; k < kOneWaves * kRadix; k += kOneThreads) (&cnt[0][0])[k] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < kItems; ++it) {
+      const bool ok = base + it * kWave < n;
+      const uint32_t d = (key[it] >> shift) & (kRadix - 1);
+      const uint64_t peers = peer_mask(d, ok, __ballot(ok), tab);
+      rank[it] = 0;
+      if (ok) {
+        const uint32_t before = cnt[w][d];
+        rank[it] = before + (uint32_t)__popcll(peers & lt);
+        if (lane == (uint32_t)(__ffsll((unsigned long long)peers) - 1)) cnt[w][d] = before + (uint32_t)__popcll(peers);
+      }
+    }
+    __syncthreads();
+    // where each wave's keys of a digit start: the digits before, then the
+    // waves before (the first 256 threads, one digit each)
+    uint32_t run = 0, inc = 0;
+    if (tid < (uint32_t)kRadix) {
+#pragma unroll
+      for (int k = 0; k < kOneWaves; ++k) {
+        const uint32_t c = cnt[k][tid];
+        cnt[k][tid] = run;
+        run += c;
+      }
+      inc = wave_inclusive_scan(run);
+      if (lane == kWave - 1) wsum[w] = inc;
+    }
+    __syncthreads();
+    if (tid < (uint32_t)kRadix) {
+      uint32_t start = inc - run;
+      for (uint32_t k = 0; k < w; ++k) start += wsum[k];
+#pragma unroll
+      for (int k = 0; k < kOneWaves; ++k) cnt[k][tid] += start;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < kItems; ++it) {
+      if (base + it * kWave >= n) continue;
+      const uint32_t p = cnt[w][(key[it] >> shift) & (kRadix - 1)] + rank[it];
+      if (p < n) stage[p] = ((uint64_t)val[it] << 32) | key[it];  // (always, for a consistent ranking)
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < kItems; ++it) {
+      if (base + it * kWave >= n) continue;
+      const uint64_t kv = stage[base + it * kWave];
+      key[it] = (uint32_t)kv;
+      val[it] = (uint32_t)(kv >> 32);
+    }
+  }
+#pragma unroll
+  for (int it = 0; it < kItems; ++it) {
+    const uint32_t i = base + it * kWave;
+    if (i < n) {
+      keys_out[i] = key[it];
+      vals_out[i] = val[it];
     }
   }
 }
@@ -341,9 +445,15 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 
 int sort_passes(uint32_t key_bits) { return (int)((key_bits + kBits - 1) / kBits); }
 
-uint32_t sort_tiles(uint32_t n) { return (n + kTile - 1) / kTile; }
+uint32_t sort_tiles(uint32_t n) {
+  const uint32_t tile = n <= kSmallTileMax ? kSmallTile : kSortTile;
+  return (n + tile - 1) / tile;
+}
 
-size_t sort_block_count_elems(uint32_t n) { return (size_t)kRadix * sort_tiles(n); }
+// (enough for every count up to n: the small tiles are at most 512)
+size_t sort_block_count_elems(uint32_t n) {
+  return (size_t)kRadix * std::max(sort_tiles(n), sort_tiles(std::min(n, kSmallTileMax)));
+}
 
 hipError_t launch_sort_to(hipStream_t s, uint32_t* keys_in, uint32_t* vals_in, uint32_t* keys_out,
                           uint32_t* vals_out, uint32_t n, uint32_t key_bits, const SortScratch& scratch) {
@@ -358,6 +468,15 @@ hipError_t launch_sort_to(hipStream_t s, uint32_t* keys_in, uint32_t* vals_in, u
   if (n > scratch.capacity || !scratch.keys_alt || !scratch.vals_alt || !scratch.block_counts ||
       !scratch.row_totals || (keys_out == keys_in) != (vals_out == vals_in))
     return hipErrorInvalidValue;
+  if (n <= kOneMax) {
+    if (n <= (uint32_t)kOneThreads * 4u)
+      hipLaunchKernelGGL(k_sort_tile<4>, dim3(1), dim3(kOneThreads), 0, s, keys_in, vals_in, keys_out, vals_out, n,
+                         passes);
+    else
+      hipLaunchKernelGGL(k_sort_tile<8>, dim3(1), dim3(kOneThreads), 0, s, keys_in, vals_in, keys_out, vals_out, n,
+                         passes);
+    return hipGetLastError();
+  }
   const uint32_t tiles = sort_tiles(n);
   // two downsweep blocks a CU (256 CUs), each taking tiles in turn
   const uint32_t down_blocks = std::min(tiles, 512u);
@@ -380,17 +499,21 @@ hipError_t launch_sort_to(hipStream_t s, uint32_t* keys_in, uint32_t* vals_in, u
       }
     }
     const uint32_t shift = (uint32_t)(p * kBits);
-    const bool vec = aligned16(ki) && aligned16(vi);
-    if (vec) hipLaunchKernelGGL(k_upsweep<true>, dim3(tiles), dim3(kUThreads), 0, s, ki, n, shift, scratch.block_counts, tiles);
-    else hipLaunchKernelGGL(k_upsweep<false>, dim3(tiles), dim3(kUThreads), 0, s, ki, n, shift, scratch.block_counts, tiles);
-    hipLaunchKernelGGL(k_scan_rows, dim3(kRadix), dim3(kThreads), 0, s, scratch.block_counts, tiles,
-                       scratch.row_totals);
-    if (vec)
-      hipLaunchKernelGGL(k_downsweep<true>, dim3(down_blocks), dim3(kDThreads), 0, s, ki, vi, ko, vo, n, shift,
-                         scratch.block_counts, scratch.row_totals, tiles);
-    else
-      hipLaunchKernelGGL(k_downsweep<false>, dim3(down_blocks), dim3(kDThreads), 0, s, ki, vi, ko, vo, n, shift,
-                         scratch.block_counts, scratch.row_totals, tiles);
+    const bool vec = aligned16(ki) && aligned16(vi), small = n <= kSmallTileMax;
+#define DEM_SORT_PASS(V, I)                                                                                       \
+  do {                                                                                                            \
+    hipLaunchKernelGGL((k_upsweep<V, I>), dim3(tiles), dim3(kUThreads), 0, s, ki, n, shift, scratch.block_counts, \
+                       tiles);                                                                                    \
+    hipLaunchKernelGGL(k_scan_rows, dim3(kRadix), dim3(kThreads), 0, s, scratch.block_counts, tiles,              \
+                       scratch.row_totals);                                                                       \
+    hipLaunchKernelGGL((k_downsweep<V, I>), dim3(down_blocks), dim3(kDThreads), 0, s, ki, vi, ko, vo, n, shift,   \
+                       scratch.block_counts, scratch.row_totals, tiles);                                          \
+  } while (0)
+    if (vec && small) DEM_SORT_PASS(true, kSmallItems);
+    else if (vec) DEM_SORT_PASS(true, kLargeItems);
+    else if (small) DEM_SORT_PASS(false, kSmallItems);
+    else DEM_SORT_PASS(false, kLargeItems);
+#undef DEM_SORT_PASS
     ki = ko;
     vi = vo;
   }

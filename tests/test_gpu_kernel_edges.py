@@ -112,3 +112,28 @@ def test_contact_lists_across_windows(gpu_ctx, oracle, n, attract):
     finally:
         sim.close()
         ref.close()
+
+
+@pytest.mark.parametrize("key_bits", [8, 13, 24, 32])
+@pytest.mark.parametrize("n", [2, 64, 4095, 4096, 4097, 8191, 8192, 8193, 10241, 1048576, 1048577])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_sort_tile_edges(gpu_ctx, n, key_bits, offset):
+    """The sort in one workgroup, in small and in large tiles, at their
+    limits, from aligned and unaligned arrays; ties keep their order."""
+    import torch
+
+    g = 1 << min(key_bits, 16)
+    s = sc.column_collapse(cols=8, rows=8)
+    s.instances = [sc.Instance(box=(1.0, 1.0), extent=(1.0, 1.0), grid=(g, (1 << key_bits) // g - (key_bits == 32)))]
+    gpu_ctx.load_scene(s)
+    top = s.instances[0].cells
+    k = np.random.default_rng(n).integers(0, top, n, dtype=np.uint64).astype(np.uint32)
+    k[n // 3: n // 2] = k[0]
+    v = np.arange(n, dtype=np.uint32)
+    dk, dv = (torch.zeros(n + 4, dtype=torch.int32, device="cuda")[offset:offset + n] for _ in range(2))
+    dk.copy_(torch.from_numpy(k.view(np.int32)))
+    dv.copy_(torch.from_numpy(v.view(np.int32)))
+    api.sortParticles(gpu_ctx, dk, dv, n)
+    order = np.argsort(k, kind="stable")
+    assert np.array_equal(dk.cpu().numpy().view(np.uint32), k[order])
+    assert np.array_equal(dv.cpu().numpy().view(np.uint32), order.astype(np.uint32))
