@@ -316,7 +316,7 @@ int dem_sim_resort_counts(dem_sim* sim, uint32_t* movers, uint32_t* listed);
 /* DEM_STEP_LIST makes collide first mark, row by row, the candidates that
  * may touch (position and radius only) and then run the contact law over
  * the marked ones: fewer idle lanes on contact-dense states (not together
- * with PREFETCH or BATCH).  Same results. */
+ * with PREFETCH or BATCH).  A new context starts with it.  Same results. */
 #define DEM_STEP_LIST 0x20
 /* Particles a lane of hash, reorder and integrate: log2 of 1, 2 or 4 in bits
  * 8-9 (hash), 10-11 (reorder) and 12-13 (integrate); 0 is one a lane.
