@@ -588,11 +588,15 @@ int sim_alloc(dem_sim* m, T** p, size_t count) {
   return DEM_OK;
 }
 
-void sim_free(dem_sim* m) {
-  for (int k = 0; k < 2; ++k) {
-    if (m->exec[k]) (void)hipGraphExecDestroy(m->exec[k]);
-    if (m->exec_inc[k]) (void)hipGraphExecDestroy(m->exec_inc[k]);
+void drop_graphs(dem_sim* m) {
+  for (hipGraphExec_t* g = &m->exec[0][0][0]; g != &m->exec[0][0][0] + 8; ++g) {
+    if (*g) (void)hipGraphExecDestroy(*g);
+    *g = nullptr;
   }
+}
+
+void sim_free(dem_sim* m) {
+  drop_graphs(m);
   if (m->h_count) (void)hipHostFree(m->h_count);
   for (hipEvent_t& e : m->look)
     if (e) (void)hipEventDestroy(e);
@@ -629,7 +633,16 @@ dem::ShiftState shift_state(dem_sim* m) {
 // slot or key changes are moved where they belong, cellStart/cellEnd are
 // fixed around them, and collide + integrate run on the sorted state in
 // place (integrate computes the next step's keys and mover bits as in the
-// other layout).
+// other layout).  As one kernel they write positions, velocities and spins
+// (which neighbours still read) to the same slots of the other buffer, and
+// the two buffers of these fields change places.
+void flip_buffers(dem_sim* m) {
+  std::swap(m->pos[0], m->pos[1]);
+  std::swap(m->vel[0], m->vel[1]);
+  std::swap(m->omega[0], m->omega[1]);
+  m->flipped = !m->flipped;
+}
+
 hipError_t sim_step_inplace(dem_sim* m, hipStream_t s, hipEvent_t* ev, const StepHook* hook) {
   dem_context* ctx = m->ctx;
   const StepConst& c = ctx->c;
@@ -655,12 +668,23 @@ hipError_t sim_step_inplace(dem_sim* m, hipStream_t s, hipEvent_t* ev, const Ste
     co.react_m = m->react_m;
   }
   const float* radius = m->rad ? m->radius[b] : nullptr;
+  dem::NextKeys nk;
+  nk.key = m->key;
+  nk.bits = m->resort.bits;
+  nk.tile_count = m->resort.tile_count;
   // collide leaves acc and alpha of its quiet runs unwritten; integrate
   // reads the runs' flags
-  e = dem::launch_collide(c, s, ctx->bs_collide, m->pos[b], m->vel[b], m->acc, m->omega[b], m->alpha, m->type[b],
-                          radius, m->cs[b], m->cell_end, m->pressure, n, collide_mode(ctx), control ? &co : nullptr,
-                          nullptr, m->quiet);
+  if (ctx->fuse)
+    e = dem::launch_collide_integrate(c, s, ctx->bs_collide, m->pos[b], m->vel[b], m->omega[b], m->theta[b],
+                                      m->type[b], radius, m->cs[b], m->cell_end, m->acc, m->alpha, m->pressure,
+                                      m->pos[b ^ 1], m->vel[b ^ 1], m->omega[b ^ 1], m->theta[b], nk, n,
+                                      collide_mode(ctx), control ? &co : nullptr, m->quiet);
+  else
+    e = dem::launch_collide(c, s, ctx->bs_collide, m->pos[b], m->vel[b], m->acc, m->omega[b], m->alpha, m->type[b],
+                            radius, m->cs[b], m->cell_end, m->pressure, n, collide_mode(ctx),
+                            control ? &co : nullptr, nullptr, m->quiet);
   if (e != hipSuccess) return e;
+  if (ctx->fuse) flip_buffers(m);
   m->acc_lazy = true;
   if (control) {
     e = dem::launch_control_finish(s, co, m->react_bx, m->react_by, m->react_bm, n, ctx->d_reaction, ctx->d_control,
@@ -669,19 +693,18 @@ hipError_t sim_step_inplace(dem_sim* m, hipStream_t s, hipEvent_t* ev, const Ste
   }
   m->sorted_key = m->skey[b];
   if (hook && hook->fn) {
-    // the sorted pre-integrate state is buffer b itself
-    e = hook->fn(hook->user, m, s, b, b, true);
+    // the sorted pre-integrate state is buffer b itself, or what was its
+    // positions, velocities and spins before the fused kernel
+    e = hook->fn(hook->user, m, s, ctx->fuse ? b ^ 1 : b, b, true);
     if (e != hipSuccess) return e;
   }
   if (ev) (void)hipEventRecord(ev[5], s);
-  dem::NextKeys nk;
-  nk.key = m->key;
-  nk.bits = m->resort.bits;
-  nk.tile_count = m->resort.tile_count;
-  e = dem::launch_integrate_to(c, s, ctx->bs_integrate, m->pos[b], m->vel[b], m->theta[b], m->omega[b], m->pos[b],
-                               m->vel[b], m->theta[b], m->omega[b], m->acc, m->alpha, m->type[b], radius,
-                               m->pressure, n, &nk, nullptr, ctx->per_integrate, m->quiet);
-  if (e != hipSuccess) return e;
+  if (!ctx->fuse) {
+    e = dem::launch_integrate_to(c, s, ctx->bs_integrate, m->pos[b], m->vel[b], m->theta[b], m->omega[b], m->pos[b],
+                                 m->vel[b], m->theta[b], m->omega[b], m->acc, m->alpha, m->type[b], radius,
+                                 m->pressure, n, &nk, nullptr, ctx->per_integrate, m->quiet);
+    if (e != hipSuccess) return e;
+  }
   if (ev) (void)hipEventRecord(ev[6], s);
   m->sorted_key = m->skey[b];
   m->sorted_idx = m->sidx;
@@ -703,7 +726,7 @@ hipError_t sim_step_on(dem_sim* m, hipStream_t s, hipEvent_t* ev, bool resort, c
   //  * full (fused collide + integrate, or a hook that records the sorted
   //    pre-integrate state): reorder sorts every field into kScratch, from
   //    which collide + integrate write buffer t.
-  if (resort && sim_inplace(m, hook)) return sim_step_inplace(m, s, ev, hook);
+  if (resort && sim_inplace(m)) return sim_step_inplace(m, s, ev, hook);
   const int o = m->cur, t = o ^ 1;
   const bool gather = !ctx->fuse && !(hook && hook->fn);
   const int S = gather ? t : kScratch;
@@ -765,7 +788,7 @@ hipError_t sim_step_on(dem_sim* m, hipStream_t s, hipEvent_t* ev, bool resort, c
   if (!gather && ctx->fuse) {
     e = dem::launch_collide_integrate(c, s, ctx->bs_collide, m->pos[S], m->vel[S], m->omega[S], m->theta[S],
                                       m->type[t], S_radius, m->cs[t], m->cell_end, m->acc, m->alpha, m->pressure,
-                                      m->pos[t], m->vel[t], m->omega[t], m->theta[t], nk, n, ctx->cmode,
+                                      m->pos[t], m->vel[t], m->omega[t], m->theta[t], nk, n, collide_mode(ctx),
                                       control ? &co : nullptr);
     if (e != hipSuccess) return e;
     if (control) {
@@ -808,7 +831,11 @@ hipError_t sim_step_on(dem_sim* m, hipStream_t s, hipEvent_t* ev, bool resort, c
   return hipSuccess;
 }
 
-bool sim_inplace(const dem_sim* m, const StepHook*) { return !m->ctx->copy && !m->ctx->fuse; }
+// With the fused kernel, small states reorder as a whole instead: the in-place
+// re-sort's kernels have the longer chains of dependent loads (65,536 discs:
+// 25 us a step against 28).
+constexpr uint32_t kWholeMax = 262144;
+bool sim_inplace(const dem_sim* m) { return !m->ctx->copy && !(m->ctx->fuse && m->n <= kWholeMax); }
 
 namespace {
 // acc = alpha = +0 in the runs of 64 slots that collide marked quiet.
@@ -881,43 +908,43 @@ int sim_check(dem_sim* m) {
   return ensure_device(m->ctx);
 }
 
-int sim_capture(dem_sim* m) {
+// The graph of two steps, radix-sorted or re-sorted, from the present buffers
+// (they are back in place after two steps), captured on first use.
+int sim_graph(dem_sim* m, bool resort, hipGraphExec_t* exec) {
   dem_context* ctx = m->ctx;
-  if (!m->cap_stream) DEM_HIP(ctx, hipStreamCreateWithFlags(&m->cap_stream, hipStreamNonBlocking), "hipStreamCreate");
-  for (int k = 0; k < 2; ++k) {
-    if (m->exec[k]) (void)hipGraphExecDestroy(m->exec[k]);
-    if (m->exec_inc[k]) (void)hipGraphExecDestroy(m->exec_inc[k]);
-    m->exec[k] = m->exec_inc[k] = nullptr;
-  }
-  const int saved = m->cur;
-  uint32_t* const saved_key = m->sorted_key;
-  uint32_t* const saved_idx = m->sorted_idx;
-  const bool saved_list = m->perm_list;
-  for (int variant = 0; variant < 2; ++variant) {
-    for (int start = 0; start < 2; ++start) {
-      hipGraph_t g = nullptr;
-      DEM_HIP(ctx, hipStreamBeginCapture(m->cap_stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
-      m->cur = start;
-      hipError_t e1 = sim_step_on(m, m->cap_stream, nullptr, variant == 1);
-      hipError_t e2 = e1 == hipSuccess ? sim_step_on(m, m->cap_stream, nullptr, variant == 1) : e1;
-      hipError_t e3 = hipStreamEndCapture(m->cap_stream, &g);
-      m->cur = saved;
-      m->cell_start = m->cs[saved];
-      m->sorted_key = saved_key;
-      m->sorted_idx = saved_idx;
-      m->perm_list = saved_list;
-      if (e2 != hipSuccess) {
-        if (g) (void)hipGraphDestroy(g);
-        return hip_fail(ctx, e2, "capturing the step");
-      }
-      if (e3 != hipSuccess) return hip_fail(ctx, e3, "hipStreamEndCapture");
-      hipGraphExec_t* slot = variant == 1 ? &m->exec_inc[start] : &m->exec[start];
-      hipError_t e4 = hipGraphInstantiate(slot, g, nullptr, nullptr, 0);
-      (void)hipGraphDestroy(g);
-      if (e4 != hipSuccess) return hip_fail(ctx, e4, "hipGraphInstantiate");
+  hipGraphExec_t* slot = &m->exec[resort][m->cur][m->flipped];
+  if (!*slot) {
+    if (!m->cap_stream)
+      DEM_HIP(ctx, hipStreamCreateWithFlags(&m->cap_stream, hipStreamNonBlocking), "hipStreamCreate");
+    const int saved = m->cur;
+    const bool saved_flip = m->flipped, saved_list = m->perm_list, saved_lazy = m->acc_lazy;
+    uint32_t* const saved_key = m->sorted_key;
+    uint32_t* const saved_idx = m->sorted_idx;
+    hipGraph_t g = nullptr;
+    DEM_HIP(ctx, hipStreamBeginCapture(m->cap_stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
+    hipError_t e1 = sim_step_on(m, m->cap_stream, nullptr, resort);
+    if (e1 == hipSuccess) e1 = sim_step_on(m, m->cap_stream, nullptr, resort);
+    const hipError_t e2 = hipStreamEndCapture(m->cap_stream, &g);
+    m->cur = saved;
+    if (m->flipped != saved_flip) flip_buffers(m);
+    m->cell_start = m->cs[saved];
+    m->sorted_key = saved_key;
+    m->sorted_idx = saved_idx;
+    m->perm_list = saved_list;
+    m->acc_lazy = saved_lazy;
+    if (e1 != hipSuccess) {
+      if (g) (void)hipGraphDestroy(g);
+      return hip_fail(ctx, e1, "capturing the step");
+    }
+    if (e2 != hipSuccess) return hip_fail(ctx, e2, "hipStreamEndCapture");
+    const hipError_t e3 = hipGraphInstantiate(slot, g, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(g);
+    if (e3 != hipSuccess) {
+      *slot = nullptr;
+      return hip_fail(ctx, e3, "hipGraphInstantiate");
     }
   }
-  m->graph_gen = ctx->generation;
+  *exec = *slot;
   return DEM_OK;
 }
 
@@ -1143,8 +1170,8 @@ int dem_sim_step_graph(dem_sim* m, uint32_t steps) {
     --steps;
   }
   if (steps == 0) return DEM_OK;
-  if (!m->exec[0] || m->graph_gen != ctx->generation)
-    if (int r = sim_capture(m)) return r;
+  if (m->graph_gen != ctx->generation) drop_graphs(m);
+  m->graph_gen = ctx->generation;
   // The automatic sort choice reads counts that the replays write: with
   // every replay queued at once they would all be chosen from the counts of
   // before the call.  It queues the replays in groups of kLookGroup instead,
@@ -1159,7 +1186,9 @@ int dem_sim_step_graph(dem_sim* m, uint32_t steps) {
     hipEvent_t& slot = m->look[(r / G) & 1u];
     if (look && r % G == 0 && r >= 2u * G) DEM_HIP(ctx, hipEventSynchronize(slot), "hipEventSynchronize");
     const bool resort = sim_use_resort(m);
-    DEM_HIP(ctx, hipGraphLaunch(resort ? m->exec_inc[m->cur] : m->exec[m->cur], ctx->stream), "hipGraphLaunch");
+    hipGraphExec_t exec = nullptr;
+    if (int rc = sim_graph(m, resort, &exec)) return rc;
+    DEM_HIP(ctx, hipGraphLaunch(exec, ctx->stream), "hipGraphLaunch");
     if (look && r % G == G - 1u) DEM_HIP(ctx, hipEventRecord(slot, ctx->stream), "hipEventRecord");
     m->resort_ok = true;
     m->perm_list = resort && sim_inplace(m);
@@ -1548,33 +1577,35 @@ int dem_sim_autotune(dem_sim* m, uint32_t* block) {
   const float* D_omega = inplace ? S_omega : m->omega[o];
   const float* D_theta = inplace ? S_theta : m->theta[o];
   const uint32_t* gat = inplace ? nullptr : si;
+  uint32_t* quiet = inplace ? m->quiet : nullptr;
   auto collide = [&](int b) {
     return dem::launch_collide(c, s, b, S_pos, D_vel, m->acc, D_omega, m->alpha, m->type[t], S_radius,
                                m->cell_start, m->cell_end, m->pressure, n, pf | (ctx->wide ? kWideMode : 0),
-                               nullptr, gat);
+                               nullptr, gat, quiet);
   };
   auto integrate = [&](int b) {
     return dem::launch_integrate_to(c, s, b, S_pos, D_vel, D_theta, D_omega, tpos, tvel, ttheta, tomega, m->acc,
-                                    m->alpha, m->type[t], S_radius, m->pressure, n, &nk, gat, tper);
+                                    m->alpha, m->type[t], S_radius, m->pressure, n, &nk, gat, tper, quiet);
   };
   auto fused = [&](int b) {
     return dem::launch_collide_integrate(c, s, b, S_pos, S_vel, S_omega, S_theta, m->type[t], S_radius,
                                          m->cell_start, m->cell_end, m->acc, m->alpha, m->pressure, tpos, tvel,
-                                         tomega, ttheta, nk, n, pf);
+                                         tomega, inplace ? m->theta[K] : ttheta, nk, n, ctx->wide ? kWideMode : 0, nullptr, quiet);
   };
   int best[4] = {ctx->bs_hash, ctx->bs_reorder, ctx->bs_collide, ctx->bs_integrate};
   int best_per[4] = {ctx->per_hash, ctx->per_reorder, 1, ctx->per_integrate};
   float best_t[4] = {1e30f, 1e30f, 1e30f, 1e30f};
   float t_full = 1e30f;  // the fused layout's reorder (every field) at the best block size
   int bs_full = ctx->bs_reorder, per_full = ctx->per_reorder;
-  // collide and fused block sizes for each candidate mode
+  // collide's block size for each candidate mode, and the fused kernel's
   constexpr int kModes = 4;
-  int best_c[kModes], best_f[kModes];
-  float t_c[kModes], t_f[kModes];
+  int best_c[kModes], best_f = ctx->bs_collide;
+  float t_c[kModes], t_f = 1e30f;
   for (int p = 0; p < kModes; ++p) {
-    best_c[p] = best_f[p] = ctx->bs_collide;
-    t_c[p] = t_f[p] = 1e30f;
+    best_c[p] = ctx->bs_collide;
+    t_c[p] = 1e30f;
   }
+  if (e == hipSuccess) e = collide(ctx->bs_collide);  // the accelerations and quiet runs that integrate reads
   for (int bs : cand) {
     if (e != hipSuccess) break;
     float tm = 0;
@@ -1601,23 +1632,9 @@ int dem_sim_autotune(dem_sim* m, uint32_t* block) {
       e = time_it(collide, bs, &tm);
       if (e != hipSuccess) break;
       if (tm < t_c[p]) { t_c[p] = tm; best_c[p] = bs; }
-      if (p == 2) continue;  // the fused kernel has no batched mode
-      e = time_it(fused, bs, &tm);
-      if (e != hipSuccess) break;
-      if (tm < t_f[p]) { t_f[p] = tm; best_f[p] = bs; }
     }
-  }
-  // the in-place layout's apply launches with nothing listed (their cost
-  // when few particles change slot); the last in-place step's index is
-  // materialized first, since its list is cleared for this
-  float t_apply = 0.0f;
-  if (e == hipSuccess && inplace) {
-    if (m->perm_list) e = dem::launch_shift_index(s, m->shift, m->sidx, n);
-    m->perm_list = false;
-    if (e == hipSuccess) e = dem::launch_fill(s, m->shift.count, 0u, 2);
-    const dem::ShiftState st = shift_state(m);
-    if (e == hipSuccess)
-      e = time_it([&](int) { return dem::launch_resort_shift_apply(s, st, m->shift, m->cells, n); }, 0, &t_apply);
+    if (e == hipSuccess) e = time_it(fused, bs, &tm);
+    if (e == hipSuccess && tm < t_f) { t_f = tm; best_f = bs; }
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
@@ -1626,22 +1643,28 @@ int dem_sim_autotune(dem_sim* m, uint32_t* block) {
   if (ttheta) (void)hipFree(ttheta);
   if (tomega) (void)hipFree(tomega);
   m->resort_ok = false;  // the cell arrays and keys now hold the tuning step's data
-  m->acc_lazy = false;   // and acc, alpha the tuning collide's (every slot written)
+  m->acc_lazy = inplace;  // and acc, alpha the tuning collide's (in place without the quiet runs')
   if (e != hipSuccess) return hip_fail(ctx, e, "autotune");
-  // collide + integrate as one kernel or two, in whichever candidate mode is
-  // fastest here (the split layout's reorder moves fewer bytes than the
-  // fused layout's)
+  // collide + integrate as one kernel or two, the latter in whichever
+  // candidate mode is fastest here.  In place both follow the same re-sort;
+  // the copy layout reorders every field for the one kernel and only the
+  // positions for the two.
   bool fuse = false;
   int mode = 0;
   float tbest = 1e30f;
-  const float t_move = inplace ? t_apply : best_t[1];  // the split layout's reorder
-  for (int p = 0; p < kModes; ++p) {
-    if (t_move + t_c[p] + best_t[3] < tbest) { tbest = t_move + t_c[p] + best_t[3]; fuse = false; mode = p; }
-    if (p != 2 && t_full + t_f[p] < tbest) { tbest = t_full + t_f[p]; fuse = true; mode = p; }
+  const float t_move = inplace ? 0.0f : best_t[1], t_move_full = inplace ? 0.0f : t_full;
+  for (int p = 0; p < kModes; ++p)
+    if (t_move + t_c[p] + best_t[3] < tbest) {
+      tbest = t_move + t_c[p] + best_t[3];
+      mode = p;
+    }
+  if (t_move_full + t_f < tbest) {
+    fuse = true;
+    mode = 3;
   }
   ctx->bs_hash = best[0];
   ctx->bs_reorder = fuse ? bs_full : best[1];
-  ctx->bs_collide = fuse ? best_f[mode] : best_c[mode];
+  ctx->bs_collide = fuse ? best_f : best_c[mode];
   ctx->bs_integrate = best[3];
   ctx->per_hash = best_per[0];
   ctx->per_reorder = fuse ? per_full : best_per[1];

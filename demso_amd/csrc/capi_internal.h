@@ -65,7 +65,7 @@ struct dem_context {
 };
 
 // Every field of the owned simulation's state lives in buffer `cur` (0 or 1)
-// between steps; a step writes the next state into buffer cur ^ 1.  The
+// between steps; a step writes the next state into buffer cur ^ 1, or in place.  The
 // dynamic fields (pos, vel, theta, omega) have a third buffer, kScratch, for
 // the fully sorted copy that the fused collide + integrate and the adjoint's
 // recorded steps read.
@@ -115,8 +115,13 @@ struct dem_sim {
   int sort_mode = 0;            // 0 auto, 1 radix sort every step, 2 re-sort whenever resort_ok
   int cur = 0;
   hipStream_t cap_stream = nullptr;
-  hipGraphExec_t exec[2] = {nullptr, nullptr};      // two radix-sorted steps, by starting buffer
-  hipGraphExec_t exec_inc[2] = {nullptr, nullptr};  // two re-sorted steps, by starting buffer
+  // two steps, radix-sorted ([0]) or re-sorted ([1]), by the starting buffer
+  // and by flipped; each captured when it is first needed
+  hipGraphExec_t exec[2][2][2] = {};
+  // whether the two buffers of pos, vel and omega have changed places: the
+  // fused step in place writes them into the other buffer, whose pointers
+  // then take buffer cur's place
+  bool flipped = false;
   uint64_t graph_gen = 0;
   // sort_mode 0: an event recorded after every kLookGroup-th replay (or
   // eager step); before it starts a group, the host waits on the event of
@@ -141,13 +146,12 @@ bool multi(const dem_context* ctx);
 int sim_check(dem_sim* m);
 // One step (src/main.cu:431-507) on stream s; ev (7 events) or NULL.
 // resort: sort by dem::launch_resort (needs m->resort_ok) instead of the
-// radix sort; without a hook and with the split collide/integrate layout the
-// state is then re-sorted in place (unless ctx->copy).
+// radix sort; the state is then re-sorted in place (unless ctx->copy).
 // hook: given the step's sorted pre-integrate state, e.g. to store it (the
 // adjoint): dyn is the buffer holding the sorted pos/vel/omega (kScratch in
-// the full layout, where the hook runs after integrate, or the state buffer
-// itself in place, where it runs between collide and integrate), stat the
-// buffer of the sorted radius/type; list: the step's sorted index is the
+// the full layout, where the hook runs after integrate; in place the state
+// buffer itself, where it runs between collide and integrate, or the other
+// buffer after the fused kernel), stat the buffer of the sorted radius/type; list: the step's sorted index is the
 // identity except at the slots listed in m->shift (in place), else it is
 // m->sorted_idx.
 struct StepHook {
@@ -162,7 +166,7 @@ bool sim_use_resort(dem_sim* m);
 // into acc and alpha (nothing if they are complete).
 hipError_t sim_acc_complete(dem_sim* m, hipStream_t s);
 // Whether a re-sorted step of m runs in place (see sim_step_on).
-bool sim_inplace(const dem_sim* m, const StepHook* hook = nullptr);
+bool sim_inplace(const dem_sim* m);
 
 }  // namespace dem
 

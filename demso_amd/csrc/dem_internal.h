@@ -200,15 +200,16 @@ hipError_t launch_integrate_to(const StepConst& c, hipStream_t s, int block, con
                                uint32_t n, const NextKeys* next = nullptr, const uint32_t* gat = nullptr,
                                int per = 1, const uint32_t* quiet = nullptr);
 // collide + integrate + the next step's hash in one kernel: forces from the
-// sorted state *_in, acc/alpha/pressure as collide writes them, the
-// integrated state to *_out (a different buffer).
+// sorted state *_in, acc/alpha/pressure as collide writes them (quiet: as
+// launch_collide's), the integrated state to *_out (a different buffer;
+// theta_out may be theta_in).
 hipError_t launch_collide_integrate(const StepConst& c, hipStream_t s, int block, const float2* pos_in,
                                     const float2* vel_in, const float* omega_in, const float* theta_in,
                                     const uint32_t* type, const float* radius, const uint32_t* cell_start,
                                     const uint32_t* cell_end, float2* acc, float* alpha, float* pressure,
                                     float2* pos_out, float2* vel_out, float* omega_out, float* theta_out,
                                     const NextKeys& next, uint32_t n, int mode = 0,
-                                    const struct ControlOut* ctl = nullptr);
+                                    const struct ControlOut* ctl = nullptr, uint32_t* quiet = nullptr);
 // The controlled particle's reaction: per-block tree sums of the three
 // per-particle reaction vectors into bx/by/bm (ceil(n/kReactBlock) each),
 // their ordered sum into reaction[3], then (move) its kinematic move.
