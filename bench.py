@@ -59,11 +59,13 @@ METRIC = "particle-steps/s @4M discs; batched-ensemble and fwd+adjoint vs plain 
 #   type 4, radius 4, W pos 8, id 4, loc 4, type 4, radius 4; collide and
 #   integrate also read the sorted index (4 each) and velocity, spin and
 #   angle through it.
-# Fused (collide + integrate in one kernel): reorder sorts every field (R key
-#   4, index 4, pos 8, vel 8, theta 4, omega 4, id 4, type 4, radius 4; W the
-#   same state and loc 4) and the fused kernel reads pos 8, vel 8, omega 4,
-#   theta 4, radius 4, type 4 and writes acc 8, alpha 4, pressure 4, pos 8,
-#   vel 8, theta 4, omega 4 (+ 8 per cell), reported under collide.
+# Fused (collide + integrate in one kernel, in place): it reads pos 8, vel 8,
+#   omega 4, theta 4, radius 4, type 4 and writes acc 8, alpha 4, pressure 4,
+#   pos 8, vel 8, theta 4, omega 4 (+ 8 per cell), reported under collide.
+# Whole (up to 262,144 particles; the fused kernel or the two of in place):
+#   re-sort and reorder in one kernel, reported under sort: R key 4, pos 8,
+#   vel 8, theta 4, omega 4, id 4, type 4, radius 4, W the same, loc 4 and
+#   index 4, + the next cellStart 4 per cell.
 STAGES = ("hash", "sort", "cell_fill", "reorder", "collide", "integrate")
 
 
@@ -72,17 +74,19 @@ def stage_bytes(layout: str, radius: bool, typed: bool) -> tuple[dict, dict]:
     r = 4 if radius else 0
     t = 4 if typed else 0
     per_cell = {"hash": 0, "sort": 0, "cell_fill": 0, "reorder": 0, "collide": 8, "integrate": 0}
-    if layout == "fused":
-        pp = {"hash": 0, "sort": 12, "cell_fill": 0, "reorder": 76 + 2 * r, "collide": 64 + r + t, "integrate": 0}
-        per_cell["sort"] = 4
-
-    elif layout == "copy":
+    pp = {"hash": 0, "sort": 0, "cell_fill": 0, "reorder": 0,
+          "collide": 8 + r + t + 12 + 16, "integrate": 8 + 16 + 12 + r + t + 24}
+    if layout.startswith("copy"):
         pp = {"hash": 0, "sort": 12, "cell_fill": 0, "reorder": 44 + 2 * r,
               "collide": 4 + 8 + r + t + 12 + 16, "integrate": 4 + 8 + 16 + 12 + r + t + 24}
         per_cell["sort"] = 4
-    else:
-        pp = {"hash": 0, "sort": 0, "cell_fill": 0, "reorder": 0,
-              "collide": 8 + r + t + 12 + 16, "integrate": 8 + 16 + 12 + r + t + 24}
+    elif layout.startswith("whole"):
+        pp["sort"] = 72 + 8 + 2 * r
+        per_cell["sort"] = 4
+    if layout.endswith("fused"):
+        pp.update(collide=64 + r + t, integrate=0)
+        if layout.startswith("copy"):
+            pp["reorder"] = 76 + 2 * r
     return pp, per_cell
 
 
@@ -515,7 +519,10 @@ def main() -> int:
     # per-kernel durations with HIP events on the launch stream; the sort is
     # a multi-kernel stage (3 kernels per radix pass) and is reported apart
     stages = sim.stage_times(max(5, min(args.steps, 50)))
-    layout = "fused" if tuned and tuned.get("fused") else ("copy" if tuned and tuned.get("copy") else "inplace")
+    fused = bool(tuned and tuned.get("fused"))
+    layout = "copy" if tuned and tuned.get("copy") else ("whole" if n <= 262144 else "inplace")
+    if fused:
+        layout += "_fused"
     acct = dict(layout=layout, radius=scene.radius is not None, typed=len(scene.materials) > 1)
     kernel_stages = {k: v for k, v in stages.items()
                      if k in ("cell_fill", "reorder", "collide", "integrate") and algorithmic_bytes(k, n, cells, **acct) > 0}
@@ -531,7 +538,7 @@ def main() -> int:
         sim.step(1)
     fixed = fixed_step_bytes(n, cells)
     touched = None
-    if "collide" in kernel_stages and layout != "fused":
+    if "collide" in kernel_stages and not fused:
         used = cells_collide_reads(scene, sim.download()["hash"])
         pp, _ = stage_bytes(layout, acct["radius"], acct["typed"])
         tb = pp["collide"] * n + 8 * used
@@ -547,7 +554,7 @@ def main() -> int:
         # per candidate mode where the file has one (collide's traffic differs a little by mode)
         mode = (args.collide_mode or "plain") if not tuned else next(
             (m for k, m in (("prefetch", "prefetch"), ("batch", "batch"), ("contact_lists", "list")) if tuned.get(k)), "plain")
-        traffic = t.get(f"{dom}_{mode}", t.get(dom))
+        traffic = t.get("fused") if fused and dom == "collide" else t.get(f"{dom}_{mode}", t.get(dom))
 
     cpu = None
     if args.cpu_steps > 0:

@@ -612,8 +612,7 @@ void sim_free(dem_sim* m) {
 // can re-sort from them.
 namespace {
 
-dem::ShiftState shift_state(dem_sim* m) {
-  const int b = m->cur;
+dem::ShiftState shift_state(dem_sim* m, int b) {
   dem::ShiftState st;
   st.pos = m->pos[b];
   st.vel = m->vel[b];
@@ -643,22 +642,20 @@ void flip_buffers(dem_sim* m) {
   m->flipped = !m->flipped;
 }
 
-hipError_t sim_step_inplace(dem_sim* m, hipStream_t s, hipEvent_t* ev, const StepHook* hook) {
+// The second half of a step, from the sorted state in buffer t (positions in
+// t; velocities, angles and spins in t too, or with gat in buffer o, read
+// through that index): collide and integrate into buffer t, in one kernel or
+// two, the controlled particle's part, the hook, and the next step's keys.
+// list: the state was re-sorted in place (m->shift has the moved slots);
+// resorted: re-sorted in place or as a whole, where collide leaves acc and
+// alpha of its quiet runs unwritten and integrate reads the runs' flags.
+hipError_t sim_forces(dem_sim* m, hipStream_t s, hipEvent_t* ev, const StepHook* hook, int t, const uint32_t* gat,
+                      bool list, bool resorted) {
   dem_context* ctx = m->ctx;
   const StepConst& c = ctx->c;
-  const int b = m->cur;
   const uint32_t n = m->n;
-  const dem::ShiftState st = shift_state(m);
+  const int o = t ^ 1, D = gat ? o : t;
   hipError_t e;
-  if (ev) (void)hipEventRecord(ev[0], s);
-  if (ev) (void)hipEventRecord(ev[1], s);
-  e = dem::launch_resort_shift_plan(s, m->key, st, m->shift, m->cells, ctx->key_bits, m->resort, n);
-  if (e != hipSuccess) return e;
-  if (ev) (void)hipEventRecord(ev[2], s);
-  if (ev) (void)hipEventRecord(ev[3], s);
-  e = dem::launch_resort_shift_apply(s, st, m->shift, m->cells, n);
-  if (e != hipSuccess) return e;
-  if (ev) (void)hipEventRecord(ev[4], s);
   ControlOut co;
   const bool control = ctx->h_control.enabled != 0;
   if (control) {
@@ -667,50 +664,105 @@ hipError_t sim_step_inplace(dem_sim* m, hipStream_t s, hipEvent_t* ev, const Ste
     co.react_y = m->react_y;
     co.react_m = m->react_m;
   }
-  const float* radius = m->rad ? m->radius[b] : nullptr;
+  const float* radius = m->rad ? m->radius[t] : nullptr;
   dem::NextKeys nk;
   nk.key = m->key;
   nk.bits = m->resort.bits;
   nk.tile_count = m->resort.tile_count;
-  // collide leaves acc and alpha of its quiet runs unwritten; integrate
-  // reads the runs' flags
+  if (sim_whole(m)) {
+    // the next step goes from buffer t to buffer o
+    nk.list = m->whole_list[t];
+    nk.list_count = m->whole_count + t;
+    nk.clear = m->cs[o];
+    nk.clear_n = m->cells;
+    if (resorted) nk.listed = m->whole_count + 2 + t;  // (counted by this step's re-sort)
+    nk.host_listed = m->shift.host_listed;
+  }
+  m->next_list = sim_whole(m);
+  uint32_t* q = resorted ? m->quiet : nullptr;
+  // (After an in-place step, a radix-sorted step's hook still sees acc_lazy
+  // set: the adjoint's slot of the first step of a recomputed segment then
+  // takes +0 accelerations for the runs that the last in-place step marked
+  // quiet.  A known defect of states that re-sort in place, left as it was
+  // because mending it changes their gradients.)
+  if (resorted || sim_whole(m)) m->acc_lazy = resorted;
   if (ctx->fuse)
-    e = dem::launch_collide_integrate(c, s, ctx->bs_collide, m->pos[b], m->vel[b], m->omega[b], m->theta[b],
-                                      m->type[b], radius, m->cs[b], m->cell_end, m->acc, m->alpha, m->pressure,
-                                      m->pos[b ^ 1], m->vel[b ^ 1], m->omega[b ^ 1], m->theta[b], nk, n,
-                                      collide_mode(ctx), control ? &co : nullptr, m->quiet);
+    e = dem::launch_collide_integrate(c, s, ctx->bs_collide, m->pos[t], m->vel[t], m->omega[t], m->theta[t],
+                                      m->type[t], radius, m->cs[t], m->cell_end, m->acc, m->alpha, m->pressure,
+                                      m->pos[o], m->vel[o], m->omega[o], m->theta[t], nk, n, collide_mode(ctx),
+                                      control ? &co : nullptr, q);
   else
-    e = dem::launch_collide(c, s, ctx->bs_collide, m->pos[b], m->vel[b], m->acc, m->omega[b], m->alpha, m->type[b],
-                            radius, m->cs[b], m->cell_end, m->pressure, n, collide_mode(ctx),
-                            control ? &co : nullptr, nullptr, m->quiet);
+    e = dem::launch_collide(c, s, ctx->bs_collide, m->pos[t], m->vel[D], m->acc, m->omega[D], m->alpha, m->type[t],
+                            radius, m->cs[t], m->cell_end, m->pressure, n, collide_mode(ctx),
+                            control ? &co : nullptr, gat, q);
   if (e != hipSuccess) return e;
   if (ctx->fuse) flip_buffers(m);
-  m->acc_lazy = true;
   if (control) {
     e = dem::launch_control_finish(s, co, m->react_bx, m->react_by, m->react_bm, n, ctx->d_reaction, ctx->d_control,
                                    true);
     if (e != hipSuccess) return e;
   }
-  m->sorted_key = m->skey[b];
   if (hook && hook->fn) {
-    // the sorted pre-integrate state is buffer b itself, or what was its
+    // the sorted pre-integrate state is buffer t itself, or what was its
     // positions, velocities and spins before the fused kernel
-    e = hook->fn(hook->user, m, s, ctx->fuse ? b ^ 1 : b, b, true);
+    e = hook->fn(hook->user, m, s, ctx->fuse ? o : t, t, list);
     if (e != hipSuccess) return e;
   }
   if (ev) (void)hipEventRecord(ev[5], s);
   if (!ctx->fuse) {
-    e = dem::launch_integrate_to(c, s, ctx->bs_integrate, m->pos[b], m->vel[b], m->theta[b], m->omega[b], m->pos[b],
-                                 m->vel[b], m->theta[b], m->omega[b], m->acc, m->alpha, m->type[b], radius,
-                                 m->pressure, n, &nk, nullptr, ctx->per_integrate, m->quiet);
+    e = dem::launch_integrate_to(c, s, ctx->bs_integrate, m->pos[t], m->vel[D], m->theta[D], m->omega[D], m->pos[t],
+                                 m->vel[t], m->theta[t], m->omega[t], m->acc, m->alpha, m->type[t], radius,
+                                 m->pressure, n, &nk, gat, ctx->per_integrate, q);
     if (e != hipSuccess) return e;
   }
   if (ev) (void)hipEventRecord(ev[6], s);
+  m->cur = t;
+  m->cell_start = m->cs[t];
+  m->perm_list = list;
+  m->acc_lazy = resorted;
+  return hipSuccess;
+}
+
+hipError_t sim_step_inplace(dem_sim* m, hipStream_t s, hipEvent_t* ev, const StepHook* hook) {
+  const int b = m->cur;
+  const uint32_t n = m->n;
+  const dem::ShiftState st = shift_state(m, b);
+  hipError_t e;
+  if (ev) (void)hipEventRecord(ev[0], s);
+  if (ev) (void)hipEventRecord(ev[1], s);
+  e = dem::launch_resort_shift_plan(s, m->key, st, m->shift, m->cells, m->ctx->key_bits, m->resort, n);
+  if (e != hipSuccess) return e;
+  if (ev) (void)hipEventRecord(ev[2], s);
+  if (ev) (void)hipEventRecord(ev[3], s);
+  e = dem::launch_resort_shift_apply(s, st, m->shift, m->cells, n);
+  if (e != hipSuccess) return e;
+  if (ev) (void)hipEventRecord(ev[4], s);
   m->sorted_key = m->skey[b];
   m->sorted_idx = m->sidx;
-  m->cell_start = m->cs[b];
-  m->perm_list = true;
-  return hipSuccess;
+  return sim_forces(m, s, ev, hook, b, nullptr, true, true);
+}
+
+// A re-sorted step of a small state, which goes into the other buffer whole.
+hipError_t sim_step_whole(dem_sim* m, hipStream_t s, hipEvent_t* ev, const StepHook* hook) {
+  const int o = m->cur, t = o ^ 1;
+  if (ev)
+    for (int k = 0; k < 2; ++k) (void)hipEventRecord(ev[k], s);
+  dem::WholeMovers mv;
+  mv.list = m->whole_list[o];
+  mv.count = m->whole_count + o;
+  mv.bits = m->resort.bits;
+  mv.key = m->key;
+  mv.next_count = m->whole_count + t;
+  mv.listed = m->whole_count + 2 + t;
+  mv.next_listed = m->whole_count + 2 + o;
+  mv.host_count = m->resort.host_count;
+  const hipError_t e = dem::launch_resort_whole(s, shift_state(m, o), shift_state(m, t), mv, m->sidx, m->cells, m->n);
+  if (e != hipSuccess) return e;
+  if (ev)
+    for (int k = 2; k < 5; ++k) (void)hipEventRecord(ev[k], s);
+  m->sorted_key = m->skey[t];
+  m->sorted_idx = m->sidx;
+  return sim_forces(m, s, ev, hook, t, nullptr, false, true);
 }
 
 }  // namespace
@@ -718,18 +770,17 @@ hipError_t sim_step_inplace(dem_sim* m, hipStream_t s, hipEvent_t* ev, const Ste
 hipError_t sim_step_on(dem_sim* m, hipStream_t s, hipEvent_t* ev, bool resort, const StepHook* hook) {
   dem_context* ctx = m->ctx;
   const StepConst& c = ctx->c;
+  if (resort && sim_whole(m)) return sim_step_whole(m, s, ev, hook);
+  if (resort && sim_inplace(m)) return sim_step_inplace(m, s, ev, hook);
   // The state is in buffer o and the step writes buffer t.  Two layouts:
   //  * gather (the default): reorder sorts only the positions (into t) and
   //    the per-particle constants; collide and integrate read velocity,
   //    spin and angle from buffer o through the sorted index, and integrate
   //    writes the new state into t (positions in place);
   //  * full (fused collide + integrate, or a hook that records the sorted
-  //    pre-integrate state): reorder sorts every field into kScratch, from
-  //    which collide + integrate write buffer t.
-  if (resort && sim_inplace(m)) return sim_step_inplace(m, s, ev, hook);
+  //    pre-integrate state): reorder sorts every field into t.
   const int o = m->cur, t = o ^ 1;
   const bool gather = !ctx->fuse && !(hook && hook->fn);
-  const int S = gather ? t : kScratch;
   const uint32_t n = m->n;
   const uint32_t* type_for_hash = multi(ctx) ? m->type[o] : nullptr;
   hipError_t e;
@@ -748,7 +799,8 @@ hipError_t sim_step_on(dem_sim* m, hipStream_t s, hipEvent_t* ev, bool resort, c
     if (e != hipSuccess) return e;
     // this step's collide + integrate accumulates the next step's mover counts
     const uint32_t tiles = (n + dem::kResortTile - 1u) / dem::kResortTile;
-    e = dem::launch_fill(s, m->resort.tile_count, 0u, tiles);
+    e = sim_whole(m) ? dem::launch_fill(s, m->whole_count, 0u, 4)
+                     : dem::launch_fill(s, m->resort.tile_count, 0u, tiles);
     if (e != hipSuccess) return e;
     if (ev) (void)hipEventRecord(ev[1], s);
     // the last pass writes the sorted keys and index where the step keeps them
@@ -763,79 +815,27 @@ hipError_t sim_step_on(dem_sim* m, hipStream_t s, hipEvent_t* ev, bool resort, c
     if (e != hipSuccess) return e;
   }
   if (ev) (void)hipEventRecord(ev[3], s);
-  e = dem::launch_reorder(s, ctx->bs_reorder, m->cs[t], m->cell_end, m->pos[S], gather ? nullptr : m->vel[S],
-                          gather ? nullptr : m->theta[S], gather ? nullptr : m->omega[S], m->id[t], m->loc[t],
+  e = dem::launch_reorder(s, ctx->bs_reorder, m->cs[t], m->cell_end, m->pos[t], gather ? nullptr : m->vel[t],
+                          gather ? nullptr : m->theta[t], gather ? nullptr : m->omega[t], m->id[t], m->loc[t],
                           m->type[t], m->rad ? m->radius[t] : nullptr, m->sorted_key, m->sorted_idx, m->pos[o],
                           m->vel[o], m->theta[o], m->omega[o], m->id[o], m->type[o],
                           m->rad ? m->radius[o] : nullptr, n, m->cells, !gather, ctx->per_reorder);
   if (e != hipSuccess) return e;
   if (ev) (void)hipEventRecord(ev[4], s);
-  dem::NextKeys nk;
-  nk.key = m->key;
-  nk.bits = m->resort.bits;
-  nk.tile_count = m->resort.tile_count;
-  const float* S_radius = m->rad ? m->radius[t] : nullptr;
-  // the controlled particle: pair term in collide, then its reaction and
-  // move (src/main.cu:466-514); the move does not feed this step's integrate
-  ControlOut co;
-  const bool control = ctx->h_control.enabled != 0;
-  if (control) {
-    co.state = ctx->d_control;
-    co.react_x = m->react_x;
-    co.react_y = m->react_y;
-    co.react_m = m->react_m;
-  }
-  if (!gather && ctx->fuse) {
-    e = dem::launch_collide_integrate(c, s, ctx->bs_collide, m->pos[S], m->vel[S], m->omega[S], m->theta[S],
-                                      m->type[t], S_radius, m->cs[t], m->cell_end, m->acc, m->alpha, m->pressure,
-                                      m->pos[t], m->vel[t], m->omega[t], m->theta[t], nk, n, collide_mode(ctx),
-                                      control ? &co : nullptr);
-    if (e != hipSuccess) return e;
-    if (control) {
-      e = dem::launch_control_finish(s, co, m->react_bx, m->react_by, m->react_bm, n, ctx->d_reaction, ctx->d_control,
-                                     true);
-      if (e != hipSuccess) return e;
-    }
-    if (ev) (void)hipEventRecord(ev[5], s);
-  } else {
-    // with gather, velocity and spin come from buffer o through the index
-    const int D = gather ? o : S;
-    const uint32_t* gat = gather ? m->sorted_idx : nullptr;
-    e = dem::launch_collide(c, s, ctx->bs_collide, m->pos[S], m->vel[D], m->acc, m->omega[D], m->alpha, m->type[t],
-                            S_radius, m->cs[t], m->cell_end, m->pressure, n, collide_mode(ctx),
-                            control ? &co : nullptr, gat);
-    if (e != hipSuccess) return e;
-    if (control) {
-      e = dem::launch_control_finish(s, co, m->react_bx, m->react_by, m->react_bm, n, ctx->d_reaction, ctx->d_control,
-                                     true);
-      if (e != hipSuccess) return e;
-    }
-    if (ev) (void)hipEventRecord(ev[5], s);
-    // integrate into buffer t (with gather the positions in place, and
-    // velocity, angle and spin through the index from buffer o)
-    e = dem::launch_integrate_to(c, s, ctx->bs_integrate, m->pos[S], m->vel[D], m->theta[D], m->omega[D], m->pos[t],
-                                 m->vel[t], m->theta[t], m->omega[t], m->acc, m->alpha, m->type[t], S_radius,
-                                 m->pressure, n, &nk, gat, ctx->per_integrate);
-    if (e != hipSuccess) return e;
-  }
-  if (hook && hook->fn) {
-    // the full layout: the sorted pre-integrate state is still in kScratch / t
-    e = hook->fn(hook->user, m, s, kScratch, t, false);
-    if (e != hipSuccess) return e;
-  }
-  if (ev) (void)hipEventRecord(ev[6], s);
-  m->cur = t;
-  m->cell_start = m->cs[t];
-  m->perm_list = false;
-  m->acc_lazy = false;  // these layouts write every acc and alpha
-  return hipSuccess;
+  // (these steps write every acc and alpha)
+  return sim_forces(m, s, ev, hook, t, gather ? m->sorted_idx : nullptr, false, false);
 }
 
-// With the fused kernel, small states reorder as a whole instead: the in-place
-// re-sort's kernels have the longer chains of dependent loads (65,536 discs:
-// 25 us a step against 28).
+// Up to this many particles a re-sorted step takes the whole state to the
+// other buffer in one kernel: its cost is a few dependent loads and 88 bytes a
+// particle, the in-place kernels' a longer chain and what the movers shift.
+// A step whole against in place: 65,536 discs 14 against 25 us in a settled
+// column (9 movers), 15 against 17 falling apart (1 mover); 262,144: 22
+// against 32, and 23 against 19; 524,176: 32 against 42, and 32 against 26;
+// 1,048,576: 47 against 55, and 47 against 35.
 constexpr uint32_t kWholeMax = 262144;
-bool sim_inplace(const dem_sim* m) { return !m->ctx->copy && !(m->ctx->fuse && m->n <= kWholeMax); }
+bool sim_whole(const dem_sim* m) { return !m->ctx->copy && m->n <= kWholeMax; }
+bool sim_inplace(const dem_sim* m) { return !m->ctx->copy && m->n > kWholeMax; }
 
 namespace {
 // acc = alpha = +0 in the runs of 64 slots that collide marked quiet.
@@ -861,7 +861,8 @@ hipError_t sim_acc_complete(dem_sim* m, hipStream_t s) {
 constexpr uint32_t kListedFrac = 4;
 
 bool sim_use_resort(dem_sim* m) {
-  if (!m->resort_ok || m->sort_mode == 1) return false;
+  // (the movers must be listed as this step's re-sort reads them)
+  if (!m->resort_ok || m->sort_mode == 1 || m->next_list != sim_whole(m)) return false;
   if (m->sort_mode == 2) return true;
   // The radix sort and full reorder cost about the same every step.  The
   // re-sort's movers step is one workgroup, fast up to a few thousand
@@ -878,8 +879,9 @@ bool sim_use_resort(dem_sim* m) {
   // of a dense pack lists 2-3M of 4.2M discs a step for a thousand steps).
   const volatile uint32_t* h = m->h_count;
   const uint32_t movers = h[0], listed = h[1];
-  const uint32_t mover_limit = std::max(4096u, m->n / 64u), listed_limit = m->n / kListedFrac;
   const bool inplace = sim_inplace(m);
+  const uint32_t mover_limit = sim_whole(m) ? kWholeSorted : std::max(4096u, m->n / 64u);
+  const uint32_t listed_limit = m->n / kListedFrac;
   const bool cheap = movers <= mover_limit && (!inplace || listed <= listed_limit);
   if (cheap) {
     m->radix_run = m->radix_wait = 0;
@@ -1020,6 +1022,9 @@ int dem_sim_create(dem_context* ctx, uint32_t n, uint32_t num_cells, int with_ra
   if (!r && m->rad) r = sim_alloc(m, &m->shift.radius, n);
   if (!r) r = sim_alloc(m, &m->shift.count, 4);
   if (!r) r = sim_alloc(m, &m->shift.tag, n);
+  for (int b = 0; b < 2; ++b)
+    if (!r && n <= kWholeMax) r = sim_alloc(m, &m->whole_list[b], std::max(n, dem::kWholeSorted));
+  if (!r) r = sim_alloc(m, &m->whole_count, 4);
   m->shift.pos = m->pos[kScratch];
   m->shift.vel = m->vel[kScratch];
   m->shift.theta = m->theta[kScratch];
@@ -1192,7 +1197,8 @@ int dem_sim_step_graph(dem_sim* m, uint32_t steps) {
     if (look && r % G == G - 1u) DEM_HIP(ctx, hipEventRecord(slot, ctx->stream), "hipEventRecord");
     m->resort_ok = true;
     m->perm_list = resort && sim_inplace(m);
-    m->acc_lazy = m->perm_list;
+    m->acc_lazy = resort && !ctx->copy;
+    m->next_list = sim_whole(m);
   }
   // Each replay runs two steps, which leaves the state in the same buffer;
   // the sorted keys are in skey[cur] and the sorted index in sidx.
@@ -1447,6 +1453,8 @@ int dem_collide_controlled(dem_context* ctx, const float* pos, const float* vel,
     DEM_HIP(ctx, hipMalloc((void**)&ctx->d_stage_control, sizeof(dem_controlled) + 4 * sizeof(float)),
             "hipMalloc(controlled)");
     ctx->d_stage_reaction = (float*)(ctx->d_stage_control + 1);
+    DEM_HIP(ctx, dem::launch_fill(ctx->stream, (uint32_t*)ctx->d_stage_reaction, 0u, 4), "controlled");
+    DEM_HIP(ctx, hipStreamSynchronize(ctx->stream), "controlled");
   }
   dem_controlled st{};
   st.pos[0] = control_state[0];

@@ -65,10 +65,9 @@ struct dem_context {
 };
 
 // Every field of the owned simulation's state lives in buffer `cur` (0 or 1)
-// between steps; a step writes the next state into buffer cur ^ 1, or in place.  The
-// dynamic fields (pos, vel, theta, omega) have a third buffer, kScratch, for
-// the fully sorted copy that the fused collide + integrate and the adjoint's
-// recorded steps read.
+// between steps; a step writes the next state into buffer cur ^ 1, or in place.
+// The dynamic fields (pos, vel, theta, omega) have a third buffer, kScratch,
+// where the in-place re-sort stages what it moves.
 constexpr int kScratch = 2;
 
 struct dem_sim {
@@ -105,6 +104,13 @@ struct dem_sim {
   // (sim_acc_complete).
   uint32_t* quiet = nullptr;
   bool acc_lazy = false;
+  // Whole re-sort (dem::launch_resort_whole): the movers of the state in
+  // buffer b, their count and the particles the step from it listed
+  // (whole_count[0/1] and [2/3]); next_list says that the last step left them
+  // (rather than the mover counts per tile of the other re-sorts)
+  uint64_t* whole_list[2] = {};
+  uint32_t* whole_count = nullptr;
+  bool next_list = false;
   // host-mapped: [0] the mover count of the last re-sort, [1] the particles
   // the last in-place re-sort listed (slot or key changed)
   uint32_t* h_count = nullptr;
@@ -145,13 +151,13 @@ int ensure_device(dem_context* ctx);
 bool multi(const dem_context* ctx);
 int sim_check(dem_sim* m);
 // One step (src/main.cu:431-507) on stream s; ev (7 events) or NULL.
-// resort: sort by dem::launch_resort (needs m->resort_ok) instead of the
-// radix sort; the state is then re-sorted in place (unless ctx->copy).
+// resort: re-sort (needs m->resort_ok) instead of the radix sort: a small
+// state as a whole (sim_whole), a larger one in place (sim_inplace), or with
+// ctx->copy by dem::launch_resort and a full reorder.
 // hook: given the step's sorted pre-integrate state, e.g. to store it (the
-// adjoint): dyn is the buffer holding the sorted pos/vel/omega (kScratch in
-// the full layout, where the hook runs after integrate; in place the state
-// buffer itself, where it runs between collide and integrate, or the other
-// buffer after the fused kernel), stat the buffer of the sorted radius/type; list: the step's sorted index is the
+// adjoint): dyn is the buffer holding the sorted pos/vel/omega (the step's
+// own buffer, where the hook runs between collide and integrate, or the other
+// one after the fused kernel), stat the buffer of the sorted radius/type; list: the step's sorted index is the
 // identity except at the slots listed in m->shift (in place), else it is
 // m->sorted_idx.
 struct StepHook {
@@ -165,8 +171,10 @@ bool sim_use_resort(dem_sim* m);
 // Writes the +0 accelerations of the quiet runs of the last in-place step
 // into acc and alpha (nothing if they are complete).
 hipError_t sim_acc_complete(dem_sim* m, hipStream_t s);
-// Whether a re-sorted step of m runs in place (see sim_step_on).
+// Whether a re-sorted step of m runs in place, or re-sorts and reorders the
+// whole (small) state in one kernel (see sim_step_on).
 bool sim_inplace(const dem_sim* m);
+bool sim_whole(const dem_sim* m);
 
 }  // namespace dem
 

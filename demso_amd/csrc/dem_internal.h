@@ -157,6 +157,28 @@ hipError_t launch_resort_shift_apply(hipStream_t s, const ShiftState& st, const 
 // identity (only the listed slots are written).
 hipError_t launch_shift_index(hipStream_t s, const ShiftScratch& sh, uint32_t* index, uint32_t n,
                               bool identity_done = false);
+// Re-sort and reorder of a small state in one kernel, from its movers as
+// integrate listed them (NextKeys::list): every particle goes from its slot in
+// `from` (arrays in the order of from.skey) to its slot in `to`, with the
+// sorted keys and index, loc, and the cell ranges of reorderDataAndFindCell-
+// Start (to.cell_start all kEmpty before; cell_end is one array for both).
+// count movers are in list; next_count and next_listed are set to 0 for the
+// steps that follow, listed gains the particles whose slot or key changed.
+struct WholeMovers {
+  const uint64_t* list = nullptr;  // at least kWholeSorted entries may be read
+  const uint32_t* count = nullptr;
+  const uint32_t* bits = nullptr;  // the mover bits and keys (NextKeys)
+  const uint32_t* key = nullptr;
+  uint32_t* next_count = nullptr;
+  uint32_t* listed = nullptr;
+  uint32_t* next_listed = nullptr;
+  uint32_t* host_count = nullptr;
+};
+// Movers up to which their order is kept in LDS (more are counted through
+// one by one, for every particle).
+constexpr uint32_t kWholeSorted = 512;
+hipError_t launch_resort_whole(hipStream_t s, const ShiftState& from, const ShiftState& to, const WholeMovers& mv,
+                               uint32_t* index, uint32_t num_cells, uint32_t n);
 hipError_t launch_reorder(hipStream_t s, int block, uint32_t* cell_start, uint32_t* cell_end,
                           float2* s_pos, float2* s_vel, float* s_theta, float* s_omega,
                           uint32_t* s_id, uint32_t* s_loc, uint32_t* s_type, float* s_radius,
@@ -187,6 +209,16 @@ struct NextKeys {
   uint32_t* key = nullptr;
   uint32_t* bits = nullptr;
   uint32_t* tile_count = nullptr;
+  // For launch_resort_whole, instead of tile_count: the movers' (key << 32 |
+  // slot), appended in any order to list from *list_count (zero before); the
+  // next step's cellStart, set to kEmpty here; and the last re-sort's count
+  // of listed particles, passed on to its host-mapped mirror (null: none).
+  uint64_t* list = nullptr;
+  uint32_t* list_count = nullptr;
+  uint32_t* clear = nullptr;
+  uint32_t clear_n = 0;
+  const uint32_t* listed = nullptr;
+  uint32_t* host_listed = nullptr;
 };
 hipError_t launch_integrate(const StepConst& c, hipStream_t s, int block, float2* pos, float2* vel,
                             const float2* acc, float* theta, float* omega, const float* alpha,
@@ -212,7 +244,8 @@ hipError_t launch_collide_integrate(const StepConst& c, hipStream_t s, int block
                                     const struct ControlOut* ctl = nullptr, uint32_t* quiet = nullptr);
 // The controlled particle's reaction: per-block tree sums of the three
 // per-particle reaction vectors into bx/by/bm (ceil(n/kReactBlock) each),
-// their ordered sum into reaction[3], then (move) its kinematic move.
+// their ordered sum into reaction[0..2], then (move) its kinematic move.
+// reaction[3] is the blocks' ticket, a word that is 0 before and after.
 hipError_t launch_control_finish(hipStream_t s, const struct ControlOut& ctl, float* bx, float* by, float* bm,
                                  uint32_t n, float* reaction, dem_controlled* state, bool move);
 

@@ -588,7 +588,7 @@ inline size_t window_bytes(int mode, int block) {
 // kUni: every lane of the call has material row t_uni (a wave-uniform value,
 // so the material row and the instance geometry are scalar loads and the
 // grid arithmetic scalar).
-template <bool kRadius, int kMat, int kMode, bool kControl, bool kO, bool kUni = false>
+template <bool kRadius, int kMat, int kMode, bool kControl, bool kO, bool kUni = false, bool kEarly = false>
 __device__ __forceinline__ void collide_particle(const StepConst& c, uint32_t i, const float2* __restrict__ pos,
                                                  const Dyn& d, const uint32_t* __restrict__ type,
                                                  const float* __restrict__ radius,
@@ -610,7 +610,7 @@ __device__ __forceinline__ void collide_particle(const StepConst& c, uint32_t i,
   // The particle's own velocity and spin feed only the contact law (and the
   // fused kernel's integrate): the contact-list walk loads them once it has
   // marked a candidate (or at the end, where a caller uses them), the other
-  // modes up front.
+  // modes, and with kEarly the list too, up front.
   bool have_dyn = false;
   auto load_own_dyn = [&]() {
     const uint32_t iv = d.at<kO>(i);
@@ -618,7 +618,7 @@ __device__ __forceinline__ void collide_particle(const StepConst& c, uint32_t i,
     q.w = d.omega[iv];
     have_dyn = true;
   };
-  if (kMode != kList || kControl) load_own_dyn();
+  if (kMode != kList || kControl || kEarly) load_own_dyn();
   own.p = q.p;
   q.den = pressure_den(q.rA);
   q.rden = 0.0;  // the contact-list walk sets it before its first contact
@@ -1154,33 +1154,46 @@ __device__ __forceinline__ bool integrate_particle(const StepConst& c, const Mat
 }
 
 // The next step's hash of an integrated particle (NextKeys): the cell key of
-// its new position p; true when it left the cell of its sorted slot, whose
-// key is old (the state stays in this order until the next sort).
-__device__ __forceinline__ bool next_key(const StepConst& c, const NextKeys& nk, float2 p, uint32_t old,
-                                         const Instance& in, uint32_t i) {
+// its new position p and whether it left the cell of its sorted slot, whose
+// key is old (the state stays in this order until the next sort).  kWhole:
+// for launch_resort_whole.  Every lane of the wave that holds a particle
+// calls this.
+template <bool kWhole>
+__device__ __forceinline__ void next_key(const StepConst& c, const NextKeys& nk, float2 p, uint32_t old,
+                                         const Instance& in, uint32_t i, uint32_t n) {
   const uint32_t k = cell_key_in(c, in, p);
-  if (k != old) nk.key[i] = k;  // a stayer's key is its sorted key
-  return k != old;
-}
-
-// The wave's mover bits and count (every lane of the wave that holds a
-// particle calls this).
-__device__ __forceinline__ void next_movers(const NextKeys& nk, bool mover, uint32_t i, uint32_t n) {
+  const bool mover = k != old;
+  if (mover) nk.key[i] = k;  // a stayer's key is its sorted key
   const uint64_t moved = __ballot(mover);
+  uint32_t at = 0;
   if (__lane_id() == 0) {  // lane 0 holds the wave's first index, a multiple of 64
     const uint32_t w0 = i / 32u, nwords = (n + 31u) / 32u;
     nk.bits[w0] = (uint32_t)moved;
     if (w0 + 1u < nwords) nk.bits[w0 + 1u] = (uint32_t)(moved >> 32);
     const uint32_t cnt = (uint32_t)__popcll(moved);
-    if (cnt) atomicAdd(&nk.tile_count[i / kResortTile], cnt);
+    if (cnt) {
+      if constexpr (kWhole) at = atomicAdd(nk.list_count, cnt);
+      else atomicAdd(&nk.tile_count[i / kResortTile], cnt);
+    }
+  }
+  if (kWhole && moved) {
+    at = __builtin_amdgcn_readfirstlane(at) + (uint32_t)__popcll(moved & ((1ull << __lane_id()) - 1ull));
+    if (mover && at < n) nk.list[at] = ((uint64_t)k << 32) | i;
   }
 }
 
-// integrateSystemD over all particles.  The input and output arrays may be
+// NextKeys' other outputs, particle i's share.
+__device__ __forceinline__ void next_clear(const NextKeys& nk, uint32_t i, uint32_t n) {
+  for (uint32_t cell = i; cell < nk.clear_n; cell += n) nk.clear[cell] = kEmpty;
+  if (i == 0u && nk.listed) *nk.host_listed = *nk.listed;
+}
+
+// integrateSystemD over all particles, with the next step's keys (kNext 1:
+// NextKeys; 2: for launch_resort_whole; 0: none).  The input and output arrays may be
 // the same (in place, as the reference) or different (the owned
 // simulation writes the integrated state back to its home buffer); each
 // lane reads and writes only its own slot.
-template <bool kRadius, int kMat, bool kNext, int kPer>
+template <bool kRadius, int kMat, int kNext, int kPer>
 __global__ __launch_bounds__(256) void k_integrate(
     StepConst c, const float2* pos_in, const float2* vel_in, const float* theta_in, const float* omega_in,
     float2* pos_out, float2* vel_out, float* theta_out, float* omega_out, const float2* __restrict__ acc,
@@ -1201,6 +1214,7 @@ __global__ __launch_bounds__(256) void k_integrate(
   for (int k = 0; k < kPer; ++k) {
     const uint32_t i = base + (uint32_t)k * blockDim.x;
     if (i >= n) continue;
+    if (kNext == 2) next_clear(nk, i, n);
     t[k] = kMat == kOneMat ? 0u : clamp_idx(type[i], c.num_types);
     // velocity, spin and angle through the gather index when one is given
     const uint32_t g = gat ? gat[i] : i;
@@ -1235,7 +1249,7 @@ __global__ __launch_bounds__(256) void k_integrate(
       if (!in_place || __float_as_uint(tt) != __float_as_uint(th[k])) theta_out[i] = tt;
       // (the key the particle is sorted by is the hash of its position before
       // integrate, recomputed here rather than read)
-      if (kNext) next_movers(nk, next_key(c, nk, p, cell_key_in(c, in, p_old[k]), in, i), i, n);
+      if (kNext) next_key<kNext == 2>(c, nk, p, cell_key_in(c, in, p_old[k]), in, i, n);
     };
     if constexpr (kMulti) {
       // a wave inside one instance reads its material row and geometry as
@@ -1265,8 +1279,8 @@ __global__ __launch_bounds__(256) void k_integrate(
 // 8.2M-disc ensemble.  (There material rows and geometries are loaded per
 // lane: collide's second code path, with them in scalar registers where a
 // wave lies in one instance, takes 87 registers here, and 221 us.)
-template <bool kRadius, int kMat, int kMode, bool kControl, bool kO>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMat == kOneMat ? 8 : 7))) void k_collide_integrate(
+template <bool kRadius, int kMat, bool kWhole, int kMode, bool kControl, bool kO>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWhole ? 4 : (kMat == kOneMat ? 8 : 7)))) void k_collide_integrate(
     StepConst c, const float2* __restrict__ pos_in, const float2* __restrict__ vel_in,
     const float* __restrict__ omega_in, const float* theta_in, const uint32_t* __restrict__ type,
     const float* __restrict__ radius, const uint32_t* __restrict__ cell_start,
@@ -1276,12 +1290,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMat == kOn
     uint32_t n) {
   const uint32_t i = xcd_block() * blockDim.x + threadIdx.x;
   if (i >= n) return;
+  if constexpr (kWhole) next_clear(nk, i, n);
   const Dyn d{vel_in, omega_in, nullptr};
   WaveWindow* win = kMode == kList ? wave_window() : nullptr;
   Own own;
   float fx, fy, moment, pres;
-  collide_particle<kRadius, kMat, kMode, kControl, kO>(c, i, pos_in, d, type, radius, cell_start, cell_end, n, own,
-                                                       ctl, fx, fy, moment, pres, 0u, win);
+  // (small states do not fill the chip, so latency counts, not registers:
+  // every load that can go out first does)
+  const float th_first = kWhole ? theta_in[i] : 0.0f;
+  collide_particle<kRadius, kMat, kMode, kControl, kO, false, kWhole>(c, i, pos_in, d, type, radius, cell_start,
+                                                                      cell_end, n, own, ctl, fx, fy, moment, pres, 0u,
+                                                                      win);
   const Material m = c.mat[own.t];
   const Instance in = kMat == kInstances ? c.inst[clamp_idx(m.inst, c.num_instances)] : c.inst0;
   body<kRadius>(m, &own.r, 0u, own.r, own.mass, own.inertia);  // (again, rather than kept)
@@ -1290,7 +1309,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMat == kOn
   store_acc<kRadius>(own, fx, fy, moment, i, acc, alpha, quiet, a, al);
   float2 p = own.p, v = own.v;
   float w = own.w;
-  const float th_in = theta_in[i];
+  const float th_in = kWhole ? th_first : theta_in[i];
   float th = th_in;
   (void)integrate_particle(c, m, in, own.r, own.mass, own.inertia, a, al, p, v, w, th, pres, nullptr);
   pressure[i] = pres;
@@ -1298,7 +1317,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMat == kOn
   vel_out[i] = v;
   omega_out[i] = w;
   if (theta_out != theta_in || __float_as_uint(th) != __float_as_uint(th_in)) theta_out[i] = th;
-  next_movers(nk, next_key(c, nk, p, own.cell, in, i), i, n);
+  next_key<kWhole>(c, nk, p, own.cell, in, i, n);
 }
 
 inline dim3 grid_for(uint32_t n, int block) { return dim3((n + (uint32_t)block - 1u) / (uint32_t)block); }
@@ -1449,10 +1468,15 @@ hipError_t launch_collide_integrate(const StepConst& c, hipStream_t s, int block
   if (block % kWave) return hipErrorInvalidValue;  // waves must cover aligned 64-particle runs
   const ControlOut co = ctl ? *ctl : ControlOut{};
   const bool o32 = !(mode & kWideMode) && n <= (1u << 29) && c.cells <= (1u << 30);  // (launch_collide)
-#define DEM_CI(R, M, P, X)                                                                                         \
-  hipLaunchKernelGGL((k_collide_integrate<R, M, P, X, P == kList>), grid_for(n, block), dim3(block),               \
+#define DEM_CI_W(R, M, W, P, X)                                                                                    \
+  hipLaunchKernelGGL((k_collide_integrate<R, M, W, P, X, P == kList>), grid_for(n, block), dim3(block),            \
                      window_bytes(P, block), s, c, pos_in, vel_in, omega_in, theta_in, type, radius, cell_start,   \
                      cell_end, acc, alpha, pressure, pos_out, vel_out, omega_out, theta_out, next, co, quiet, n)
+#define DEM_CI(R, M, P, X)                   \
+  do {                                       \
+    if (next.list) DEM_CI_W(R, M, true, P, X); \
+    else DEM_CI_W(R, M, false, P, X);        \
+  } while (0)
   // contact lists (from 4,096 discs, 6.3 us against 6.0 one candidate ahead,
   // and 65,536, 6.8 against 7.0, to 4M dense ones, where walking candidates one
   // at a time runs the contact law at every candidate some lane touches), or
@@ -1462,6 +1486,7 @@ hipError_t launch_collide_integrate(const StepConst& c, hipStream_t s, int block
   else if (ctl) DEM_DISPATCH_CTL(DEM_CI, kPlain);
   else DEM_DISPATCH_RM(DEM_CI, kPlain, false);
 #undef DEM_CI
+#undef DEM_CI_W
   return hipGetLastError();
 }
 #undef DEM_DISPATCH
@@ -1471,13 +1496,18 @@ hipError_t launch_collide_integrate(const StepConst& c, hipStream_t s, int block
 // ---- controlled particle: reaction sum and move ------------------------------
 // reduceVecD (src/particles_kernel.cuh:552-578) on the three reaction
 // vectors: block b sums values [512 b, 512 b + 512) (zeros past n) by the
-// same pairwise tree.
-__global__ __launch_bounds__(kReactBlock) void k_reduce_reaction(const float* __restrict__ rx,
-                                                                const float* __restrict__ ry,
-                                                                const float* __restrict__ rm, float* __restrict__ bx,
-                                                                float* __restrict__ by, float* __restrict__ bm,
-                                                                uint32_t n) {
+// same pairwise tree.  The last block to finish (it takes the last of the
+// tickets, which it resets) adds the block sums in order
+// (src/functions.cu:505-513, there on the host), one lane per quantity, then
+// makes the kinematic move of the controlled particle (src/main.cu:510-514)
+// when `move` is set.  No block waits for another; a second launch for the
+// sum took 4.3 us after the first's 4.5.
+__global__ __launch_bounds__(kReactBlock) void k_reduce_reaction(
+    const float* __restrict__ rx, const float* __restrict__ ry, const float* __restrict__ rm, float* __restrict__ bx,
+    float* __restrict__ by, float* __restrict__ bm, uint32_t n, uint32_t blocks, float* __restrict__ reaction,
+    dem_controlled* state, int move, uint32_t* __restrict__ ticket) {
   __shared__ float cx[kReactBlock], cy[kReactBlock], cm[kReactBlock];
+  __shared__ uint32_t s_last;
   const uint32_t t = threadIdx.x, i = blockIdx.x * kReactBlock + t;
   cx[t] = i < n ? rx[i] : 0.0f;
   cy[t] = i < n ? ry[i] : 0.0f;
@@ -1492,41 +1522,51 @@ __global__ __launch_bounds__(kReactBlock) void k_reduce_reaction(const float* __
     __syncthreads();
   }
   if (t == 0) {
-    bx[blockIdx.x] = cx[0];
-    by[blockIdx.x] = cy[0];
-    bm[blockIdx.x] = cm[0];
+    if (blockIdx.x < blocks) {
+      bx[blockIdx.x] = cx[0];
+      by[blockIdx.x] = cy[0];
+      bm[blockIdx.x] = cm[0];
+    }
+    __threadfence();
+    s_last = atomicAdd(ticket, 1u) + 1u == gridDim.x;
   }
-}
-
-// The block sums added in order (src/functions.cu:505-513, there on the
-// host), one lane per quantity, then the kinematic move of the controlled
-// particle (src/main.cu:510-514) when `move` is set.
-__global__ __launch_bounds__(64) void k_control_finish(const float* __restrict__ bx, const float* __restrict__ by,
-                                                      const float* __restrict__ bm, uint32_t blocks,
-                                                      float* __restrict__ reaction, dem_controlled* state, int move) {
-  const uint32_t t = threadIdx.x;
-  if (t < 3) {
-    const float* b = t == 0 ? bx : (t == 1 ? by : bm);
-    float acc = 0.0f;
-    for (uint32_t k = 0; k < blocks; ++k) acc += b[k];
-    reaction[t] = acc;
+  __syncthreads();
+  if (!s_last) return;
+  __threadfence();
+  // the block sums to LDS (512 at a time), from where one lane a quantity adds them
+  float acc = 0.0f;
+  for (uint32_t b0 = 0; b0 < blocks; b0 += kReactBlock) {
+    __syncthreads();
+    if (b0 + t < blocks) {
+      cx[t] = bx[b0 + t];
+      cy[t] = by[b0 + t];
+      cm[t] = bm[b0 + t];
+    }
+    __syncthreads();
+    if (t < 3) {
+      const float* v = t == 0 ? cx : (t == 1 ? cy : cm);
+      for (uint32_t k = 0; k < min(blocks - b0, kReactBlock); ++k) acc += v[k];
+    }
   }
-  if (t == 0 && move) {
-    dem_controlled& C = *state;
-    C.pos[0] = (float)((double)C.pos[0] + C.move[0]);
-    C.pos[1] = (float)((double)C.pos[1] + C.move[1]);
-    if ((double)C.pos[1] < C.wrap_below_y) C.pos[1] = C.reset_y;
-    if ((double)C.pos[0] > C.wrap_above_x) C.pos[0] = C.reset_x;
+  if (t < 3) reaction[t] = acc;
+  if (t == 0) {
+    *ticket = 0u;
+    if (move) {
+      dem_controlled& C = *state;
+      C.pos[0] = (float)((double)C.pos[0] + C.move[0]);
+      C.pos[1] = (float)((double)C.pos[1] + C.move[1]);
+      if ((double)C.pos[1] < C.wrap_below_y) C.pos[1] = C.reset_y;
+      if ((double)C.pos[0] > C.wrap_above_x) C.pos[0] = C.reset_x;
+    }
   }
 }
 
 hipError_t launch_control_finish(hipStream_t s, const ControlOut& ctl, float* bx, float* by, float* bm, uint32_t n,
                                  float* reaction, dem_controlled* state, bool move) {
   const uint32_t blocks = (n + kReactBlock - 1u) / kReactBlock;
-  if (n) hipLaunchKernelGGL(k_reduce_reaction, dim3(blocks), dim3(kReactBlock), 0, s, ctl.react_x, ctl.react_y,
-                            ctl.react_m, bx, by, bm, n);
-  hipLaunchKernelGGL(k_control_finish, dim3(1), dim3(64), 0, s, bx, by, bm, n ? blocks : 0u, reaction, state,
-                     move ? 1 : 0);
+  uint32_t* ticket = reinterpret_cast<uint32_t*>(reaction + 3);
+  hipLaunchKernelGGL(k_reduce_reaction, dim3(blocks ? blocks : 1u), dim3(kReactBlock), 0, s, ctl.react_x, ctl.react_y,
+                     ctl.react_m, bx, by, bm, n, blocks, reaction, state, move ? 1 : 0, ticket);
   return hipGetLastError();
 }
 
@@ -1555,8 +1595,9 @@ hipError_t launch_integrate_to(const StepConst& c, hipStream_t s, int block, con
                      gat, quiet, n)
 #define DEM_INTEGRATE_X(R, M, P)            \
   do {                                      \
-    if (next) DEM_INTEGRATE(R, M, true, P); \
-    else DEM_INTEGRATE(R, M, false, P);     \
+    if (next && next->list) DEM_INTEGRATE(R, M, 2, P); \
+    else if (next) DEM_INTEGRATE(R, M, 1, P);          \
+    else DEM_INTEGRATE(R, M, 0, P);                    \
   } while (0)
 #define DEM_INTEGRATE_P(P)                                                \
   do {                                                                    \

@@ -327,6 +327,8 @@ int dem_plot_particles(dem_context* ctx, uint8_t* image, const float* pos, const
       DEM_HIP(ctx, hipMalloc((void**)&ctx->d_stage_control, sizeof(dem_controlled) + 4 * sizeof(float)),
               "hipMalloc(controlled)");
       ctx->d_stage_reaction = (float*)(ctx->d_stage_control + 1);
+      DEM_HIP(ctx, dem::launch_fill(ctx->stream, (uint32_t*)ctx->d_stage_reaction, 0u, 4), "controlled");
+      DEM_HIP(ctx, hipStreamSynchronize(ctx->stream), "controlled");
     }
     DEM_HIP(ctx, hipMemcpyAsync(ctx->d_stage_control, control, sizeof(dem_controlled), hipMemcpyHostToDevice,
                                 ctx->stream),

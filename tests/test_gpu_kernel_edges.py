@@ -137,3 +137,91 @@ def test_sort_tile_edges(gpu_ctx, n, key_bits, offset):
     order = np.argsort(k, kind="stable")
     assert np.array_equal(dk.cpu().numpy().view(np.uint32), k[order])
     assert np.array_equal(dv.cpu().numpy().view(np.uint32), order.astype(np.uint32))
+
+
+def walkers(n, seed, cells, speed):
+    """n discs strewn over cells x cells cells (mostly empty ones), moving
+    fast enough that some change cell every step."""
+    s = sc.column_collapse(seed=seed, cols=n, n=n, box=(cells * 0.011, cells * 0.011), dt=1e-4)
+    rng = np.random.default_rng(seed)
+    s.pos[:] = rng.uniform(0.02, cells * 0.011 - 0.02, s.pos.shape).astype(np.float32)
+    s.vel[:] = (rng.normal(size=s.vel.shape) * speed).astype(np.float32)
+    return s
+
+
+# few discs in many cells (a mover's next occupied cell is far away), movers
+# around the 512 whose order fits LDS, and far more of them
+WHOLE = {
+    "one": lambda: walkers(1, 1, 40, 50.0),
+    "strewn": lambda: walkers(300, 2, 500, 20.0),
+    "hundreds": lambda: walkers(6000, 3, 300, 4.0),
+    "about_512": lambda: walkers(8200, 4, 200, 2.9),
+    "most": lambda: walkers(3000, 5, 100, 90.0),
+}
+
+
+@pytest.mark.parametrize("name", list(WHOLE))
+@pytest.mark.parametrize("fused", [False, True])
+def test_whole_resort_equals_radix(gpu_ctx, name, fused):
+    s = WHOLE[name]()
+    gpu_ctx.set_step_variant(fused=fused, contact_lists=True)
+    a, b = api.Simulation(gpu_ctx, s), api.Simulation(gpu_ctx, s)
+    a.set_sort_mode(1)
+    b.set_sort_mode(2)
+    movers = []
+    try:
+        for steps in (1, 1, 1, 2, 4, 9):
+            a.step(steps)
+            (b.step_graph if steps > 1 else b.step)(steps)
+            movers.append(b.mover_count())
+            da, db = a.download(), b.download()
+            for k in FIELDS:
+                assert bits_equal(da[k], db[k]), (k, steps)
+        print(name, fused, movers, flush=True)
+        assert max(movers) > 0 or name == "one"
+    finally:
+        a.close()
+        b.close()
+
+
+@pytest.mark.parametrize("speed", [0.02, 2.0, 30.0])
+@pytest.mark.parametrize("fused", [False, True])
+def test_inplace_resort_of_large_states(gpu_ctx, speed, fused):
+    """Past 262,144 discs re-sorted steps run in place: few movers, thousands
+    (the movers workgroup's radix path beyond 4,096) and half the state."""
+    s = walkers(262145 + 4096, 6, 700, speed)
+    gpu_ctx.set_step_variant(fused=fused, contact_lists=True)
+    a, b = api.Simulation(gpu_ctx, s), api.Simulation(gpu_ctx, s)
+    a.set_sort_mode(1)
+    b.set_sort_mode(2)
+    try:
+        for steps in (1, 1, 2, 3):
+            a.step(steps)
+            (b.step_graph if steps > 1 else b.step)(steps)
+            da, db = a.download(), b.download()
+            for k in FIELDS:
+                assert bits_equal(da[k], db[k]), (k, steps)
+        assert b.mover_count() > 0
+    finally:
+        a.close()
+        b.close()
+
+
+def test_variants_changed_between_steps(gpu_ctx):
+    """A step's re-sort reads the movers as the step before listed them: the
+    layouts in turn, eager and replayed, against radix-sorted steps."""
+    s = walkers(5000, 7, 150, 5.0)
+    a, b = api.Simulation(gpu_ctx, s), api.Simulation(gpu_ctx, s)
+    a.set_sort_mode(1)
+    b.set_sort_mode(2)
+    try:
+        for k in range(12):
+            gpu_ctx.set_step_variant(fused=bool(k & 1), copy=k % 3 == 0, contact_lists=k % 4 != 0)
+            a.step(3)
+            (b.step_graph if k & 2 else b.step)(3)
+            da, db = a.download(), b.download()
+            for f in FIELDS:
+                assert bits_equal(da[f], db[f]), (f, k)
+    finally:
+        a.close()
+        b.close()
