@@ -12,7 +12,9 @@
 //                     switch decisions
 //   k_adj_collide   : reverse of the pair law (:235-307) over the 3x3
 //                     neighbourhood, one lane per particle gathering the
-//                     neighbours' force/moment adjoints (no atomics on state)
+//                     neighbours' force/moment adjoints (no atomics on state);
+//                     for large states k_adj_mark lists the particles with
+//                     contacts first and k_adj_listed takes those
 //   k_adj_permute   : adjoint of the sort permutation (scatter; after an
 //                     in-place re-sort of more than kScatterMax particles, in
 //                     place at the moved slots instead)
@@ -42,6 +44,10 @@ constexpr int kParams = 4;  // kn, kt, cn, mu
 // one full scatter (a launch costs more than copying the whole adjoint
 // state); beyond it, only the listed slots are saved and put back.
 constexpr uint32_t kScatterMax = 262144;
+// Up to this many particles the walk over the candidates and the reverse of
+// the pair law are one kernel (65,536 discs in contact: 8.7 us, against 4.8 +
+// 11.2 in two); beyond, where most of a settling state has no contact, two.
+constexpr uint32_t kMarkMin = 262144;
 
 __device__ __forceinline__ uint32_t clampi(uint32_t t, uint32_t count) { return t < count ? t : count - 1u; }
 
@@ -86,6 +92,8 @@ __device__ __forceinline__ void body_of(const Material& m, const float* __restri
 // Adds a lane's gradient contributions for material t: one atomic per
 // parameter per wave when the whole wave shares the material, else per lane.
 __device__ __forceinline__ void flush_grads(double g[kParams], uint32_t t, bool active, double* __restrict__ grad) {
+  // (most waves have no contact or wall hit: nothing to add)
+  if (!__any(active && (g[0] != 0.0 || g[1] != 0.0 || g[2] != 0.0 || g[3] != 0.0))) return;
   const uint32_t t0 = __shfl(t, 0);
   const bool uniform = __all(!active || t == t0);
   if (uniform) {
@@ -498,10 +506,227 @@ __device__ __forceinline__ void adj_candidate(const StepConst& c, const AdjIn& S
   }
 }
 
+// The candidate cells of a particle, as the forward walks them.
+struct AdjCells {
+  Instance in;
+  int gx, gy;
+  bool clamp, vx0, vx2, contiguous;
+  uint32_t x0, x1, x2;
+};
+
+__device__ __forceinline__ AdjCells cells_of(const StepConst& c, const Instance& in, float2 p) {
+  AdjCells k;
+  k.in = in;
+  k.clamp = c.flags & DEM_GRID_CLAMP;
+  k.gx = to_int_sat(floorf(p.x * (float)in.grid[0] / in.extent[0]));
+  k.gy = to_int_sat(floorf(p.y * (float)in.grid[1] / in.extent[1]));
+  if (k.clamp) {
+    k.gx = min(max(k.gx, 0), (int)in.grid[0] - 1);
+    k.gy = min(max(k.gy, 0), (int)in.grid[1] - 1);
+  }
+  const uint32_t G0 = in.grid[0];
+  k.vx0 = !k.clamp || k.gx > 0;
+  k.vx2 = !k.clamp || k.gx < (int)G0 - 1;
+  k.x0 = ((uint32_t)k.gx - 1u) & (k.clamp ? 0xFFFFFFFFu : G0 - 1u);
+  k.x1 = k.clamp ? (uint32_t)k.gx : ((uint32_t)k.gx & (G0 - 1u));
+  k.x2 = ((uint32_t)k.gx + 1u) & (k.clamp ? 0xFFFFFFFFu : G0 - 1u);
+  k.contiguous = k.clamp || (k.x0 + 1u == k.x1 && k.x1 + 1u == k.x2);
+  return k;
+}
+
+// The candidates of particle i within the forward's distance prefilter: bit k
+// of h[y] is candidate rs[y] + k of row y.  Contiguous rows (the usual case):
+// all three rows' candidate ranges are loaded at once, then walked together
+// (three loads in flight).  False where the rows cannot be marked so (one of
+// more than 64 candidates, a wrapping grid's edge).
+template <bool kRadius>
+__device__ __forceinline__ bool mark_rows(const StepConst& c, const AdjIn& S, const AdjCells& q, float2 pA, float rA,
+                                          uint32_t i, const uint32_t* __restrict__ cell_start,
+                                          const uint32_t* __restrict__ cell_end, uint32_t n, uint64_t (&h)[3],
+                                          uint32_t (&rs)[3]) {
+  if (!q.contiguous) return false;
+  const uint32_t G0 = q.in.grid[0], G1 = q.in.grid[1];
+  uint32_t re[3];
+#pragma unroll
+  for (int y = 0; y < 3; ++y) {
+    const int iy = q.gy + y - 1;
+    const bool ok = !q.clamp || (iy >= 0 && iy < (int)G1);
+    const uint32_t cy = q.clamp ? (ok ? (uint32_t)iy : 0u) : ((uint32_t)iy & (G1 - 1u));
+    const uint32_t row = q.in.cell_base + cy * G0;
+    const uint32_t a0 = row + (q.vx0 ? q.x0 : q.x1), a1 = row + q.x1, a2 = row + (q.vx2 ? q.x2 : q.x1);
+    const uint32_t s0r = cell_start[a0], s1r = cell_start[a1], s2r = cell_start[a2];
+    const uint32_t e0r = cell_end[a0], e1r = cell_end[a1], e2r = cell_end[a2];
+    const uint32_t s0 = ok && q.vx0 ? s0r : kEmpty, s1 = ok ? s1r : kEmpty, s2 = ok && q.vx2 ? s2r : kEmpty;
+    const bool n0 = s0 != kEmpty, n1 = s1 != kEmpty, n2 = s2 != kEmpty;
+    rs[y] = n0 ? s0 : (n1 ? s1 : (n2 ? s2 : 0u));
+    re[y] = (n0 || n1 || n2) ? min(n2 ? e2r : (n1 ? e1r : e0r), n) : 0u;
+    if (re[y] < rs[y]) re[y] = rs[y];
+  }
+  const uint32_t len[3] = {re[0] - rs[0], re[1] - rs[1], re[2] - rs[2]};
+  const uint32_t L = max(len[0], max(len[1], len[2]));
+  if (L > 64u) return false;
+  h[0] = h[1] = h[2] = 0u;
+  for (uint32_t k = 0; k < L; ++k) {
+    float2 pb[3];
+    float rb[3];
+    uint32_t jy[3];
+#pragma unroll
+    for (int y = 0; y < 3; ++y) {
+      jy[y] = k < len[y] ? rs[y] + k : i;
+      pb[y] = S.pos[jy[y]];
+      rb[y] = kRadius ? S.radius[jy[y]] : c.mat[clampi(S.type[jy[y]], c.num_types)].radius;
+    }
+#pragma unroll
+    for (int y = 0; y < 3; ++y) {
+      const float rx = pb[y].x - pA.x, ry = pb[y].y - pA.y;
+      const float d2 = rx * rx + ry * ry;
+      const float R = rA + rb[y];
+      const bool maybe = !(d2 > (R * R) * 1.00000095367431640625f) || R < 1.0842022e-19f;
+      h[y] |= (uint64_t)(maybe && jy[y] != i) << k;
+    }
+  }
+  return true;
+}
+
+// The particles with marks, listed tile by tile (kMarkTile sorted particles:
+// the entries of tile b start at b * kMarkTile, count[b] of them); one whose
+// rows cannot be marked is listed with first[0] = kEmpty.
+constexpr uint32_t kMarkTile = 256;
+struct AdjList {
+  uint32_t* count = nullptr;
+  uint32_t* id = nullptr;
+  uint64_t* mask[3] = {};
+  uint32_t* first[3] = {};
+};
+
+// The reverse of the pair law is long and takes 150 registers (three waves a
+// SIMD), while most particles of a sparse state have no contact and nothing
+// to do there.  So for large states the walk over the candidates is a kernel
+// of its own, at full occupancy, that lists the particles with marks, and the
+// law runs over the list: 97 + 26 us for 4.7M discs, against 265 us in one.  (One
+// list for all, an append a wave, took 337 us: 74,000 atomics on one word.)
+template <bool kRadius, bool kMulti>
+__global__ __launch_bounds__(kMarkTile) void k_adj_mark(StepConst c, AdjIn S, const uint32_t* __restrict__ cell_start,
+                                                        const uint32_t* __restrict__ cell_end, AdjList list,
+                                                        uint32_t n) {
+  __shared__ uint32_t s_cnt[kMarkTile / kWave];
+  const uint32_t tile = xcd_block(), i = tile * kMarkTile + threadIdx.x, w = threadIdx.x / (uint32_t)kWave;
+  bool emit = false;
+  uint64_t h[3] = {0u, 0u, 0u};
+  uint32_t rs[3] = {0u, 0u, 0u};
+  if (i < n) {
+    const uint32_t tA = kMulti || !kRadius ? clampi(S.type[i], c.num_types) : 0u;
+    const Instance in = kMulti ? c.inst[clampi(c.mat[tA].inst, c.num_instances)] : c.inst0;
+    const float rA = kRadius ? S.radius[i] : c.mat[tA].radius;
+    const float2 pA = S.pos[i];
+    const bool marked = mark_rows<kRadius>(c, S, cells_of(c, in, pA), pA, rA, i, cell_start, cell_end, n, h, rs);
+    if (!marked) rs[0] = kEmpty;
+    emit = !marked || (h[0] | h[1] | h[2]) != 0u;
+  }
+  const uint64_t lanes = __ballot(emit);
+  if (__lane_id() == 0) s_cnt[w] = (uint32_t)__popcll(lanes);
+  __syncthreads();
+  uint32_t at = tile * kMarkTile + (uint32_t)__popcll(lanes & ((1ull << __lane_id()) - 1ull));
+  for (uint32_t k = 0; k < w; ++k) at += s_cnt[k];
+  if (threadIdx.x == 0) {
+    uint32_t total = 0;
+    for (uint32_t k = 0; k < kMarkTile / kWave; ++k) total += s_cnt[k];
+    list.count[tile] = total;
+  }
+  if (emit) {
+    list.id[at] = i;
+#pragma unroll
+    for (int y = 0; y < 3; ++y) {
+      list.mask[y][at] = h[y];
+      list.first[y][at] = rs[y];
+    }
+  }
+}
+
 // Reverse of the pair law for particle i over its 3x3 neighbourhood, in the
-// forward's candidate order: cells by row (y = -1, 0, 1) and column; the
-// three cells of a row are consecutive keys, walked as one range of sorted
+// forward's candidate order: cells by row (y = -1, 0, 1) and column; the three
+// cells of a row are consecutive keys, walked as one range of sorted
 // candidates (cell by cell where a wrapping grid breaks that at an edge).
+// Candidates out of contact contribute nothing, so the sums over the marks
+// (marked, bits h from candidates rs) are the sums over every candidate, in
+// the same order.  Without marks at hand (find) they are found here.
+template <bool kRadius, bool kMulti, bool kFind>
+__device__ __forceinline__ void adj_particle(const StepConst& c, const AdjIn& S,
+                                             const uint32_t* __restrict__ cell_start,
+                                             const uint32_t* __restrict__ cell_end, uint32_t i, uint32_t tA,
+                                             bool marked, uint64_t (&h)[3], uint32_t (&rs)[3],
+                                             const double2* __restrict__ lF, const double* __restrict__ lM,
+                                             double2* __restrict__ lxp, double2* __restrict__ lvp,
+                                             double* __restrict__ lwp, double* __restrict__ grad, double (&g)[kParams],
+                                             uint32_t n) {
+  AdjA q;
+  q.tA = tA;
+  q.A = c.mat[tA];
+  float massA, inertiaA;
+  body_of<kRadius>(q.A, S.radius, i, q.rA, massA, inertiaA);
+  q.pA = S.pos[i];
+  q.vA = S.vel[i];
+  q.wA = S.omega[i];
+  q.lFA = lF[i];
+  q.lMA = lM[i];
+  q.dx_acc = make_double2(0.0, 0.0);
+  q.drv_acc = make_double2(0.0, 0.0);
+  q.dw_acc = 0.0;
+  const Instance in = kMulti ? c.inst[clampi(q.A.inst, c.num_instances)] : c.inst0;
+  if constexpr (kFind)
+    marked = mark_rows<kRadius>(c, S, cells_of(c, in, q.pA), q.pA, q.rA, i, cell_start, cell_end, n, h, rs);
+  if (marked) {
+#pragma unroll
+    for (int y = 0; y < 3; ++y)
+      for (uint64_t hy = h[y]; hy; hy &= hy - 1u)
+        adj_candidate<kRadius>(c, S, lF, lM, grad, i, rs[y] + (uint32_t)__builtin_ctzll(hy), q, g);
+  } else {
+    const AdjCells k = cells_of(c, in, q.pA);
+    const uint32_t G0 = in.grid[0], G1 = in.grid[1];
+    for (int y = -1; y <= 1; ++y) {
+      const int iy = k.gy + y;
+      uint32_t cy;
+      if (k.clamp) {
+        if (iy < 0 || iy >= (int)G1) continue;
+        cy = (uint32_t)iy;
+      } else {
+        cy = (uint32_t)iy & (G1 - 1u);
+      }
+      const uint32_t row = in.cell_base + cy * G0;
+      if (k.contiguous) {
+        // the row's candidates: from the first non-empty cell's start to the
+        // last non-empty cell's end
+        const uint32_t a0 = row + (k.vx0 ? k.x0 : k.x1), a1 = row + k.x1, a2 = row + (k.vx2 ? k.x2 : k.x1);
+        const uint32_t s0 = k.vx0 ? cell_start[a0] : kEmpty, s1 = cell_start[a1],
+                       s2 = k.vx2 ? cell_start[a2] : kEmpty;
+        const bool n0 = s0 != kEmpty, n1 = s1 != kEmpty, n2 = s2 != kEmpty;
+        if (!(n0 || n1 || n2)) continue;
+        const uint32_t first = n0 ? s0 : (n1 ? s1 : s2);
+        const uint32_t end = min(n2 ? cell_end[a2] : (n1 ? cell_end[a1] : cell_end[a0]), n);
+        for (uint32_t j = first; j < end; ++j) adj_candidate<kRadius>(c, S, lF, lM, grad, i, j, q, g);
+      } else {
+        const uint32_t xs[3] = {k.x0, k.x1, k.x2};
+        for (int x = 0; x < 3; ++x) {
+          const uint32_t key = row + xs[x];
+          const uint32_t st = cell_start[key];
+          if (st == kEmpty) continue;
+          const uint32_t en = min(cell_end[key], n);
+          for (uint32_t j = st; j < en; ++j) adj_candidate<kRadius>(c, S, lF, lM, grad, i, j, q, g);
+        }
+      }
+    }
+  }
+  double2 lxi = lxp[i], lvi = lvp[i];
+  lxi.x -= q.dx_acc.x;
+  lxi.y -= q.dx_acc.y;
+  lvi.x -= q.drv_acc.x;
+  lvi.y -= q.drv_acc.y;
+  lxp[i] = lxi;
+  lvp[i] = lvi;
+  lwp[i] = lwp[i] + (double)q.rA * q.dw_acc;
+}
+
+// ... over every particle (small states),
 template <bool kRadius, bool kMulti>
 __global__ __launch_bounds__(256) void k_adj_collide(StepConst c, AdjIn S, const uint32_t* __restrict__ cell_start,
                                                      const uint32_t* __restrict__ cell_end,
@@ -510,131 +735,59 @@ __global__ __launch_bounds__(256) void k_adj_collide(StepConst c, AdjIn S, const
                                                      double* __restrict__ lwp, double* __restrict__ grad, uint32_t n) {
   const uint32_t i = xcd_block() * blockDim.x + threadIdx.x;
   const bool active = i < n;
-  const uint32_t ii = active ? i : 0u;
-  const uint32_t tA = clampi(S.type[ii], c.num_types);
+  const uint32_t tA = clampi(S.type[active ? i : 0u], c.num_types);
   double g[kParams] = {0.0, 0.0, 0.0, 0.0};
-  if (active) {
-    AdjA q;
-    q.tA = tA;
-    q.A = c.mat[tA];
-    const Instance in = kMulti ? c.inst[clampi(q.A.inst, c.num_instances)] : c.inst0;
-    float massA, inertiaA;
-    body_of<kRadius>(q.A, S.radius, i, q.rA, massA, inertiaA);
-    q.pA = S.pos[i];
-    q.vA = S.vel[i];
-    q.wA = S.omega[i];
-    const bool clamp = c.flags & DEM_GRID_CLAMP;
-    int gx = to_int_sat(floorf(q.pA.x * (float)in.grid[0] / in.extent[0]));
-    int gy = to_int_sat(floorf(q.pA.y * (float)in.grid[1] / in.extent[1]));
-    if (clamp) {
-      gx = min(max(gx, 0), (int)in.grid[0] - 1);
-      gy = min(max(gy, 0), (int)in.grid[1] - 1);
-    }
-    q.lFA = lF[i];
-    q.lMA = lM[i];
-    q.dx_acc = make_double2(0.0, 0.0);
-    q.drv_acc = make_double2(0.0, 0.0);
-    q.dw_acc = 0.0;
-    const uint32_t G0 = in.grid[0], G1 = in.grid[1];
-    const bool vx0 = !clamp || gx > 0, vx2 = !clamp || gx < (int)G0 - 1;
-    const uint32_t x0 = ((uint32_t)gx - 1u) & (clamp ? 0xFFFFFFFFu : G0 - 1u);
-    const uint32_t x1 = clamp ? (uint32_t)gx : ((uint32_t)gx & (G0 - 1u));
-    const uint32_t x2 = ((uint32_t)gx + 1u) & (clamp ? 0xFFFFFFFFu : G0 - 1u);
-    const bool contiguous = clamp || (x0 + 1u == x1 && x1 + 1u == x2);
-    // Contiguous rows (the usual case): all three rows' candidate ranges are
-    // loaded at once; rows of at most 64 candidates are walked together
-    // marking the candidates the forward's prefilter lets through (three
-    // loads in flight), then the pair adjoint runs over the marks in row
-    // order.  Candidates out of contact contribute nothing, so the sums are
-    // the same, in the same order, as walking every candidate.
-    bool walked = false;
-    if (contiguous) {
-      uint32_t rs[3], re[3];
-#pragma unroll
-      for (int y = 0; y < 3; ++y) {
-        const int iy = gy + y - 1;
-        const bool ok = !clamp || (iy >= 0 && iy < (int)G1);
-        const uint32_t cy = clamp ? (ok ? (uint32_t)iy : 0u) : ((uint32_t)iy & (G1 - 1u));
-        const uint32_t row = in.cell_base + cy * G0;
-        const uint32_t a0 = row + (vx0 ? x0 : x1), a1 = row + x1, a2 = row + (vx2 ? x2 : x1);
-        const uint32_t s0r = cell_start[a0], s1r = cell_start[a1], s2r = cell_start[a2];
-        const uint32_t e0r = cell_end[a0], e1r = cell_end[a1], e2r = cell_end[a2];
-        const uint32_t s0 = ok && vx0 ? s0r : kEmpty, s1 = ok ? s1r : kEmpty, s2 = ok && vx2 ? s2r : kEmpty;
-        const bool n0 = s0 != kEmpty, n1 = s1 != kEmpty, n2 = s2 != kEmpty;
-        rs[y] = n0 ? s0 : (n1 ? s1 : (n2 ? s2 : 0u));
-        re[y] = (n0 || n1 || n2) ? min(n2 ? e2r : (n1 ? e1r : e0r), n) : 0u;
-        if (re[y] < rs[y]) re[y] = rs[y];
-      }
-      const uint32_t len0 = re[0] - rs[0], len1 = re[1] - rs[1], len2 = re[2] - rs[2];
-      if (len0 <= 64u && len1 <= 64u && len2 <= 64u) {
-        walked = true;
-        uint64_t h[3] = {0u, 0u, 0u};
-        const uint32_t L = max(len0, max(len1, len2));
-        for (uint32_t k = 0; k < L; ++k) {
-          const uint32_t jy[3] = {k < len0 ? rs[0] + k : i, k < len1 ? rs[1] + k : i, k < len2 ? rs[2] + k : i};
-          float2 pb[3];
-          float rb[3];
-#pragma unroll
-          for (int y = 0; y < 3; ++y) {
-            pb[y] = S.pos[jy[y]];
-            rb[y] = kRadius ? S.radius[jy[y]] : c.mat[clampi(S.type[jy[y]], c.num_types)].radius;
-          }
-#pragma unroll
-          for (int y = 0; y < 3; ++y) {
-            const float rx = pb[y].x - q.pA.x, ry = pb[y].y - q.pA.y;
-            const float d2 = rx * rx + ry * ry;
-            const float R = q.rA + rb[y];
-            const bool maybe = !(d2 > (R * R) * 1.00000095367431640625f) || R < 1.0842022e-19f;
-            h[y] |= (uint64_t)(maybe && jy[y] != i) << k;
-          }
-        }
-#pragma unroll
-        for (int y = 0; y < 3; ++y)
-          for (uint64_t hy = h[y]; hy; hy &= hy - 1u)
-            adj_candidate<kRadius>(c, S, lF, lM, grad, i, rs[y] + (uint32_t)__builtin_ctzll(hy), q, g);
-      }
-    }
-    for (int y = -1; y <= 1 && !walked; ++y) {
-      const int iy = gy + y;
-      uint32_t cy;
-      if (clamp) {
-        if (iy < 0 || iy >= (int)G1) continue;
-        cy = (uint32_t)iy;
-      } else {
-        cy = (uint32_t)iy & (G1 - 1u);
-      }
-      const uint32_t row = in.cell_base + cy * G0;
-      if (contiguous) {
-        // the row's candidates: from the first non-empty cell's start to the
-        // last non-empty cell's end
-        const uint32_t a0 = row + (vx0 ? x0 : x1), a1 = row + x1, a2 = row + (vx2 ? x2 : x1);
-        const uint32_t s0 = vx0 ? cell_start[a0] : kEmpty, s1 = cell_start[a1], s2 = vx2 ? cell_start[a2] : kEmpty;
-        const bool n0 = s0 != kEmpty, n1 = s1 != kEmpty, n2 = s2 != kEmpty;
-        if (!(n0 || n1 || n2)) continue;
-        const uint32_t rs = n0 ? s0 : (n1 ? s1 : s2);
-        const uint32_t re = min(n2 ? cell_end[a2] : (n1 ? cell_end[a1] : cell_end[a0]), n);
-        for (uint32_t j = rs; j < re; ++j) adj_candidate<kRadius>(c, S, lF, lM, grad, i, j, q, g);
-      } else {
-        const uint32_t xs[3] = {x0, x1, x2};
-        for (int k = 0; k < 3; ++k) {
-          const uint32_t key = row + xs[k];
-          const uint32_t st = cell_start[key];
-          if (st == kEmpty) continue;
-          const uint32_t en = min(cell_end[key], n);
-          for (uint32_t j = st; j < en; ++j) adj_candidate<kRadius>(c, S, lF, lM, grad, i, j, q, g);
-        }
-      }
-    }
-    double2 lxi = lxp[i], lvi = lvp[i];
-    lxi.x -= q.dx_acc.x;
-    lxi.y -= q.dx_acc.y;
-    lvi.x -= q.drv_acc.x;
-    lvi.y -= q.drv_acc.y;
-    lxp[i] = lxi;
-    lvp[i] = lvi;
-    lwp[i] = lwp[i] + (double)q.rA * q.dw_acc;
-  }
+  uint64_t h[3];
+  uint32_t rs[3];
+  if (active)
+    adj_particle<kRadius, kMulti, true>(c, S, cell_start, cell_end, i, tA, false, h, rs, lF, lM, lxp, lvp, lwp, grad, g,
+                                        n);
   flush_grads(g, tA, active, grad);
+}
+
+// ... or over the listed ones: a block takes `group` (at most kListTiles)
+// tiles' entries as one list.
+constexpr uint32_t kListTiles = 32;
+template <bool kRadius, bool kMulti>
+__global__ __launch_bounds__(256) void k_adj_listed(StepConst c, AdjIn S, const uint32_t* __restrict__ cell_start,
+                                                    const uint32_t* __restrict__ cell_end, AdjList list,
+                                                    uint32_t tiles, uint32_t group, const double2* __restrict__ lF,
+                                                    const double* __restrict__ lM, double2* __restrict__ lxp,
+                                                    double2* __restrict__ lvp, double* __restrict__ lwp,
+                                                    double* __restrict__ grad, uint32_t n) {
+  __shared__ uint32_t s_end[kListTiles];  // entries of the group's tiles up to and with each
+  const uint32_t t0 = xcd_block() * group;
+  if (threadIdx.x < kListTiles) {
+    const uint32_t t = threadIdx.x;
+    uint32_t x = t < group && t0 + t < tiles ? list.count[t0 + t] : 0u;
+#pragma unroll
+    for (uint32_t o = 1; o < kListTiles; o <<= 1) {
+      const uint32_t y = __shfl_up(x, o);
+      if (t >= o) x += y;
+    }
+    s_end[t] = x;
+  }
+  __syncthreads();
+  const uint32_t listed = s_end[kListTiles - 1u];
+  for (uint32_t e0 = 0; e0 < listed; e0 += blockDim.x) {
+    const uint32_t e = e0 + threadIdx.x;
+    const bool active = e < listed;
+    uint32_t tile = 0;  // the first whose end is above e
+#pragma unroll
+    for (uint32_t step = kListTiles / 2u; step; step >>= 1)
+      if (s_end[tile + step - 1u] <= (active ? e : e0)) tile += step;
+    const uint32_t at = (t0 + tile) * kMarkTile + (active ? e : e0) - (tile ? s_end[tile - 1u] : 0u);
+    const uint32_t i = list.id[at];
+    const uint32_t tA = clampi(S.type[i], c.num_types);
+    double g[kParams] = {0.0, 0.0, 0.0, 0.0};
+    if (active) {
+      uint64_t h[3] = {list.mask[0][at], list.mask[1][at], list.mask[2][at]};
+      uint32_t rs[3] = {list.first[0][at], list.first[1][at], list.first[2][at]};
+      adj_particle<kRadius, kMulti, false>(c, S, cell_start, cell_end, i, tA, rs[0] != kEmpty, h, rs, lF, lM, lxp, lvp,
+                                           lwp, grad, g, n);
+    }
+    flush_grads(g, tA, active, grad);
+  }
 }
 
 inline dim3 grid_of(uint32_t n) { return dim3((n + 255u) / 256u); }
@@ -676,6 +829,7 @@ struct dem_adjoint {
   // adjoint state (FP64)
   double2 *lx = nullptr, *lv = nullptr, *lxp = nullptr, *lvp = nullptr, *lF = nullptr;
   double *lw = nullptr, *lwp = nullptr, *lM = nullptr, *grad = nullptr;
+  AdjList list{};  // the particles with contacts of the step being reversed
   std::vector<void*> allocs;
 };
 
@@ -778,6 +932,15 @@ int dem_adj_create(dem_sim* sim, uint32_t checkpoint_every, dem_adjoint** out) {
   if (!r) r = adj_alloc(a, &a->lF, n);
   if (!r) r = adj_alloc(a, &a->lM, n);
   if (!r) r = adj_alloc(a, &a->grad, (size_t)kParams * DEM_MAX_TYPES);
+  if (n > kMarkMin) {
+    const size_t entries = (n + kMarkTile - 1u) / kMarkTile * kMarkTile;
+    if (!r) r = adj_alloc(a, &a->list.count, entries / kMarkTile);
+    if (!r) r = adj_alloc(a, &a->list.id, entries);
+    for (int y = 0; y < 3; ++y) {
+      if (!r) r = adj_alloc(a, &a->list.mask[y], entries);
+      if (!r) r = adj_alloc(a, &a->list.first[y], entries);
+    }
+  }
   if (!r) r = alloc_checkpoint(a, a->final_state);
   if (r) {
     dem_adj_destroy(a);
@@ -891,21 +1054,32 @@ int dem_adj_backward(dem_adjoint* a, const float* grad_pos, const float* grad_ve
       DEM_HIP(ctx, launch_fill(s, m->cell_start, kEmpty, m->cells), "adj fill");
       hipLaunchKernelGGL(k_cell_bounds, grid_of(n), dim3(256), 0, s, a->skey + off, m->cell_start, m->cell_end, n,
                          m->cells);
-#define DEM_ADJ(K, ...)                                                                                 \
+#define DEM_ADJ(K, GRID, ...)                                                                           \
   do {                                                                                                  \
     if (m->rad) {                                                                                       \
-      if (mul) hipLaunchKernelGGL((K<true, true>), grid_of(n), dim3(256), 0, s, __VA_ARGS__);             \
-      else hipLaunchKernelGGL((K<true, false>), grid_of(n), dim3(256), 0, s, __VA_ARGS__);               \
+      if (mul) hipLaunchKernelGGL((K<true, true>), GRID, dim3(256), 0, s, __VA_ARGS__);                   \
+      else hipLaunchKernelGGL((K<true, false>), GRID, dim3(256), 0, s, __VA_ARGS__);                     \
     } else {                                                                                            \
-      if (mul) hipLaunchKernelGGL((K<false, true>), grid_of(n), dim3(256), 0, s, __VA_ARGS__);            \
-      else hipLaunchKernelGGL((K<false, false>), grid_of(n), dim3(256), 0, s, __VA_ARGS__);              \
+      if (mul) hipLaunchKernelGGL((K<false, true>), GRID, dim3(256), 0, s, __VA_ARGS__);                  \
+      else hipLaunchKernelGGL((K<false, false>), GRID, dim3(256), 0, s, __VA_ARGS__);                    \
     }                                                                                                   \
   } while (0)
-      DEM_ADJ(k_adj_integrate, c, S, (const float2*)(a->sacc + off), (const float*)(a->salpha + off),
+      DEM_ADJ(k_adj_integrate, grid_of(n), c, S, (const float2*)(a->sacc + off), (const float*)(a->salpha + off),
               (const double2*)a->lx,
               (const double2*)a->lv, (const double*)a->lw, a->lxp, a->lvp, a->lwp, a->lF, a->lM, a->grad, n);
-      DEM_ADJ(k_adj_collide, c, S, (const uint32_t*)m->cell_start, (const uint32_t*)m->cell_end,
-              (const double2*)a->lF, (const double*)a->lM, a->lxp, a->lvp, a->lwp, a->grad, n);
+      if (n <= kMarkMin) {
+        DEM_ADJ(k_adj_collide, grid_of(n), c, S, (const uint32_t*)m->cell_start, (const uint32_t*)m->cell_end,
+                (const double2*)a->lF, (const double*)a->lM, a->lxp, a->lvp, a->lwp, a->grad, n);
+      } else {
+        // groups of tiles as large as leave four blocks a CU
+        const uint32_t tiles = (n + kMarkTile - 1u) / kMarkTile;
+        const uint32_t group = std::min(kListTiles, std::max(1u, tiles / 1024u));
+        DEM_ADJ(k_adj_mark, dim3(tiles), c, S, (const uint32_t*)m->cell_start, (const uint32_t*)m->cell_end, a->list,
+                n);
+        DEM_ADJ(k_adj_listed, dim3((tiles + group - 1u) / group), c, S, (const uint32_t*)m->cell_start,
+                (const uint32_t*)m->cell_end, a->list, tiles, group, (const double2*)a->lF, (const double*)a->lM,
+                a->lxp, a->lvp, a->lwp, a->grad, n);
+      }
 #undef DEM_ADJ
       if (a->slot_inplace[k] && n > kScatterMax) {
         hipLaunchKernelGGL(k_adj_perm_save, grid_of(n), dim3(256), 0, s, a->sindex + off, a->lxp, a->lvp, a->lwp,

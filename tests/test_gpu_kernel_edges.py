@@ -225,3 +225,49 @@ def test_variants_changed_between_steps(gpu_ctx):
     finally:
         a.close()
         b.close()
+
+
+def test_adjoint_of_large_state_lists(gpu_ctx):
+    """Past 262,144 discs the adjoint lists the particles with contacts first:
+    88 copies of one system in a batch (boundaries of tiles and list groups
+    everywhere in it; free, touching and heaped discs) against the system
+    alone, which takes the one-kernel path: gradients of the state bit for
+    bit, of the parameters to the order of their sums."""
+    import dataclasses
+
+    import torch
+
+    one = packed_rows(3001, seed=9)
+    one.pos[1000:2000, 0] *= np.float32(1.02)
+    one.pos[1000:2000, 1] += np.float32(0.2)  # (free discs)
+    copies = 88
+    many = one.copy()
+    for f in ("pos", "vel", "theta", "omega", "radius"):
+        setattr(many, f, np.concatenate([getattr(one, f)] * copies))
+    many.type = np.repeat(np.arange(copies, dtype=np.uint32), one.n)
+    many.id = np.arange(copies * one.n, dtype=np.uint32)
+    many.loc = many.id.copy()
+    g = one.instances[0]
+    many.instances = [dataclasses.replace(g, cell_base=k * g.cells) for k in range(copies)]
+    many.materials = [dataclasses.replace(one.materials[0], instance=k) for k in range(copies)]
+    assert many.n > 262144
+    rng = np.random.default_rng(0)
+    W, V = rng.normal(size=(one.n, 2)).astype(np.float32), rng.normal(size=(one.n, 2)).astype(np.float32)
+    out = []
+    for s, k in ((one, 1), (many, copies)):
+        sim = api.Simulation(gpu_ctx, s)
+        adj = api.Adjoint(sim, checkpoint_every=3)
+        adj.forward(3)
+        gp, gv, par = adj.backward(torch.from_numpy(np.tile(W, (k, 1))).cuda(), torch.from_numpy(np.tile(V, (k, 1))).cuda(),
+                                   num_types=k)
+        out.append((gp.cpu().numpy(), gv.cpu().numpy(), par.cpu().numpy()))
+        adj.close()
+        sim.close()
+    (gp1, gv1, par1), (gpm, gvm, parm) = out
+    assert np.count_nonzero(par1) >= 3
+    for k in (0, 1, 40, copies - 1):
+        at = slice(k * one.n, (k + 1) * one.n)
+        assert bits_equal(gpm[at], gp1) and bits_equal(gvm[at], gv1), k
+    # a sum of n terms in another order: n eps of the terms' magnitudes at most
+    scale = np.abs(par1).max()
+    assert np.all(np.abs(parm - par1) <= 1e-9 * np.maximum(np.abs(par1), 1e-3 * scale))
