@@ -49,6 +49,10 @@ constexpr uint32_t kScatterMax = 262144;
 // 11.2 in two); beyond, where most of a settling state has no contact, two.
 constexpr uint32_t kMarkMin = 262144;
 
+// Threads a workgroup of every kernel here (a constant: a kernel that asks the
+// runtime begins with a vector load and a wait for it).
+constexpr uint32_t kAdjBlock = 256;
+
 __device__ __forceinline__ uint32_t clampi(uint32_t t, uint32_t count) { return t < count ? t : count - 1u; }
 
 __device__ __forceinline__ float series_f(float a, float b) {
@@ -67,13 +71,6 @@ __device__ __forceinline__ void series_grad(double a, double b, double& da, doub
 }
 
 __device__ __forceinline__ double sgn(double x) { return x > 0.0 ? 1.0 : (x < 0.0 ? -1.0 : 0.0); }
-
-// Same conversion as the forward kernels: NaN -> 0, saturation, truncation.
-__device__ __forceinline__ int to_int_sat(float g) {
-  int r = (int)fminf(fmaxf(g, -2147483648.0f), 2147483520.0f);
-  r = (g >= 2147483648.0f) ? 2147483647 : r;
-  return (g == g) ? r : 0;
-}
 
 template <bool kRadius>
 __device__ __forceinline__ void body_of(const Material& m, const float* __restrict__ radius, uint32_t i, float& r,
@@ -128,7 +125,7 @@ struct AdjIn {
 __global__ void k_adj_init(const uint32_t* __restrict__ id, const float* __restrict__ gpos,
                            const float* __restrict__ gvel, double2* __restrict__ lx, double2* __restrict__ lv,
                            double* __restrict__ lw, uint32_t n) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t i = blockIdx.x * kAdjBlock + threadIdx.x;
   if (i >= n) return;
   const uint32_t d = min(id[i], n - 1u);
   lx[i] = gpos ? make_double2(gpos[2 * d], gpos[2 * d + 1]) : make_double2(0.0, 0.0);
@@ -139,7 +136,7 @@ __global__ void k_adj_init(const uint32_t* __restrict__ id, const float* __restr
 __global__ void k_adj_out(const uint32_t* __restrict__ id, const double2* __restrict__ lx,
                           const double2* __restrict__ lv, float* __restrict__ gpos0, float* __restrict__ gvel0,
                           uint32_t n) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t i = blockIdx.x * kAdjBlock + threadIdx.x;
   if (i >= n) return;
   const uint32_t d = id[i];
   if (d >= n) return;
@@ -167,7 +164,7 @@ __global__ void k_store_slot(const float2* __restrict__ pos, const float2* __res
                              float* __restrict__ somega, float* __restrict__ sradius, uint32_t* __restrict__ stype,
                              uint32_t* __restrict__ sindex, uint32_t* __restrict__ skey, float2* __restrict__ sacc,
                              float* __restrict__ salpha, uint32_t n) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t i = blockIdx.x * kAdjBlock + threadIdx.x;
   if (i >= n) return;
   spos[i] = pos[i];
   svel[i] = vel[i];
@@ -184,7 +181,7 @@ __global__ void k_store_slot(const float2* __restrict__ pos, const float2* __res
 // cellStart/cellEnd of sorted keys (cellStart pre-filled with EMPTY)
 __global__ void k_cell_bounds(const uint32_t* __restrict__ key, uint32_t* __restrict__ cs, uint32_t* __restrict__ ce,
                               uint32_t n, uint32_t num_cells) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t i = blockIdx.x * kAdjBlock + threadIdx.x;
   if (i >= n) return;
   const uint32_t h = key[i];
   if (i == 0 || h != key[i - 1]) {
@@ -198,7 +195,7 @@ __global__ void k_adj_permute(const uint32_t* __restrict__ index, const double2*
                               const double2* __restrict__ lvp, const double* __restrict__ lwp,
                               double2* __restrict__ lx, double2* __restrict__ lv, double* __restrict__ lw,
                               uint32_t n) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t i = blockIdx.x * kAdjBlock + threadIdx.x;
   if (i >= n) return;
   const uint32_t src = index[i];
   if (src >= n) return;
@@ -216,7 +213,7 @@ __global__ void k_adj_perm_save(const uint32_t* __restrict__ index, const double
                                 const double2* __restrict__ lvp, const double* __restrict__ lwp,
                                 double2* __restrict__ tx, double2* __restrict__ tv, double* __restrict__ tw,
                                 uint32_t n) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t i = blockIdx.x * kAdjBlock + threadIdx.x;
   if (i >= n || index[i] == i) return;
   tx[i] = lxp[i];
   tv[i] = lvp[i];
@@ -227,7 +224,7 @@ __global__ void k_adj_perm_put(const uint32_t* __restrict__ index, const double2
                                const double2* __restrict__ tv, const double* __restrict__ tw,
                                double2* __restrict__ lxp, double2* __restrict__ lvp, double* __restrict__ lwp,
                                uint32_t n) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t i = blockIdx.x * kAdjBlock + threadIdx.x;
   if (i >= n) return;
   const uint32_t src = index[i];
   if (src == i || src >= n) return;
@@ -246,7 +243,7 @@ __global__ __launch_bounds__(256) void k_adj_integrate(StepConst c, AdjIn S, con
                                                        double2* __restrict__ lvp, double* __restrict__ lwp,
                                                        double2* __restrict__ lF, double* __restrict__ lM,
                                                        double* __restrict__ grad, uint32_t n) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t i = blockIdx.x * kAdjBlock + threadIdx.x;
   const bool active = i < n;
   const uint32_t ii = active ? i : 0u;
   const uint32_t t = clampi(S.type[ii], c.num_types);
@@ -518,8 +515,7 @@ __device__ __forceinline__ AdjCells cells_of(const StepConst& c, const Instance&
   AdjCells k;
   k.in = in;
   k.clamp = c.flags & DEM_GRID_CLAMP;
-  k.gx = to_int_sat(floorf(p.x * (float)in.grid[0] / in.extent[0]));
-  k.gy = to_int_sat(floorf(p.y * (float)in.grid[1] / in.extent[1]));
+  grid_pos(in, p, k.gx, k.gy);
   if (k.clamp) {
     k.gx = min(max(k.gx, 0), (int)in.grid[0] - 1);
     k.gy = min(max(k.gy, 0), (int)in.grid[1] - 1);
@@ -733,7 +729,7 @@ __global__ __launch_bounds__(256) void k_adj_collide(StepConst c, AdjIn S, const
                                                      const double2* __restrict__ lF, const double* __restrict__ lM,
                                                      double2* __restrict__ lxp, double2* __restrict__ lvp,
                                                      double* __restrict__ lwp, double* __restrict__ grad, uint32_t n) {
-  const uint32_t i = xcd_block() * blockDim.x + threadIdx.x;
+  const uint32_t i = xcd_block() * kAdjBlock + threadIdx.x;
   const bool active = i < n;
   const uint32_t tA = clampi(S.type[active ? i : 0u], c.num_types);
   double g[kParams] = {0.0, 0.0, 0.0, 0.0};
@@ -769,7 +765,7 @@ __global__ __launch_bounds__(256) void k_adj_listed(StepConst c, AdjIn S, const 
   }
   __syncthreads();
   const uint32_t listed = s_end[kListTiles - 1u];
-  for (uint32_t e0 = 0; e0 < listed; e0 += blockDim.x) {
+  for (uint32_t e0 = 0; e0 < listed; e0 += kAdjBlock) {
     const uint32_t e = e0 + threadIdx.x;
     const bool active = e < listed;
     uint32_t tile = 0;  // the first whose end is above e
@@ -790,7 +786,7 @@ __global__ __launch_bounds__(256) void k_adj_listed(StepConst c, AdjIn S, const 
   }
 }
 
-inline dim3 grid_of(uint32_t n) { return dim3((n + 255u) / 256u); }
+inline dim3 grid_of(uint32_t n) { return dim3((n + kAdjBlock - 1u) / kAdjBlock); }
 
 }  // namespace
 }  // namespace dem
@@ -884,7 +880,7 @@ hipError_t store_slot_hook(void* user, dem_sim* m, hipStream_t s, int dyn, int s
   const size_t off = a->slot_off;
   const uint32_t n = m->n;
   a->slot_inplace[off / n] = list ? 1 : 0;
-  hipLaunchKernelGGL(k_store_slot, grid_of(n), dim3(256), 0, s, m->pos[dyn], m->vel[dyn], m->omega[dyn],
+  hipLaunchKernelGGL(k_store_slot, grid_of(n), dim3(kAdjBlock), 0, s, m->pos[dyn], m->vel[dyn], m->omega[dyn],
                      m->rad ? m->radius[stat] : nullptr, m->type[stat], list ? nullptr : m->sorted_idx,
                      m->sorted_key, m->acc, m->alpha, m->acc_lazy ? m->quiet : nullptr,
                      a->spos + off, a->svel + off, a->somega + off, a->sradius ? a->sradius + off : nullptr,
@@ -1021,7 +1017,7 @@ int dem_adj_backward(dem_adjoint* a, const float* grad_pos, const float* grad_ve
   const StepConst& c = ctx->c;
   const bool mul = multi(ctx);
   // adjoint of the final state, from gradients given by particle id
-  hipLaunchKernelGGL(k_adj_init, grid_of(n), dim3(256), 0, s, a->final_state.id, grad_pos, grad_vel, a->lx, a->lv,
+  hipLaunchKernelGGL(k_adj_init, grid_of(n), dim3(kAdjBlock), 0, s, a->final_state.id, grad_pos, grad_vel, a->lx, a->lv,
                      a->lw, n);
   DEM_HIP(ctx, hipMemsetAsync(a->grad, 0, sizeof(double) * kParams * c.num_types, s), "grad reset");
   const uint32_t nseg = (a->steps + a->K - 1) / a->K;
@@ -1052,16 +1048,16 @@ int dem_adj_backward(dem_adjoint* a, const float* grad_pos, const float* grad_ve
       const size_t off = (size_t)k * n;
       AdjIn S{a->spos + off, a->svel + off, a->somega + off, a->sradius ? a->sradius + off : nullptr, a->stype + off};
       DEM_HIP(ctx, launch_fill(s, m->cell_start, kEmpty, m->cells), "adj fill");
-      hipLaunchKernelGGL(k_cell_bounds, grid_of(n), dim3(256), 0, s, a->skey + off, m->cell_start, m->cell_end, n,
+      hipLaunchKernelGGL(k_cell_bounds, grid_of(n), dim3(kAdjBlock), 0, s, a->skey + off, m->cell_start, m->cell_end, n,
                          m->cells);
 #define DEM_ADJ(K, GRID, ...)                                                                           \
   do {                                                                                                  \
     if (m->rad) {                                                                                       \
-      if (mul) hipLaunchKernelGGL((K<true, true>), GRID, dim3(256), 0, s, __VA_ARGS__);                   \
-      else hipLaunchKernelGGL((K<true, false>), GRID, dim3(256), 0, s, __VA_ARGS__);                     \
+      if (mul) hipLaunchKernelGGL((K<true, true>), GRID, dim3(kAdjBlock), 0, s, __VA_ARGS__);                   \
+      else hipLaunchKernelGGL((K<true, false>), GRID, dim3(kAdjBlock), 0, s, __VA_ARGS__);                     \
     } else {                                                                                            \
-      if (mul) hipLaunchKernelGGL((K<false, true>), GRID, dim3(256), 0, s, __VA_ARGS__);                  \
-      else hipLaunchKernelGGL((K<false, false>), GRID, dim3(256), 0, s, __VA_ARGS__);                    \
+      if (mul) hipLaunchKernelGGL((K<false, true>), GRID, dim3(kAdjBlock), 0, s, __VA_ARGS__);                  \
+      else hipLaunchKernelGGL((K<false, false>), GRID, dim3(kAdjBlock), 0, s, __VA_ARGS__);                    \
     }                                                                                                   \
   } while (0)
       DEM_ADJ(k_adj_integrate, grid_of(n), c, S, (const float2*)(a->sacc + off), (const float*)(a->salpha + off),
@@ -1082,9 +1078,9 @@ int dem_adj_backward(dem_adjoint* a, const float* grad_pos, const float* grad_ve
       }
 #undef DEM_ADJ
       if (a->slot_inplace[k] && n > kScatterMax) {
-        hipLaunchKernelGGL(k_adj_perm_save, grid_of(n), dim3(256), 0, s, a->sindex + off, a->lxp, a->lvp, a->lwp,
+        hipLaunchKernelGGL(k_adj_perm_save, grid_of(n), dim3(kAdjBlock), 0, s, a->sindex + off, a->lxp, a->lvp, a->lwp,
                            a->lx, a->lv, a->lw, n);
-        hipLaunchKernelGGL(k_adj_perm_put, grid_of(n), dim3(256), 0, s, a->sindex + off, a->lx, a->lv, a->lw,
+        hipLaunchKernelGGL(k_adj_perm_put, grid_of(n), dim3(kAdjBlock), 0, s, a->sindex + off, a->lx, a->lv, a->lw,
                            a->lxp, a->lvp, a->lwp, n);
         std::swap(a->lx, a->lxp);
         std::swap(a->lv, a->lvp);
@@ -1093,14 +1089,14 @@ int dem_adj_backward(dem_adjoint* a, const float* grad_pos, const float* grad_ve
         // the full scatter (for an in-place step too, whose stored index is
         // the identity outside its listed slots: one launch instead of two,
         // which is faster wherever launches cost more than the whole copy)
-        hipLaunchKernelGGL(k_adj_permute, grid_of(n), dim3(256), 0, s, a->sindex + off, a->lxp, a->lvp, a->lwp,
+        hipLaunchKernelGGL(k_adj_permute, grid_of(n), dim3(kAdjBlock), 0, s, a->sindex + off, a->lxp, a->lvp, a->lwp,
                            a->lx, a->lv, a->lw, n);
       }
       DEM_HIP(ctx, hipGetLastError(), "adjoint kernels");
     }
   }
   // lx/lv now follow the order of the first checkpoint
-  hipLaunchKernelGGL(k_adj_out, grid_of(n), dim3(256), 0, s, a->ckpt[0].id, a->lx, a->lv, grad_pos0, grad_vel0, n);
+  hipLaunchKernelGGL(k_adj_out, grid_of(n), dim3(kAdjBlock), 0, s, a->ckpt[0].id, a->lx, a->lv, grad_pos0, grad_vel0, n);
   if (grad_params)
     DEM_HIP(ctx, hipMemcpyAsync(grad_params, a->grad, sizeof(double) * kParams * c.num_types, hipMemcpyDeviceToDevice, s),
             "grad copy");

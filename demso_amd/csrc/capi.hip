@@ -190,6 +190,11 @@ Instance make_instance(const float box[2], const float extent[2], const uint32_t
   in.grid[0] = grid[0];
   in.grid[1] = grid[1];
   in.cell_base = base;
+  for (int k = 0; k < 2; ++k) {
+    // rounded towards zero (grid_pos): the product is exact in the fma
+    const double e = (double)in.extent[k], y = 1.0 / e;
+    in.inv[k] = std::fma(y, e, -1.0) > 0.0 ? std::nextafter(y, 0.0) : y;
+  }
   return in;
 }
 

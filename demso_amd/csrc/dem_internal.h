@@ -23,12 +23,14 @@ struct alignas(16) Material {
   uint32_t inst, pad;
 };
 
-// Instance geometry (32 bytes): wall box, hashing extent, grid, key base.
+// Instance geometry (48 bytes): wall box, hashing extent, grid, key base, and
+// 1 / extent in double, rounded towards zero (grid_pos).
 struct alignas(16) Instance {
   float box[2];
   float extent[2];
   uint32_t grid[2];
   uint32_t cell_base, pad;
+  double inv[2];
 };
 
 // Uniform step parameters, passed by value to every kernel (kernarg ->
@@ -52,6 +54,9 @@ struct StepConst {
   // and cn, in double; null above kDPairMaxTypes material rows.
   const double* dpair;
   Instance inst0;
+  // Threads a workgroup, set by the launcher: a kernel that asks the runtime
+  // (blockDim) begins with a vector load and a wait for it.
+  uint32_t block;
 };
 constexpr uint32_t kDPairMaxTypes = 1024;
 // Material rows per context (the pair table holds up to kMaxTypes^2 entries).
@@ -78,6 +83,24 @@ __device__ __forceinline__ uint32_t xcd_block() {
   const uint32_t nb = gridDim.x, b = blockIdx.x;
   const uint32_t x = b % kXcds, local = b / kXcds, q = nb / kXcds, r = nb % kXcds;
   return x * q + min(x, r) + local;
+}
+
+// calcGridPos (src/particles_kernel.cuh:114-121): floor(p * G / extent), the
+// quotient rounded to float; NaN gives 0, a float beyond the int range the
+// nearest end of it, which is what the conversion instruction does.
+// The quotient is taken as a * (1 / extent) in double: that is within 2^-51
+// of a / extent, which lies at least 2^-49 (relatively) from every midpoint
+// of two normal floats, as a and extent have 24 bits (a 25-bit midpoint times
+// a 24-bit extent has 49), so the product rounds to the same float.  Of the
+// results below the normal floats only their sign matters, and whether they
+// round to zero: 1 / extent is never too large, so half the smallest float
+// still does.  Three operations instead of a division's eleven, one instead of
+// seven that clamp the conversion in software.
+__device__ __forceinline__ void grid_pos(const Instance& in, float2 p, int& gx, int& gy) {
+  const float qx = (float)((double)(p.x * (float)in.grid[0]) * in.inv[0]);
+  const float qy = (float)((double)(p.y * (float)in.grid[1]) * in.inv[1]);
+  asm("v_cvt_i32_f32 %0, %1" : "=v"(gx) : "v"(floorf(qx)));
+  asm("v_cvt_i32_f32 %0, %1" : "=v"(gy) : "v"(floorf(qy)));
 }
 
 // Launch helpers (defined in the .hip files).

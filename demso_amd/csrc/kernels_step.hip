@@ -17,21 +17,8 @@
 namespace dem {
 namespace {
 
-__device__ __forceinline__ int to_int_sat(float g) {
-  // NaN -> 0, saturation at the int range, plain truncation inside it
-  int r = (int)fminf(fmaxf(g, -2147483648.0f), 2147483520.0f);
-  r = (g >= 2147483648.0f) ? 2147483647 : r;
-  return (g == g) ? r : 0;
-}
-
 __device__ __forceinline__ uint32_t clamp_idx(uint32_t t, uint32_t count) {
   return t < count ? t : count - 1u;
-}
-
-// calcGridPos (src/particles_kernel.cuh:114-121): floor(p * G / extent).
-__device__ __forceinline__ void grid_pos(const Instance& in, float2 p, int& gx, int& gy) {
-  gx = to_int_sat(floorf(p.x * (float)in.grid[0] / in.extent[0]));
-  gy = to_int_sat(floorf(p.y * (float)in.grid[1] / in.extent[1]));
 }
 
 __device__ __forceinline__ void clamp_cell(const Instance& in, int& gx, int& gy) {
@@ -53,7 +40,10 @@ __device__ __forceinline__ void body(const Material& m, const float* __restrict_
   if (kRadius) {
     r = radius[i];
     mass = (m.areal * r) * r;
-    inertia = (((2.0f * mass) * r) * r) / 5.0f;
+    // t / 5 rounded to float: 0.2 is within 2^-53 of 1/5 and t / 5 at least
+    // 2^-28 from every midpoint of two floats (and never one), so the
+    // product in double rounds to the same float
+    inertia = (float)((double)(((2.0f * mass) * r) * r) * 0.2);
   } else {
     r = m.radius;
     mass = m.mass;
@@ -123,10 +113,10 @@ __global__ __launch_bounds__(256) void k_hash(StepConst c, const float2* __restr
                                               const uint32_t* __restrict__ type,
                                               uint32_t* __restrict__ hash,
                                               uint32_t* __restrict__ index, uint32_t n) {
-  const uint32_t base = blockIdx.x * blockDim.x * kPer + threadIdx.x;
+  const uint32_t base = blockIdx.x * c.block * kPer + threadIdx.x;
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
-    const uint32_t i = base + (uint32_t)k * blockDim.x;
+    const uint32_t i = base + (uint32_t)k * c.block;
     if (i < n) {
       hash[i] = cell_key<kMulti>(c, pos[i], type, i);
       index[i] = i;
@@ -247,7 +237,8 @@ struct PairCtx {
 // ulp/(2y) by less than one step of it, so q2 + r y and a/den lie on the same
 // side of every rounding midpoint, and a/den is never one).  a is a float
 // length and den = 4 pi r^2 of a float r, so no step overflows or underflows
-// in double; a non-finite length divides as the reference does.  Five FP64
+// in double.  The remainder is not finite only where the length is not or den
+// is zero or infinite, and there a y already is a / den.  Five FP64
 // operations per contact instead of a division sequence.
 __device__ __forceinline__ double pressure_quotient(float len, double den, double rden) {
   const double a = (double)len;
@@ -256,8 +247,6 @@ __device__ __forceinline__ double pressure_quotient(float len, double den, doubl
   if (__builtin_expect(__builtin_isfinite(rem), 1)) {
     qd = fma(rem, rden, qd);
     qd = fma(fma(-qd, den, a), rden, qd);
-  } else {
-    qd = a / den;
   }
   return qd;
 }
@@ -266,18 +255,68 @@ __device__ __forceinline__ float add_pressure_recip(float p, float len, double d
   return (float)((double)p + pressure_quotient(len, den, rden));
 }
 
+// RN(sqrt(x)) and y = 1 / sqrt(x) to within 2^-20 (NaN where x is not in
+// [2^-96, 2^96]: NaN, 0 and the far ends take sqrtf).  One correction of
+// x * v_rsq(x) is correctly rounded for every one of these floats (all
+// 1.6 billion compared with sqrtf on gfx950): five operations instead of
+// sqrtf's seventeen, which scale and test two neighbours.
+__device__ __forceinline__ float root(float x, float& y) {
+  y = __builtin_nanf("");
+  if (__builtin_expect(!(x >= 0x1p-96f && x <= 0x1p96f), 0)) return sqrtf(x);
+  y = __builtin_amdgcn_rsqf(x);
+  const float s = x * y;
+  return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
+}
+
+// a / b and c / b rounded to float, given y within 2^-20 of 1 / b (or NaN).
+// 1 / b in double (e = 1 - b y, y (1 + e + e^2): within 2^-52 of it for every
+// b and y that root() returns), times a: within 2^-51 of a / b, which lies at
+// least 2^-49 from every midpoint of two normal floats (a midpoint of 25 bits
+// times b's 24 has 49), so the product rounds to the same float.  Where a
+// quotient is subnormal or NaN (so for y NaN) both are divided.  Thirteen
+// operations for the two instead of 22.
+__device__ __forceinline__ void quotients(float a, float c, float b, float y, float& qa, float& qc) {
+  const double bd = (double)b, yd = (double)y;
+  const double e = __builtin_fma(-bd, yd, 1.0);
+  const double inv = __builtin_fma(yd, __builtin_fma(e, e, e), yd);
+  qa = (float)((double)a * inv);
+  qc = (float)((double)c * inv);
+  constexpr int kOdd = 0x3 | 0x10 | 0x80;  // NaN, subnormal
+  if (__builtin_expect(__builtin_amdgcn_classf(qa, kOdd) || __builtin_amdgcn_classf(qc, kOdd), 0)) {
+    qa = a / b;
+    qc = c / b;
+  }
+}
+
+// A distance's root and the unit vector (rx, ry) / dist, with kFast by root
+// and quotients (the same floats).
+template <bool kFast>
+__device__ __forceinline__ float length_of(float d2, float& y) {
+  if constexpr (kFast) return root(d2, y);
+  else return sqrtf(d2);
+}
+template <bool kFast>
+__device__ __forceinline__ void unit(float rx, float ry, float dist, float y, float& nx, float& ny) {
+  if constexpr (kFast) {
+    quotients(rx, ry, dist, y, nx, ny);
+  } else {
+    nx = rx / dist;
+    ny = ry / dist;
+  }
+}
+
 // collideSpheres' contact law (src/particles_kernel.cuh:255-303) for a
-// partner B of material tB at offset (rx, ry) and distance dist < R: the
-// force on A as collideSpheres returns it (ffx, ffy), the length of its
+// partner B of material tB at the direction (nx, ny) and distance dist < R:
+// the force on A as collideSpheres returns it (ffx, ffy), the length of its
 // normal part (the pressure term's numerator) as the return value, and the
 // friction moment term mterm (+0 without friction; the moment is a sum that
 // starts at +0 and is never -0, so adding +0 leaves it unchanged).
-__device__ __forceinline__ float contact_terms(const StepConst& c, const PairCtx& q, float rx, float ry, float dist,
+template <bool kFast>
+__device__ __forceinline__ float contact_terms(const StepConst& c, const PairCtx& q, float nx, float ny, float dist,
                                                float R, float rB, uint32_t tB, float2 vB, float wB, float& ffx,
                                                float& ffy, float& mterm) {
   const float4 pr = c.pair[q.tA * c.num_types + tB];
   const float kn = pr.x, kt = pr.y, cn = pr.z, mu = pr.w;
-  const float nx = rx / dist, ny = ry / dist;
   const float tx = -ny, ty = nx;
   const float rvx = vB.x - q.v.x, rvy = vB.y - q.v.y;
   const float vn = rvx * nx + rvy * ny;
@@ -290,7 +329,8 @@ __device__ __forceinline__ float contact_terms(const StepConst& c, const PairCtx
     ffx += s2 * nx;
     ffy += s2 * ny;
   }
-  const float flen = sqrtf(ffx * ffx + ffy * ffy);
+  float y;
+  const float flen = length_of<kFast>(ffx * ffx + ffy * ffy, y);
   mterm = 0.0f;
   if (mu != 0.0f) {
     const float sr = q.rA * q.w + rB * wB;
@@ -298,9 +338,8 @@ __device__ __forceinline__ float contact_terms(const StepConst& c, const PairCtx
     float ftx = (kt * cvx) * q.dt, fty = (kt * cvy) * q.dt;
     const float ftmax = mu * flen;
     if (!sqrt_below(ftx * ftx + fty * fty, ftmax)) {
-      const float cl = sqrtf(cvx * cvx + cvy * cvy);
-      ftx = (ftmax * cvx) / cl;
-      fty = (ftmax * cvy) / cl;
+      const float cl = length_of<kFast>(cvx * cvx + cvy * cvy, y);
+      unit<kFast>(ftmax * cvx, ftmax * cvy, cl, y, ftx, fty);
     }
     ffx += ftx;
     ffy += fty;
@@ -311,24 +350,24 @@ __device__ __forceinline__ float contact_terms(const StepConst& c, const PairCtx
 
 // The contact law with its pressure term added to pres and its moment term
 // to moment.
-template <bool kRcp = false>
-__device__ __forceinline__ void contact_force(const StepConst& c, const PairCtx& q, float rx, float ry, float dist,
+template <bool kFast = false>
+__device__ __forceinline__ void contact_force(const StepConst& c, const PairCtx& q, float nx, float ny, float dist,
                                               float R, float rB, uint32_t tB, float2 vB, float wB, float& ffx,
                                               float& ffy, float& moment, float& pres) {
   float mterm;
-  const float flen = contact_terms(c, q, rx, ry, dist, R, rB, tB, vB, wB, ffx, ffy, mterm);
-  pres = kRcp ? add_pressure_recip(pres, flen, q.den, q.rden) : add_pressure(pres, flen, q.den);
+  const float flen = contact_terms<kFast>(c, q, nx, ny, dist, R, rB, tB, vB, wB, ffx, ffy, mterm);
+  pres = kFast ? add_pressure_recip(pres, flen, q.den, q.rden) : add_pressure(pres, flen, q.den);
   moment += mterm;
 }
 
 // attractSpheres (src/particles_kernel.cuh:310-342) for a partner with
 // attraction coefficient aB: the force on A and its pressure term.
-__device__ __forceinline__ void attract_force(const PairCtx& q, float rx, float ry, float dist, float rB, float aB,
+template <bool kFast = false>
+__device__ __forceinline__ void attract_force(const PairCtx& q, float nx, float ny, float dist, float rB, float aB,
                                               float& afx, float& afy, float& pres) {
   const float aA = q.attract;
   const float adA = (float)((double)(q.rA * 2.0f) * 1.2);
   const float adB = (float)((double)(rB * 2.0f) * 1.2);
-  const float nx = rx / dist, ny = ry / dist;
   afx = 0.0f;
   afy = 0.0f;
   if (dist < adA) {
@@ -341,7 +380,9 @@ __device__ __forceinline__ void attract_force(const PairCtx& q, float rx, float 
     afx += s * nx;
     afy += s * ny;
   }
-  pres = add_pressure(pres, sqrtf(afx * afx + afy * afy), q.den);
+  float y;
+  const float len = length_of<kFast>(afx * afx + afy * afy, y);
+  pres = kFast ? add_pressure_recip(pres, len, q.den, q.rden) : add_pressure(pres, len, q.den);
 }
 
 // Velocity and spin of the sorted particles: vel[j], omega[j], or with a
@@ -402,7 +443,7 @@ struct RowSum {
   }
 };
 
-template <bool kRadius, bool kOne, bool kDyn, bool kO, bool kRcp = false>
+template <bool kRadius, bool kOne, bool kDyn, bool kO>
 __device__ __forceinline__ void candidate_at(const StepConst& c, const PairCtx& q, uint32_t j, bool self,
                                              const Cand& b, const Dyn& d, const uint32_t* __restrict__ type,
                                              RowSum& rsum, float& fx, float& fy, float& moment, float& pres) {
@@ -431,13 +472,37 @@ __device__ __forceinline__ void candidate_at(const StepConst& c, const PairCtx& 
       vB = ld<kO>(d.vel, jv);
       wB = ld<kO>(d.omega, jv);
     }
-    contact_force<kRcp>(c, q, rx, ry, dist, R, rB, tB, vB, wB, ffx, ffy, moment, pres);
+    contact_force(c, q, rx / dist, ry / dist, dist, R, rB, tB, vB, wB, ffx, ffy, moment, pres);
     cfx += ffx;
     cfy += ffy;
   }
   if (c.attract) {
     float afx, afy;
-    attract_force(q, rx, ry, dist, rB, c.mat[tB].attract, afx, afy, pres);
+    attract_force(q, rx / dist, ry / dist, dist, rB, c.mat[tB].attract, afx, afy, pres);
+    cfx += afx;
+    cfy += afy;
+  }
+}
+
+// A candidate that the contact-list walk marked (its velocity, spin and
+// material row loaded): the same sums, without the test that the mark was.
+__device__ __forceinline__ void listed_pair(const StepConst& c, const PairCtx& q, const Cand& b, float& cfx,
+                                            float& cfy, float& moment, float& pres) {
+  const float rx = b.p.x - q.p.x, ry = b.p.y - q.p.y;
+  const float R = q.rA + b.r;
+  float y, nx, ny;
+  const float dist = root(rx * rx + ry * ry, y);
+  if (!(dist < R || c.attract)) return;
+  quotients(rx, ry, dist, y, nx, ny);
+  if (dist < R) {
+    float ffx, ffy;
+    contact_force<true>(c, q, nx, ny, dist, R, b.r, b.t, b.v, b.w, ffx, ffy, moment, pres);
+    cfx += ffx;
+    cfy += ffy;
+  }
+  if (c.attract) {
+    float afx, afy;
+    attract_force<true>(q, nx, ny, dist, b.r, c.mat[b.t].attract, afx, afy, pres);
     cfx += afx;
     cfy += afy;
   }
@@ -458,12 +523,13 @@ __device__ __forceinline__ void control_pair(const StepConst& c, const PairCtx& 
   float m = 0.0f, f_x = 0.0f, f_y = 0.0f;
   if (dist < R) {
     float mterm = 0.0f;
-    contact_force(c, q, rx, ry, dist, R, rC, tC, make_float2(C.vel[0], C.vel[1]), C.omega, f_x, f_y, mterm, pres);
+    contact_force(c, q, rx / dist, ry / dist, dist, R, rC, tC, make_float2(C.vel[0], C.vel[1]), C.omega, f_x, f_y,
+                  mterm, pres);
     m = m + mterm;  // collideSpheres adds into the caller's m (0)
   }
   if (c.attract) {
     float afx, afy;
-    attract_force(q, rx, ry, dist, rC, c.mat[tC].attract, afx, afy, pres);
+    attract_force(q, rx / dist, ry / dist, dist, rC, c.mat[tC].attract, afx, afy, pres);
     f_x += afx;
     f_y += afy;
   }
@@ -497,14 +563,14 @@ __device__ __forceinline__ void candidate_load(const StepConst& c, uint32_t j, c
   }
 }
 
-template <bool kRadius, bool kOne, bool kDyn, bool kO, bool kRcp = false>
+template <bool kRadius, bool kOne, bool kDyn, bool kO>
 __device__ __forceinline__ void candidate(const StepConst& c, const PairCtx& q, uint32_t j, bool self,
                                           const float2* __restrict__ pos, const Dyn& d,
                                           const uint32_t* __restrict__ type, const float* __restrict__ radius,
                                           RowSum& rsum, float& fx, float& fy, float& moment, float& pres) {
   Cand b;
   candidate_load<kRadius, kOne, kDyn, kO>(c, j, pos, type, radius, d, b);
-  candidate_at<kRadius, kOne, kDyn, kO, kRcp>(c, q, j, self, b, d, type, rsum, fx, fy, moment, pres);
+  candidate_at<kRadius, kOne, kDyn, kO>(c, q, j, self, b, d, type, rsum, fx, fy, moment, pres);
 }
 
 // Forces on sorted particle i from its 3x3 cell neighbourhood (the body of
@@ -564,22 +630,29 @@ __device__ __forceinline__ void shift_in(uint32_t (&w)[3], const float (&x)[3], 
 // once, coalesced; each lane then walks its candidates in LDS.  The vector
 // cache looks up one line a cycle, and walking the candidates through it
 // (585 lookups a wave at 4M settling discs, where it was busy 93% of the
-// kernel's time) bound the kernel.  With the windows and the shorter marks
-// it takes 49.9 us there (58.7), 150 us on the 4M dense pack (172), 136 us on
-// the 8.2M-disc ensemble (149).  Entries: three rows of kWindow, then
+// kernel's time) bound the kernel: with the windows it took 50 us there
+// (59), 150 us on the 4M dense pack (172), 136 us on the 8.2M-disc ensemble
+// (149).  Now vector instructions bound it (397 a wave there, 78% of the time
+// issuing): with one word of marks, the rows' ranges by minimum and maximum
+// and the short roots, quotients and cells, 53 us there (54, the same hour), 128
+// us on the dense pack (151), 143 us on the ensemble (152).  Three rows of kWindow entries, then
 // kWindowSlack more, as a lane with few candidates reads on past its row's.
-// Eight waves a SIMD fit (32 x 4,864 bytes of 160 KB).
-constexpr uint32_t kWindow = 128, kWindowSlack = 64;
-struct WaveWindow {
-  float2 pos[3 * kWindow];
-  float r[3 * kWindow + kWindowSlack];  // (reads of pos past its end land here)
+// An entry's three words lie together, so a lane's walk has one address a row
+// (and no bank conflict, a wave's lanes being 3 words apart).  Eight waves a
+// SIMD fit (32 x 5,120 bytes of 160 KB).
+constexpr uint32_t kWindow = 128, kWindowSlack = 32;
+struct WindowEntry {
+  float x, y, r;
 };
-static_assert(sizeof(WaveWindow) == 4864, "eight waves a SIMD");
+struct WaveWindow {
+  WindowEntry at[3 * kWindow + kWindowSlack];
+};
+static_assert(sizeof(WaveWindow) <= 5120, "eight waves a SIMD");
 
 // This wave's windows in the block's dynamic LDS (window_bytes(block)).
 extern __shared__ __attribute__((aligned(16))) unsigned char dem_windows[];
 __device__ __forceinline__ WaveWindow* wave_window() {
-  return reinterpret_cast<WaveWindow*>(dem_windows) + threadIdx.x / (uint32_t)kWave;
+  return reinterpret_cast<WaveWindow*>(dem_windows) + __builtin_amdgcn_readfirstlane(threadIdx.x / (uint32_t)kWave);
 }
 inline size_t window_bytes(int mode, int block) {
   return mode == kList ? sizeof(WaveWindow) * (size_t)((block + kWave - 1) / kWave) : 0;
@@ -604,9 +677,10 @@ __device__ __forceinline__ void collide_particle(const StepConst& c, uint32_t i,
   const Material mA = c.mat[own.t];
   q.attract = mA.attract;
   const Instance in = kMulti ? c.inst[clamp_idx(mA.inst, c.num_instances)] : c.inst0;
-  body<kRadius>(mA, radius, i, q.rA, own.mass, own.inertia);
+  const float r_i = kRadius ? ld<kO>(radius, i) : 0.0f;
+  body<kRadius>(mA, &r_i, 0u, q.rA, own.mass, own.inertia);
   own.r = q.rA;
-  q.p = pos[i];
+  q.p = ld<kO>(pos, i);
   // The particle's own velocity and spin feed only the contact law (and the
   // fused kernel's integrate): the contact-list walk loads them once it has
   // marked a candidate (or at the end, where a caller uses them), the other
@@ -614,18 +688,17 @@ __device__ __forceinline__ void collide_particle(const StepConst& c, uint32_t i,
   bool have_dyn = false;
   auto load_own_dyn = [&]() {
     const uint32_t iv = d.at<kO>(i);
-    q.v = d.vel[iv];
-    q.w = d.omega[iv];
+    q.v = ld<kO>(d.vel, iv);
+    q.w = ld<kO>(d.omega, iv);
+    q.den = pressure_den(q.rA);
     have_dyn = true;
   };
   if (kMode != kList || kControl || kEarly) load_own_dyn();
   own.p = q.p;
-  q.den = pressure_den(q.rA);
-  q.rden = 0.0;  // the contact-list walk sets it before its first contact
   q.dt = c.dt;
   const bool clamp = c.flags & DEM_GRID_CLAMP;
   const int G0 = (int)in.grid[0], G1 = (int)in.grid[1];
-
+  float fx = 0.0f, fy = 0.0f, moment = 0.0f, pres = 0.0f;
   int gx, gy;
   grid_pos(in, q.p, gx, gy);
   if (clamp) clamp_cell(in, gx, gy);
@@ -636,45 +709,41 @@ __device__ __forceinline__ void collide_particle(const StepConst& c, uint32_t i,
   const uint32_t x2 = ((uint32_t)gx + 1u) & (clamp ? 0xFFFFFFFFu : (uint32_t)G0 - 1u);
   own.cell = in.cell_base + (clamp ? (uint32_t)gy : (uint32_t)gy & ((uint32_t)G1 - 1u)) * (uint32_t)G0 + x1;
   // a wrap that moves a column to the other edge breaks key contiguity
-  const bool contiguous = clamp || (x0 + 1u == x1 && x1 + 1u == x2);
-
-  float fx = 0.0f, fy = 0.0f, moment = 0.0f, pres = 0.0f;
-  if (contiguous) {
+  bool by_cell = !(clamp || (x0 + 1u == x1 && x1 + 1u == x2));
+  if (!by_cell) {
     // The usual case: every row's three cells are consecutive keys, so a row
     // is one candidate range [rs, re) with the cell ends b0, b1 inside it.
     // The ranges of all three rows are loaded first (their loads overlap),
     // and each candidate's position and radius are fetched one iteration
     // ahead; the summation order is unchanged.
+    // The cells' starts are increasing, an empty cell's is the largest word
+    // and its end is taken as 0, so the range is the least start and the
+    // largest end.  b0 and b1, where the second and third cell begin, are the
+    // range's start for empty cells before them (a flush of an empty sum
+    // changes nothing).  A column or row outside a clamped grid stands in as
+    // the centre one: a cell read twice changes neither the range nor what
+    // lies in which of two cells, a row's range is emptied.
     uint32_t rs[3], re[3], b0[3], b1[3];
+    const uint32_t cyc = clamp ? (uint32_t)gy : (uint32_t)gy & ((uint32_t)G1 - 1u);
+    const bool top = cyc == 0u, bottom = cyc == (uint32_t)G1 - 1u;
+    const uint32_t around = clamp ? 0u : ((uint32_t)G1 - 1u) * (uint32_t)G0;
+    const uint32_t row1 = in.cell_base + cyc * (uint32_t)G0;
+    const uint32_t rows[3] = {top ? row1 + around : row1 - (uint32_t)G0, row1,
+                              bottom ? row1 - around : row1 + (uint32_t)G0};
+    const uint32_t xl = vx0 ? x0 : x1, xr = vx2 ? x2 : x1;
 #pragma unroll
     for (int y = 0; y < 3; ++y) {
-      const int iy = gy + y - 1;
-      uint32_t cy;
-      bool ok = true;
-      if (clamp) {
-        ok = iy >= 0 && iy < G1;
-        cy = ok ? (uint32_t)iy : 0u;
-      } else {
-        cy = (uint32_t)iy & ((uint32_t)G1 - 1u);
-      }
-      const uint32_t row = in.cell_base + cy * (uint32_t)G0;
-      // All six words are loaded unconditionally from cells inside the grid
-      // (a column or row outside it reads the centre column or row 0) and
-      // then masked: no branch per load.
-      const uint32_t a0 = row + (vx0 ? x0 : x1), a1 = row + x1, a2 = row + (vx2 ? x2 : x1);
-      const uint32_t s0r = ld<kO>(cell_start, a0), s1r = ld<kO>(cell_start, a1), s2r = ld<kO>(cell_start, a2);
-      const uint32_t e0r = ld<kO>(cell_end, a0), e1r = ld<kO>(cell_end, a1), e2r = ld<kO>(cell_end, a2);
-      const uint32_t s0 = ok && vx0 ? s0r : kEmpty;
-      const uint32_t s1 = ok ? s1r : kEmpty;
-      const uint32_t s2 = ok && vx2 ? s2r : kEmpty;
-      const bool n0 = s0 != kEmpty, n1 = s1 != kEmpty, n2 = s2 != kEmpty;
-      const uint32_t e0 = n0 ? min(e0r, n) : 0u;
-      const uint32_t e1 = n1 ? min(e1r, n) : 0u;
-      const uint32_t e2 = n2 ? min(e2r, n) : 0u;
-      rs[y] = n0 ? s0 : (n1 ? s1 : (n2 ? s2 : 0u));
-      re[y] = n2 ? e2 : (n1 ? e1 : e0);
-      b0[y] = n0 ? e0 : kNoBoundary;
-      b1[y] = n1 ? e1 : kNoBoundary;
+      const uint32_t s0 = ld<kO>(cell_start, rows[y] + xl), s1 = ld<kO>(cell_start, rows[y] + x1),
+                     s2 = ld<kO>(cell_start, rows[y] + xr);
+      const uint32_t e0r = ld<kO>(cell_end, rows[y] + xl), e1r = ld<kO>(cell_end, rows[y] + x1),
+                     e2r = ld<kO>(cell_end, rows[y] + xr);
+      const uint32_t e0 = s0 != kEmpty ? e0r : 0u, e1 = s1 != kEmpty ? e1r : 0u, e2 = s2 != kEmpty ? e2r : 0u;
+      re[y] = min(max(max(e0, e1), e2), n);
+      if (y == 0) re[y] = clamp && top ? 0u : re[y];
+      if (y == 2) re[y] = clamp && bottom ? 0u : re[y];
+      rs[y] = min(min(min(s0, s1), s2), re[y]);
+      b0[y] = max(e0, rs[y]);
+      b1[y] = max(e1, b0[y]);
     }
     Cand cb[3][kBatchN];
     if (kMode == kBatch) {
@@ -687,17 +756,16 @@ __device__ __forceinline__ void collide_particle(const StepConst& c, uint32_t i,
           candidate_load<kRadius, kOne, false, kO>(c, j < re[y] ? j : 0u, pos, type, radius, d, cb[y][k]);
         }
     }
-    if (kMode == kList && (!c.attract || q.den > 0.0) && re[0] - rs[0] <= 64u && re[1] - rs[1] <= 64u &&
-        re[2] - rs[2] <= 64u) {
-      // Rows of at most 64 candidates: first one bit per candidate that may
-      // exert a force (from position and radius), then the law over the set
-      // bits of all three rows in row order, so a wave runs the law as often
-      // as its busiest lane has contacts.  Candidates that exert no force add
-      // +0, so skipping them leaves every sum unchanged; a row's partial sum
-      // is flushed when the walk moves on to a later row.  (An attracting
-      // candidate out of reach adds +0 / den to the pressure: +0 for den > 0;
-      // the 16,290-disc pile's fused step takes 15.7 us this way, 42 one
-      // candidate at a time.)
+    const uint32_t len[3] = {re[0] - rs[0], re[1] - rs[1], re[2] - rs[2]};
+    if (kMode == kList && (!c.attract || fabsf(q.rA) > 0.0f) && max(len[0], max(len[1], len[2])) <= 0xFFFFu) {
+      // First one bit per candidate that may exert a force (from position and
+      // radius), then the law over the set bits in the rows' order, so a wave
+      // runs the law as often as its busiest lane has contacts.  Candidates
+      // that exert no force add +0, so skipping them leaves every sum
+      // unchanged; a cell's partial sum is flushed when the walk moves on to a
+      // later cell.  (An attracting candidate out of reach adds +0 / den to
+      // the pressure: +0 for a radius; the 16,290-disc pile's fused step takes
+      // 15.7 us this way, 42 one candidate at a time.)
       // The three rows are walked together, from the wave's windows in LDS
       // (WaveWindow) or from global memory.  The walk is most of the kernel's
       // instructions on sparse states, so each candidate costs as few as
@@ -709,23 +777,14 @@ __device__ __forceinline__ void collide_particle(const StepConst& c, uint32_t i,
       // here is R (1 + 2^-18) within 2^-23, so d2 - R^2 rounds to a negative
       // number, or to at most 2^-125 where the squares underflow; NaN is
       // marked.
-      // A row's places: its length, and where its second and third cells
-      // start, 8 bits each (an empty cell starts where the next one does, a
-      // flush of an empty sum changes nothing).
-      uint32_t first[3], cut[3];
+      // where a row's second and third cells begin, 16 bits each
+      uint32_t cut[3];
 #pragma unroll
-      for (int y = 0; y < 3; ++y) {
-        const uint32_t c0 = b0[y] == kNoBoundary ? 0u : min(b0[y] - rs[y], 64u);
-        const uint32_t c1 = b1[y] == kNoBoundary ? c0 : min(b1[y] - rs[y], 64u);
-        first[y] = rs[y];
-        cut[y] = (re[y] - rs[y]) | c0 << 8 | c1 << 16;
-      }
-      auto length = [&](int y) { return cut[y] & 0xFFu; };
-      const uint32_t L = max(length(0), max(length(1), length(2)));
+      for (int y = 0; y < 3; ++y) cut[y] = (b0[y] - rs[y]) | (b1[y] - rs[y]) << 16;
       // At most 2^-125 where a candidate at p with radius r may exert a force.
       const float reach = q.rA * kReach;
-      auto beyond = [&](auto attract, float2 p, float r) {
-        const float rx = p.x - q.p.x, ry = p.y - q.p.y;
+      auto beyond = [&](auto attract, float x, float y, float r) {
+        const float rx = x - q.p.x, ry = y - q.p.y;
         const float d2 = __builtin_fmaf(ry, ry, rx * rx);
         float R = __builtin_fmaf(r, kReach, reach);
         // (attractSpheres reaches 2.4 times either radius)
@@ -735,21 +794,26 @@ __device__ __forceinline__ void collide_particle(const StepConst& c, uint32_t i,
       // The windows, where the whole wave is here and every lane's ranges
       // lie in them (rows far apart, as around wide empty spaces, do not fit
       // and are walked in global memory).
-      uint32_t w0[3] = {0u, 0u, 0u}, w1[3] = {0u, 0u, 0u};
-      bool in_win = win && __ballot(true) == ~0ull;
+      uint32_t w0[3], w1[3];
+      uint64_t outside = ~__ballot(win != nullptr);
 #pragma unroll
       for (int y = 0; y < 3; ++y) {
-        const uint64_t some = __ballot(length(y) != 0u);
-        if (some) {
-          const uint32_t end = first[y] + length(y);
-          w0[y] = (uint32_t)__builtin_amdgcn_readlane((int)first[y], __builtin_ctzll(some));
-          w1[y] = (uint32_t)__builtin_amdgcn_readlane((int)end, 63 - __builtin_clzll(some));
-          in_win = in_win && w1[y] - w0[y] <= kWindow &&
-                   __ballot(length(y) && (first[y] < w0[y] || end > w1[y])) == 0;
-        }
+        // (rows that are empty in the whole wave: any lane's range is empty)
+        const uint64_t some = __ballot(len[y] != 0u);
+        w0[y] = (uint32_t)__builtin_amdgcn_readlane((int)rs[y], __builtin_ctzll(some | 1ull << 63));
+        w1[y] = (uint32_t)__builtin_amdgcn_readlane((int)re[y], 63 - __builtin_clzll(some | 1ull));
+        w1[y] = some ? w1[y] : w0[y];
+        outside |= (__ballot(rs[y] < w0[y]) | __ballot(re[y] > w1[y])) & some;
+        outside |= w1[y] - w0[y] > kWindow ? ~0ull : 0ull;
       }
+      const bool in_win = outside == 0;
       if (in_win) {
         const uint32_t lane = __lane_id();
+        auto put = [&](uint32_t e, const Cand& b) {
+          win->at[e].x = b.p.x;
+          win->at[e].y = b.p.y;
+          win->at[e].r = b.r;
+        };
         auto stage = [&](uint32_t e) {
           Cand b[3];
 #pragma unroll
@@ -757,122 +821,80 @@ __device__ __forceinline__ void collide_particle(const StepConst& c, uint32_t i,
             if (w0[y] + e < w1[y]) candidate_load<kRadius, kOne, false, kO>(c, w0[y] + e, pos, type, radius, d, b[y]);
 #pragma unroll
           for (int y = 0; y < 3; ++y)
-            if (w0[y] + e < w1[y]) {
-              win->pos[(uint32_t)y * kWindow + e] = b[y].p;
-              win->r[(uint32_t)y * kWindow + e] = b[y].r;
-            }
+            if (w0[y] + e < w1[y]) put((uint32_t)y * kWindow + e, b[y]);
         };
         stage(lane);
         // what is left of the three windows: usually a few places each, taken
-        // by a third of the wave a row
-        constexpr uint32_t kThird = (uint32_t)kWave / 3u;
-        const uint32_t longest = max(w1[0] - w0[0], max(w1[1] - w0[1], w1[2] - w0[2]));
-        if (longest > (uint32_t)kWave + kThird) {
+        // by a quarter of the wave a row
+        constexpr uint32_t kQuarter = (uint32_t)kWave / 4u;
+        auto longer = [&](uint32_t k) { return (w1[0] - w0[0] > k) | (w1[1] - w0[1] > k) | (w1[2] - w0[2] > k); };
+        if (longer((uint32_t)kWave + kQuarter)) {
           stage((uint32_t)kWave + lane);
-        } else if (longest > (uint32_t)kWave) {
-          const uint32_t y = lane / kThird, e = (uint32_t)kWave + lane % kThird;
+        } else if (longer((uint32_t)kWave)) {
+          const uint32_t y = lane / kQuarter, e = (uint32_t)kWave + lane % kQuarter;
           const uint32_t a = y == 0u ? w0[0] : (y == 1u ? w0[1] : w0[2]), z = y == 0u ? w1[0] : (y == 1u ? w1[1] : w1[2]);
           if (y < 3u && a + e < z) {
             Cand b;
             candidate_load<kRadius, kOne, false, kO>(c, a + e, pos, type, radius, d, b);
-            win->pos[y * kWindow + e] = b.p;
-            win->r[y * kWindow + e] = b.r;
+            put(y * kWindow + e, b);
           }
         }
         // (one wave's LDS instructions execute in order; this keeps the
         // compiler's order)
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-#pragma unroll
-        for (int y = 0; y < 3; ++y) first[y] = length(y) ? first[y] : w0[y];  // an entry of the window for each lane
       }
       // the window entry of candidate j of row y
       auto entry = [&](int y, uint32_t j) { return j - w0[y] + (uint32_t)y * kWindow; };
-      // the rows' candidates [k0, k1), marked into w
-      auto mark = [&](auto attract, uint32_t k0, uint32_t k1, uint32_t (&w)[3]) {
-        uint32_t walked = 0;
+      // The candidates of the rows' parts (m of them from f, at most 31 a
+      // lane together) marked into w, left-aligned: the first one at bit 31.
+      // Lanes with shorter parts walk on (WaveWindow's slack) as long as any
+      // has candidates: the loop is the wave's.
+      auto mark = [&](auto attract, const uint32_t (&f)[3], const uint32_t (&m)[3], uint32_t (&w)[3]) {
+        const uint32_t L = max(m[0], max(m[1], m[2]));
+        uint32_t k = 0;
         if (in_win) {
+          const WindowEntry* e[3];
+#pragma unroll
+          for (int y = 0; y < 3; ++y) e[y] = win->at + (m[y] ? entry(y, f[y]) : (uint32_t)y * kWindow);
           // two candidates a row at a time
-          for (uint32_t k = k0; k < k1; k += 2u, walked += 2u) {
-            Cand b[3][2];
+          for (; __ballot(k < L); k += 2u) {
+            WindowEntry b[3][2];
 #pragma unroll
-            for (int y = 0; y < 3; ++y)
-#pragma unroll
-              for (uint32_t u = 0; u < 2u; ++u) {
-                b[y][u].p = win->pos[entry(y, first[y]) + k + u];
-                b[y][u].r = win->r[entry(y, first[y]) + k + u];
-              }
+            for (int y = 0; y < 3; ++y) {
+              b[y][0] = e[y][0];
+              b[y][1] = e[y][1];
+              e[y] += 2;
+            }
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
-              const float x[3] = {beyond(attract, b[0][u].p, b[0][u].r), beyond(attract, b[1][u].p, b[1][u].r),
-                                  beyond(attract, b[2][u].p, b[2][u].r)};
+              const float x[3] = {beyond(attract, b[0][u].x, b[0][u].y, b[0][u].r),
+                                  beyond(attract, b[1][u].x, b[1][u].y, b[1][u].r),
+                                  beyond(attract, b[2][u].x, b[2][u].y, b[2][u].r)};
               shift_in(w, x, 0x1p-125f);
             }
           }
         } else {
-          // a row already walked re-reads its last candidate
-          for (uint32_t k = k0; k < k1; ++k, ++walked) {
+          // a part already walked re-reads its last candidate
+          for (; __ballot(k < L); ++k) {
             Cand b[3];
 #pragma unroll
             for (int y = 0; y < 3; ++y)
-              candidate_load<kRadius, kOne, false, kO>(c, first[y] + min(k, max(length(y), 1u) - 1u), pos, type,
-                                                       radius, d, b[y]);
-            const float x[3] = {beyond(attract, b[0].p, b[0].r), beyond(attract, b[1].p, b[1].r),
-                                beyond(attract, b[2].p, b[2].r)};
+              candidate_load<kRadius, kOne, false, kO>(c, m[y] ? f[y] + min(k, m[y] - 1u) : 0u, pos, type, radius, d,
+                                                       b[y]);
+            const float x[3] = {beyond(attract, b[0].p.x, b[0].p.y, b[0].r), beyond(attract, b[1].p.x, b[1].p.y, b[1].r),
+                                beyond(attract, b[2].p.x, b[2].p.y, b[2].r)};
             shift_in(w, x, 0x1p-125f);
           }
         }
-        // left-aligned: the first candidate at bit 31 (none walked: 0)
 #pragma unroll
-        for (int y = 0; y < 3; ++y) w[y] = walked ? w[y] << (32u - walked) : 0u;
+        for (int y = 0; y < 3; ++y) w[y] = k ? w[y] << (32u - k) : 0u;
       };
-      uint32_t hlo[3] = {0u, 0u, 0u}, hhi[3] = {0u, 0u, 0u};
-      auto mark_all = [&](auto attract) {
-        mark(attract, 0u, min(L, 32u), hlo);
-        if (L > 32u) mark(attract, 32u, L, hhi);
-      };
-      if (c.attract) mark_all(std::true_type{});
-      else mark_all(std::false_type{});
-      uint64_t h[3];
-#pragma unroll
-      for (int y = 0; y < 3; ++y) {
-        h[y] = ((uint64_t)hlo[y] << 32) | hhi[y];
-        if (length(y) < 64u) h[y] &= ~(~0ull >> length(y));           // past the row's end
-        const uint32_t own_k = i - first[y];
-        if (own_k < length(y)) h[y] &= ~(1ull << (63u - own_k));  // the particle itself
-      }
-      RowSum rsum;
-      rsum.b0 = rsum.b1 = kNoBoundary;
-      int row = -1;
-      // the particle's velocity, spin and the pressure terms' reciprocal,
-      // only where a candidate may touch
-      if (h[0] | h[1] | h[2]) {
-        if (!have_dyn) load_own_dyn();
-        q.rden = 1.0 / q.den;
-      }
-      while (h[0] | h[1] | h[2]) {
-        const bool in0 = h[0] != 0, in1 = !in0 && h[1] != 0;
-        const int y = in0 ? 0 : (in1 ? 1 : 2);
-        const uint64_t hy = in0 ? h[0] : (in1 ? h[1] : h[2]);
-        const uint32_t k = (uint32_t)__builtin_clzll(hy), f = in0 ? first[0] : (in1 ? first[1] : first[2]);
-        const uint32_t j = f + k;
-        const uint64_t rest = hy & (~0ull >> 1 >> k);
-        h[0] = in0 ? rest : h[0];
-        h[1] = in1 ? rest : h[1];
-        h[2] = (!in0 && !in1) ? rest : h[2];
-        if (y != row) {
-          fx += rsum.cfx;
-          fy += rsum.cfy;
-          const uint32_t ct = in0 ? cut[0] : (in1 ? cut[1] : cut[2]);
-          rsum = RowSum{};
-          rsum.b0 = f + (ct >> 8 & 0xFFu);
-          rsum.b1 = f + (ct >> 16);
-          row = y;
-        }
+      // candidate j (entry e of the windows), as the law reads it
+      auto listed = [&](uint32_t j, uint32_t e) {
         Cand b;
         if (in_win) {
-          const uint32_t e = in0 ? entry(0, j) : (in1 ? entry(1, j) : entry(2, j));
-          b.p = win->pos[e];
-          b.r = win->r[e];
+          b.p = make_float2(win->at[e].x, win->at[e].y);
+          b.r = win->at[e].r;
           b.t = kOne ? 0u : clamp_idx(ld<kO>(type, j), c.num_types);
           const uint32_t jv = d.at<kO>(j);
           b.v = ld<kO>(d.vel, jv);
@@ -880,57 +902,173 @@ __device__ __forceinline__ void collide_particle(const StepConst& c, uint32_t i,
         } else {
           candidate_load<kRadius, kOne, true, kO>(c, j, pos, type, radius, d, b);
         }
-        candidate_at<kRadius, kOne, true, kO, true>(c, q, j, false, b, d, type, rsum, fx, fy, moment, pres);
-      }
-      fx += rsum.cfx;
-      fy += rsum.cfy;
-    } else {
-    if (!have_dyn) load_own_dyn();
+        return b;
+      };
+      // The three rows' marks follow each other in one word, and a second word
+      // has a bit where a cell begins, so a step of the contact loop is a
+      // count of zeros and a count of cells (14 instructions with 32 bits, 21
+      // with 64; rows with words of their own took 30, and registers that cost
+      // a wave a SIMD).
+      float cfx = 0.0f, cfy = 0.0f;  // the cell's partial sum
+      auto flush = [&]() {
+        fx += cfx;
+        fy += cfy;
+        cfx = 0.0f;
+        cfy = 0.0f;
+      };
+      auto marks = [&](auto word, const uint32_t (&f)[3], const uint32_t (&m)[3]) {
+        using W = decltype(word);
+        constexpr uint32_t kUp = 8u * sizeof(W) - 32u;
+        uint32_t w[3] = {0u, 0u, 0u};
+        if (c.attract) mark(std::true_type{}, f, m, w);
+        else mark(std::false_type{}, f, m, w);
 #pragma unroll
-    for (int y = 0; y < 3; ++y) {
-      RowSum rsum;
-      rsum.b0 = b0[y];
-      rsum.b1 = b1[y];
-      const uint32_t end = re[y];
-      if (kMode == kPrefetch) {
-        // each candidate's position and radius fetched one iteration ahead
-        // (pays off with many candidates per row, costs registers)
-        uint32_t j = rs[y];
-        Cand nx{};
-        if (j < end) candidate_load<kRadius, kOne, false, kO>(c, j, pos, type, radius, d, nx);
-        for (; j < end; ++j) {
-          const Cand b = nx;
-          if (j + 1u < end) candidate_load<kRadius, kOne, false, kO>(c, j + 1u, pos, type, radius, d, nx);
-          candidate_at<kRadius, kOne, false, kO>(c, q, j, j == i, b, d, type, rsum, fx, fy, moment, pres);
+        for (int y = 0; y < 3; ++y) {
+          w[y] &= ~(~0u >> m[y]);                         // past the part's end
+          w[y] &= ~(0x80000000u >> min(i - f[y], 31u));  // the particle itself (there is no 32nd candidate)
         }
+        return (W)w[0] << kUp | (W)w[1] << kUp >> m[0] | (W)w[2] << kUp >> (m[0] + m[1]);
+      };
+      // The law over the marked candidates; returns how many cells had begun
+      // at the last one.
+      auto contacts = [&](auto h, decltype(h) cells, const uint32_t (&f)[3], const uint32_t (&m)[3]) {
+        using W = decltype(h);
+        const uint32_t l1 = m[0], l2 = m[0] + m[1], f1 = f[1] - l1, f2 = f[2] - l2;
+        uint32_t cell = 0u;
+        while (h) {
+          uint32_t k, in_cell;
+          if constexpr (sizeof(W) == 8) k = (uint32_t)__builtin_clzll(h);
+          else k = (uint32_t)__builtin_clz(h);
+          const W after = (W)(~(W)0 >> 1) >> k;
+          h &= after;
+          if constexpr (sizeof(W) == 8) in_cell = (uint32_t)__popcll(cells & ~after);
+          else in_cell = (uint32_t)__popc(cells & ~after);
+          const bool in0 = k < l1, in1 = k < l2;
+          const uint32_t j = k + (in0 ? f[0] : (in1 ? f1 : f2));
+          const uint32_t e = j - (in0 ? w0[0] : (in1 ? w0[1] - kWindow : w0[2] - 2u * kWindow));
+          if (in_cell != cell) {
+            flush();
+            cell = in_cell;
+          }
+          listed_pair(c, q, listed(j, e), cfx, cfy, moment, pres);
+        }
+        return cell;
+      };
+      // every row in one pass
+      auto whole = [&](auto word) {
+        using W = decltype(word);
+        const W h = marks(word, rs, len);
+        if (h) {
+          // the particle's velocity, spin and the pressure terms' reciprocal,
+          // only where a candidate may touch
+          if (!have_dyn) load_own_dyn();
+          q.rden = 1.0 / q.den;
+          // (a row outside the grid is empty, and its boundaries lie anywhere)
+          W cells = 0;
+          uint32_t at = 0;
+#pragma unroll
+          for (int y = 0; y < 3; ++y) {
+            const W b = ((W)1 << (8u * sizeof(W) - 1u)) >> at;
+            cells |= len[y] ? b | b >> (cut[y] & 0xFFFFu) | b >> (cut[y] >> 16) : (W)0;
+            at += len[y];
+          }
+          (void)contacts(h, cells, rs, len);
+          flush();
+        }
+      };
+      const uint32_t total = len[0] + len[1] + len[2], L = max(len[0], max(len[1], len[2]));
+      if (__builtin_expect_with_probability(__ballot(total > 31u) == 0, 1, 0.9)) {
+        whole(0u);
+      } else if (__builtin_expect_with_probability(__ballot(total > 63u || L > 31u) == 0, 1, 0.9999)) {
+        whole((uint64_t)0);
       } else {
-        uint32_t j = rs[y];
-        if (kMode == kBatch) {
+        // passes over 31 of each lane's candidates at a time
+        constexpr uint32_t kPass = 31u;
+        if (!have_dyn) load_own_dyn();
+        q.rden = 1.0 / q.den;
+        for (uint32_t done = 0; __ballot(done < total); done += kPass) {
+          uint32_t f[3], m[3], cells = 0, at = 0, before = 0;
 #pragma unroll
-          for (int k = 0; k < kBatchN; ++k, ++j)
-            if (j < end)
-              candidate_at<kRadius, kOne, false, kO>(c, q, j, j == i, cb[y][k], d, type, rsum, fx, fy, moment, pres);
+          for (int y = 0; y < 3; ++y) {
+            const uint32_t lo = min(max(done, before) - before, len[y]);
+            f[y] = rs[y] + lo;
+            m[y] = min(max(done + kPass, before) - before, len[y]) - lo;
+            before += len[y];
+            // the cells that begin in this part
+            for (uint32_t b : {0u, cut[y] & 0xFFFFu, cut[y] >> 16})
+              cells |= b >= lo && b - lo < m[y] ? 0x80000000u >> (at + (b - lo)) : 0u;
+            at += m[y];
+          }
+          // (the next pass may go on with the last contact's cell)
+          if (contacts(marks(0u, f, m), cells, f, m) != (uint32_t)__popc(cells)) flush();
         }
-        for (; j < end; ++j)
-          candidate<kRadius, kOne, kMode == kPlain, kO>(c, q, j, j == i, pos, d, type, radius, rsum, fx, fy, moment,
-                                                     pres);
+        flush();
       }
-      fx += rsum.cfx;
-      fy += rsum.cfy;
+    } else if (kMode == kList) {
+      by_cell = true;
+    } else {
+#pragma unroll
+      for (int y = 0; y < 3; ++y) {
+        RowSum rsum;
+        rsum.b0 = b0[y];
+        rsum.b1 = b1[y];
+        const uint32_t end = re[y];
+        if (kMode == kPrefetch) {
+          // each candidate's position and radius fetched one iteration ahead
+          // (pays off with many candidates per row, costs registers)
+          uint32_t j = rs[y];
+          Cand nx{};
+          if (j < end) candidate_load<kRadius, kOne, false, kO>(c, j, pos, type, radius, d, nx);
+          for (; j < end; ++j) {
+            const Cand b = nx;
+            if (j + 1u < end) candidate_load<kRadius, kOne, false, kO>(c, j + 1u, pos, type, radius, d, nx);
+            candidate_at<kRadius, kOne, false, kO>(c, q, j, j == i, b, d, type, rsum, fx, fy, moment, pres);
+          }
+        } else {
+          uint32_t j = rs[y];
+          if (kMode == kBatch) {
+#pragma unroll
+            for (int k = 0; k < kBatchN; ++k, ++j)
+              if (j < end)
+                candidate_at<kRadius, kOne, false, kO>(c, q, j, j == i, cb[y][k], d, type, rsum, fx, fy, moment, pres);
+          }
+          for (; j < end; ++j)
+            candidate<kRadius, kOne, kMode == kPlain, kO>(c, q, j, j == i, pos, d, type, radius, rsum, fx, fy, moment,
+                                                       pres);
+        }
+        fx += rsum.cfx;
+        fy += rsum.cfy;
+      }
     }
-    }
-  } else {
-    // wrap mode at the grid's x edge: the three cells one by one, in the
-    // reference order
+  }
+  if (by_cell) {
+    // A wrapping grid's x edge, and rows too long for the contact list: the
+    // cells one by one, in the reference order (the list kernels' rare path:
+    // in loops, and from a cell computed again, as unrolled or with the cell
+    // kept over the list walk it decided how many registers they take).
     if (!have_dyn) load_own_dyn();
+    float2 pc = q.p;
+    asm("" : "+v"(pc.x), "+v"(pc.y));
+    uint32_t tc = own.t;
+    if constexpr (kMulti && !kUni) asm("" : "+v"(tc));
+    const Instance in = kMulti ? c.inst[clamp_idx(c.mat[tc].inst, c.num_instances)] : c.inst0;
+    const int G0 = (int)in.grid[0], G1 = (int)in.grid[1];
+    int gx, gy;
+    grid_pos(in, pc, gx, gy);
+    if (clamp) clamp_cell(in, gx, gy);
+#pragma unroll 1
     for (int y = -1; y <= 1; ++y) {
-      const uint32_t cy = ((uint32_t)gy + (uint32_t)y) & ((uint32_t)G1 - 1u);
-      const uint32_t row = in.cell_base + cy * (uint32_t)G0;
-      const uint32_t xs[3] = {x0, x1, x2};
+      const int iy = gy + y;
+      if (clamp && (iy < 0 || iy >= G1)) continue;
+      const uint32_t row = in.cell_base + (clamp ? (uint32_t)iy : (uint32_t)iy & ((uint32_t)G1 - 1u)) * (uint32_t)G0;
+#pragma unroll 1
       for (int sg = 0; sg < 3; ++sg) {
-        const uint32_t st = cell_start[row + xs[sg]];
+        const int ix = gx + sg - 1;
+        if (clamp && (ix < 0 || ix >= G0)) continue;
+        const uint32_t cell = row + (clamp ? (uint32_t)ix : (uint32_t)ix & ((uint32_t)G0 - 1u));
+        const uint32_t st = cell_start[cell];
         if (st == kEmpty) continue;
-        const uint32_t en = min(cell_end[row + xs[sg]], n);
+        const uint32_t en = min(cell_end[cell], n);
         RowSum rsum;  // one cell: no boundary inside
         rsum.b0 = kNoBoundary;
         rsum.b1 = kNoBoundary;
@@ -1032,11 +1170,15 @@ __device__ __forceinline__ void collide_kernel_body(DEM_COLLIDE_PARAMS) {
 }
 
 template <bool kRadius, int kMat, int kMode, bool kControl, bool kO>
-__global__ __launch_bounds__(256) void k_collide(DEM_COLLIDE_PARAMS) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMode == kList ? 7 : 1))) void k_collide(DEM_COLLIDE_PARAMS) {
   collide_kernel_body<kRadius, kMat, kMode, kControl, kO>(c, pos, vel, acc, omega, alpha, type, radius, cell_start,
                                                           cell_end, pressure, ctl, gat, quiet, n);
 }
 
+// The list mode is held to 72 VGPRs, 7 waves a SIMD: what spills then is the
+// walk of crowded neighbourhoods in passes.  (8 waves, 64 VGPRs and 78 SGPRs,
+// spill on the common path: 131 us against 128 on the 4M dense pack, 159
+// against 143 on the 8.2M-disc ensemble.)
 // The one-material batched mode needed 65 VGPRs with 64-bit addresses; held to 64 (8
 // waves per SIMD) it does not spill.  The other batched layouts would spill
 // 12-19 registers under the same bound, so they keep k_collide.
@@ -1206,13 +1348,13 @@ __global__ __launch_bounds__(256) void k_integrate(
   // loaded before any output is stored (the in and out arrays may be the
   // same, so the compiler could not move a later particle's loads above an
   // earlier one's stores); each lane reads and writes only its own slots.
-  const uint32_t base = blockIdx.x * blockDim.x * kPer + threadIdx.x;
+  const uint32_t base = blockIdx.x * c.block * kPer + threadIdx.x;
   uint32_t t[kPer];
   float2 p_old[kPer], v[kPer], a[kPer];
   float w[kPer], th[kPer], al[kPer], rad[kPer];
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
-    const uint32_t i = base + (uint32_t)k * blockDim.x;
+    const uint32_t i = base + (uint32_t)k * c.block;
     if (i >= n) continue;
     if (kNext == 2) next_clear(nk, i, n);
     t[k] = kMat == kOneMat ? 0u : clamp_idx(type[i], c.num_types);
@@ -1231,7 +1373,7 @@ __global__ __launch_bounds__(256) void k_integrate(
   }
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
-    const uint32_t i = base + (uint32_t)k * blockDim.x;
+    const uint32_t i = base + (uint32_t)k * c.block;
     if (i >= n) continue;
     auto run = [&](const Material& m, const Instance& in) {
       float r, mass, inertia;
@@ -1274,13 +1416,13 @@ __global__ __launch_bounds__(256) void k_integrate(
 // be theta_in).  The arithmetic is that of k_collide followed by k_integrate.
 // One pass instead of two reads positions, radii and cell ranges once, writes
 // no accelerations to read back, and streams while collide's instructions,
-// which bound it, issue: 76 us against 50 + 29 for 4M settling discs, 162
-// against 150 + 42 on the 4M dense pack, 206 against 136 + 82 on the
+// which bound it, issue: 67 us against 53 + 29 for 4M settling discs, 145
+// against 128 + 42 on the 4M dense pack, 209 against 143 + 82 on the
 // 8.2M-disc ensemble.  (There material rows and geometries are loaded per
 // lane: collide's second code path, with them in scalar registers where a
 // wave lies in one instance, takes 87 registers here, and 221 us.)
 template <bool kRadius, int kMat, bool kWhole, int kMode, bool kControl, bool kO>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWhole ? 4 : (kMat == kOneMat ? 8 : 7)))) void k_collide_integrate(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWhole ? 4 : 7))) void k_collide_integrate(
     StepConst c, const float2* __restrict__ pos_in, const float2* __restrict__ vel_in,
     const float* __restrict__ omega_in, const float* theta_in, const uint32_t* __restrict__ type,
     const float* __restrict__ radius, const uint32_t* __restrict__ cell_start,
@@ -1337,14 +1479,16 @@ inline int per_of(int per) { return per == 2 || per == 4 ? per : 1; }
 hipError_t launch_hash(const StepConst& c, hipStream_t s, int block, const float2* pos,
                        const uint32_t* type, uint32_t* hash, uint32_t* index, uint32_t n, int per) {
   if (n == 0) return hipSuccess;
+  StepConst cb = c;
+  cb.block = (uint32_t)block;
   per = per_of(per);
   const dim3 grid = grid_for((n + (uint32_t)per - 1u) / (uint32_t)per, block);
 #define DEM_HASH(P)                                                                                        \
   do {                                                                                                    \
     if (type && c.num_instances > 1)                                                                      \
-      hipLaunchKernelGGL((k_hash<true, P>), grid, dim3(block), 0, s, c, pos, type, hash, index, n);       \
+      hipLaunchKernelGGL((k_hash<true, P>), grid, dim3(block), 0, s, cb, pos, type, hash, index, n);       \
     else                                                                                                  \
-      hipLaunchKernelGGL((k_hash<false, P>), grid, dim3(block), 0, s, c, pos, type, hash, index, n);      \
+      hipLaunchKernelGGL((k_hash<false, P>), grid, dim3(block), 0, s, cb, pos, type, hash, index, n);      \
   } while (0)
   DEM_PER(DEM_HASH, per);
 #undef DEM_HASH
@@ -1435,6 +1579,8 @@ hipError_t launch_collide(const StepConst& c, hipStream_t s, int block, const fl
                           const uint32_t* cell_end, float* pressure, uint32_t n, int mode,
                           const ControlOut* ctl, const uint32_t* gat, uint32_t* quiet) {
   if (n == 0) return hipSuccess;
+  StepConst cb = c;
+  cb.block = (uint32_t)block;
   if (quiet && block % kWave) return hipErrorInvalidValue;  // the flags cover aligned 64-particle runs
   const ControlOut co = ctl ? *ctl : ControlOut{};
   // 32-bit byte offsets reach every element while n * 8 B and cells * 4 B
@@ -1445,10 +1591,10 @@ hipError_t launch_collide(const StepConst& c, hipStream_t s, int block, const fl
   do {                                                                                                      \
     if (o32)                                                                                                \
       hipLaunchKernelGGL((collide_kernel<R, M, P, X, true>()), grid_for(n, block), dim3(block),                 \
-                         window_bytes(P, block), s, c, pos,                                                      \
+                         window_bytes(P, block), s, cb, pos,                                                      \
                          vel, acc, omega, alpha, type, radius, cell_start, cell_end, pressure, co, gat, quiet, n); \
     else                                                                                                    \
-      hipLaunchKernelGGL((collide_kernel<R, M, P, X, false>()), grid_for(n, block), dim3(block), 0, s, c,     \
+      hipLaunchKernelGGL((collide_kernel<R, M, P, X, false>()), grid_for(n, block), dim3(block), 0, s, cb,     \
                          pos, vel, acc, omega, alpha, type, radius, cell_start, cell_end, pressure, co, gat, quiet, \
                          n);                                                                                \
   } while (0)
@@ -1465,12 +1611,14 @@ hipError_t launch_collide_integrate(const StepConst& c, hipStream_t s, int block
                                     const NextKeys& next, uint32_t n, int mode, const ControlOut* ctl,
                                     uint32_t* quiet) {
   if (n == 0) return hipSuccess;
+  StepConst cb = c;
+  cb.block = (uint32_t)block;
   if (block % kWave) return hipErrorInvalidValue;  // waves must cover aligned 64-particle runs
   const ControlOut co = ctl ? *ctl : ControlOut{};
   const bool o32 = !(mode & kWideMode) && n <= (1u << 29) && c.cells <= (1u << 30);  // (launch_collide)
 #define DEM_CI_W(R, M, W, P, X)                                                                                    \
   hipLaunchKernelGGL((k_collide_integrate<R, M, W, P, X, P == kList>), grid_for(n, block), dim3(block),            \
-                     window_bytes(P, block), s, c, pos_in, vel_in, omega_in, theta_in, type, radius, cell_start,   \
+                     window_bytes(P, block), s, cb, pos_in, vel_in, omega_in, theta_in, type, radius, cell_start,   \
                      cell_end, acc, alpha, pressure, pos_out, vel_out, omega_out, theta_out, next, co, quiet, n)
 #define DEM_CI(R, M, P, X)                   \
   do {                                       \
@@ -1585,12 +1733,14 @@ hipError_t launch_integrate_to(const StepConst& c, hipStream_t s, int block, con
                                uint32_t n, const NextKeys* next, const uint32_t* gat, int per,
                                const uint32_t* quiet) {
   if (n == 0) return hipSuccess;
+  StepConst cb = c;
+  cb.block = (uint32_t)block;
   if (block % kWave) return hipErrorInvalidValue;  // waves must cover aligned 64-particle runs
   per = per_of(per);
   const dim3 grid = grid_for((n + (uint32_t)per - 1u) / (uint32_t)per, block);
   const NextKeys nk = next ? *next : NextKeys{};
 #define DEM_INTEGRATE(R, M, X, P)                                                                         \
-  hipLaunchKernelGGL((k_integrate<R, M, X, P>), grid, dim3(block), 0, s, c, pos_in, vel_in, theta_in,    \
+  hipLaunchKernelGGL((k_integrate<R, M, X, P>), grid, dim3(block), 0, s, cb, pos_in, vel_in, theta_in,    \
                      omega_in, pos_out, vel_out, theta_out, omega_out, acc, alpha, type, radius, pressure, nk, \
                      gat, quiet, n)
 #define DEM_INTEGRATE_X(R, M, P)            \

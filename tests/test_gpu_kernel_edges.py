@@ -271,3 +271,86 @@ def test_adjoint_of_large_state_lists(gpu_ctx):
     # a sum of n terms in another order: n eps of the terms' magnitudes at most
     scale = np.abs(par1).max()
     assert np.all(np.abs(parm - par1) <= 1e-9 * np.maximum(np.abs(par1), 1e-3 * scale))
+
+
+@pytest.mark.parametrize("flags", [1, 0])
+@pytest.mark.parametrize("extent", [(8.0, 7.3), (1e-3, 123.456), (3.1415927, 0.7)])
+def test_cell_keys_at_cell_borders(gpu_ctx, oracle, extent, flags):
+    """Positions at the floats around every cell border (and their negatives
+    and multiples beyond the grid): the quotient that decides the cell is the
+    correctly rounded one."""
+    from test_oracle_kat import one_type_scene
+
+    grid = (64, 128)
+    axes = []
+    for e, g in zip(extent, grid):
+        x = (np.arange(0, 2 * g + 1, dtype=np.float64) * e / g).astype(np.float32)
+        near = [x]
+        for way in (np.float32(-np.inf), np.float32(np.inf)):
+            y = x
+            for _ in range(3):
+                y = np.nextafter(y, way)
+                near.append(y)
+        x = np.concatenate(near)
+        axes.append(np.concatenate([x, -x]))
+    n = max(map(len, axes))
+    rng = np.random.default_rng(1)
+    pos = np.stack([rng.permutation(np.resize(a, n)) for a in axes], 1).astype(np.float32)
+    s = one_type_scene(pos, box=extent, grid=grid, flags=flags)
+    gpu_ctx.load_scene(s)
+    want, _ = oracle.calc_hash(oracle.System(s), s.pos, s.type)
+    h, i = dev(np.zeros(n, np.uint32)), dev(np.zeros(n, np.uint32))
+    api.calcHash(gpu_ctx, dev(s.pos), i, h, n)
+    gpu_ctx.synchronize()
+    assert np.array_equal(h.cpu().numpy().view(np.uint32), want)
+
+
+def check_one_step(gpu_ctx, oracle, s):
+    gpu_ctx.set_step_variant(contact_lists=True)
+    sim, ref = api.Simulation(gpu_ctx, s), oracle.Sim(s, "f32")
+    try:
+        sim.step(1)
+        ref.step(1)
+        got, want = sim.download(), ref.state()
+        for k in ("hash", "index", "pos", "vel", "omega", "acc", "alpha", "pressure"):
+            assert bits_equal(got[k], want[k]), k
+        assert np.count_nonzero(want["acc"]) > 0
+    finally:
+        sim.close()
+        ref.close()
+
+
+@pytest.mark.parametrize("attract", [0.0, 3.0])
+@pytest.mark.parametrize("m", [31, 32, 33, 63, 64, 65, 95, 200])
+def test_crowded_neighbourhoods(gpu_ctx, oracle, m, attract):
+    """m discs in three by three cells (one or two words of marks, then passes
+    over 31), one copy in a corner of the clamped grid, against the oracle."""
+    n = 2 * m
+    s = sc.column_collapse(seed=m, cols=n, n=n, box=(1.0, 0.5))
+    g = s.instances[0]
+    cell = np.array(g.box) / np.array(g.grid)
+    rng = np.random.default_rng(m)
+    at = rng.uniform(0.05, 2.95, (n, 2))
+    s.pos[:] = ((at + np.where(np.arange(n)[:, None] < m, 4.0, 0.0)) * cell).astype(np.float32)
+    s.vel[:] = (rng.normal(size=s.vel.shape) * 0.2).astype(np.float32)
+    s.omega[:] = (rng.normal(size=n) * 30.0).astype(np.float32)
+    s.materials[0].attract = attract
+    check_one_step(gpu_ctx, oracle, s)
+
+
+def test_contacts_at_the_ends_of_the_float_range(gpu_ctx, oracle):
+    """Pairs whose squared distance is tiny or whose direction has a subnormal
+    component: the law's roots and quotients round as sqrtf and a division."""
+    xs = [1e-45, 3e-45, 7e-42, 1e-39, 3e-38, 1e-19, 5e-19, 3e-16, 1e-12, 1e-7]
+    n = 2 * len(xs)
+    s = sc.column_collapse(seed=1, cols=n, n=n, box=(0.4, 0.5))
+    for k, x in enumerate(xs):
+        y = 0.02 + 0.04 * k
+        apart = 0.0 if x >= 1e-19 else 0.004 + 0.0001 * k
+        s.pos[2 * k] = (0.0, y)
+        s.pos[2 * k + 1] = (x, y + apart)
+    rng = np.random.default_rng(2)
+    s.vel[:] = (rng.normal(size=s.vel.shape) * 0.2).astype(np.float32)
+    s.vel[4:8] *= np.float32(1e-25)
+    s.omega[:] = 0.0
+    check_one_step(gpu_ctx, oracle, s)
