@@ -1417,10 +1417,10 @@ __global__ __launch_bounds__(256) void k_integrate(
 // One pass instead of two reads positions, radii and cell ranges once, writes
 // no accelerations to read back, and streams while collide's instructions,
 // which bound it, issue: 67 us against 53 + 29 for 4M settling discs, 145
-// against 128 + 42 on the 4M dense pack, 209 against 143 + 82 on the
-// 8.2M-disc ensemble.  (There material rows and geometries are loaded per
-// lane: collide's second code path, with them in scalar registers where a
-// wave lies in one instance, takes 87 registers here, and 221 us.)
+// against 128 + 42 on the 4M dense pack, 199 against 143 + 82 on the
+// 8.2M-disc ensemble (208 with material rows and geometries loaded per lane
+// in every wave; an ensemble of 300 discs an instance, where a fifth of the
+// waves straddle two, takes 30.5 us a step either way).
 template <bool kRadius, int kMat, bool kWhole, int kMode, bool kControl, bool kO>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWhole ? 4 : 7))) void k_collide_integrate(
     StepConst c, const float2* __restrict__ pos_in, const float2* __restrict__ vel_in,
@@ -1440,10 +1440,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWhole ? 4 
   // (small states do not fill the chip, so latency counts, not registers:
   // every load that can go out first does)
   const float th_first = kWhole ? theta_in[i] : 0.0f;
-  collide_particle<kRadius, kMat, kMode, kControl, kO, false, kWhole>(c, i, pos_in, d, type, radius, cell_start,
-                                                                      cell_end, n, own, ctl, fx, fy, moment, pres, 0u,
-                                                                      win);
-  const Material m = c.mat[own.t];
+  bool uniform = false;
+  uint32_t t0 = 0;
+  if constexpr (kMat == kInstances && !kWhole) {
+    // a wave inside one instance (all but the few that straddle a boundary)
+    // reads its material row and geometry as scalars
+    const uint32_t t = clamp_idx(type[i], c.num_types);
+    t0 = __builtin_amdgcn_readfirstlane(t);
+    uniform = __ballot(t != t0) == 0;
+    if (__builtin_expect(uniform, 1))
+      collide_particle<kRadius, kMat, kMode, kControl, kO, true, kWhole>(c, i, pos_in, d, type, radius, cell_start,
+                                                                         cell_end, n, own, ctl, fx, fy, moment, pres,
+                                                                         t0, win);
+  }
+  if (!uniform)
+    collide_particle<kRadius, kMat, kMode, kControl, kO, false, kWhole>(c, i, pos_in, d, type, radius, cell_start,
+                                                                        cell_end, n, own, ctl, fx, fy, moment, pres,
+                                                                        0u, win);
+  const Material m = uniform ? c.mat[t0] : c.mat[own.t];
   const Instance in = kMat == kInstances ? c.inst[clamp_idx(m.inst, c.num_instances)] : c.inst0;
   body<kRadius>(m, &own.r, 0u, own.r, own.mass, own.inertia);  // (again, rather than kept)
   float2 a;
