@@ -1576,6 +1576,12 @@ int dem_sim_autotune(dem_sim* m, uint32_t* block) {
   nk.key = m->key;  // the sort's input, free after it
   nk.bits = m->resort.bits;
   nk.tile_count = m->resort.tile_count;
+  if (sim_whole(m)) {
+    // the kernels that small states run list their movers (the next step, a
+    // radix-sorted one, clears the count)
+    nk.list = m->whole_list[0];
+    nk.list_count = m->whole_count;
+  }
   const float2* S_pos = m->pos[K];
   const float2* S_vel = m->vel[K];
   const float* S_theta = m->theta[K];
