@@ -685,12 +685,6 @@ hipError_t sim_forces(dem_sim* m, hipStream_t s, hipEvent_t* ev, const StepHook*
   }
   m->next_list = sim_whole(m);
   uint32_t* q = resorted ? m->quiet : nullptr;
-  // (After an in-place step, a radix-sorted step's hook still sees acc_lazy
-  // set: the adjoint's slot of the first step of a recomputed segment then
-  // takes +0 accelerations for the runs that the last in-place step marked
-  // quiet.  A known defect of states that re-sort in place, left as it was
-  // because mending it changes their gradients.)
-  if (resorted || sim_whole(m)) m->acc_lazy = resorted;
   if (ctx->fuse)
     e = dem::launch_collide_integrate(c, s, ctx->bs_collide, m->pos[t], m->vel[t], m->omega[t], m->theta[t],
                                       m->type[t], radius, m->cs[t], m->cell_end, m->acc, m->alpha, m->pressure,
@@ -701,6 +695,9 @@ hipError_t sim_forces(dem_sim* m, hipStream_t s, hipEvent_t* ev, const StepHook*
                             radius, m->cs[t], m->cell_end, m->pressure, n, collide_mode(ctx),
                             control ? &co : nullptr, gat, q);
   if (e != hipSuccess) return e;
+  // (before the hook, which takes +0 for the quiet runs of a lazy step: this
+  // step's, not those that an earlier one marked)
+  m->acc_lazy = resorted;
   if (ctx->fuse) flip_buffers(m);
   if (control) {
     e = dem::launch_control_finish(s, co, m->react_bx, m->react_by, m->react_bm, n, ctx->d_reaction, ctx->d_control,
@@ -724,7 +721,6 @@ hipError_t sim_forces(dem_sim* m, hipStream_t s, hipEvent_t* ev, const StepHook*
   m->cur = t;
   m->cell_start = m->cs[t];
   m->perm_list = list;
-  m->acc_lazy = resorted;
   return hipSuccess;
 }
 

@@ -57,6 +57,23 @@ def mixed_pack(cols=32, rows=32, seed=11) -> sc.Scene:
     return s
 
 
+def batch_of(one: sc.Scene, copies: int) -> sc.Scene:
+    """`copies` of a single-instance, single-material scene in one batch, each
+    an instance with a material row of its own."""
+    import dataclasses
+
+    many = one.copy()
+    for f in ("pos", "vel", "theta", "omega", "radius"):
+        setattr(many, f, np.concatenate([getattr(one, f)] * copies))
+    many.type = np.repeat(np.arange(copies, dtype=np.uint32), one.n)
+    many.id = np.arange(copies * one.n, dtype=np.uint32)
+    many.loc = many.id.copy()
+    g = one.instances[0]
+    many.instances = [dataclasses.replace(g, cell_base=k * g.cells) for k in range(copies)]
+    many.materials = [dataclasses.replace(one.materials[0], instance=k) for k in range(copies)]
+    return many
+
+
 def state_dict(s: sc.Scene) -> dict:
     return dict(pos=s.pos, vel=s.vel, theta=s.theta, omega=s.omega, id=s.id, type=s.type, loc=s.loc,
                 radius=s.radius)
