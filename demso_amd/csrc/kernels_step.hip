@@ -1324,7 +1324,8 @@ __device__ __forceinline__ void next_key(const StepConst& c, const NextKeys& nk,
   }
 }
 
-// NextKeys' other outputs, particle i's share.
+// NextKeys' other outputs, particle i's share (the launchers refuse a clear_n
+// for which cell + n could pass 2^32 and the loop start again).
 __device__ __forceinline__ void next_clear(const NextKeys& nk, uint32_t i, uint32_t n) {
   for (uint32_t cell = i; cell < nk.clear_n; cell += n) nk.clear[cell] = kEmpty;
   if (i == 0u && nk.listed) *nk.host_listed = *nk.listed;
@@ -1475,6 +1476,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWhole ? 4 
   if (theta_out != theta_in || __float_as_uint(th) != __float_as_uint(th_in)) theta_out[i] = th;
   next_key<kWhole>(c, nk, p, own.cell, in, i, n);
 }
+
+// Whether next_clear's index stays below 2^32.
+inline bool clear_ends(const NextKeys& nk, uint32_t n) { return nk.clear_n <= 0xFFFFFFFFu - n; }
 
 inline dim3 grid_for(uint32_t n, int block) { return dim3((n + (uint32_t)block - 1u) / (uint32_t)block); }
 
@@ -1628,6 +1632,7 @@ hipError_t launch_collide_integrate(const StepConst& c, hipStream_t s, int block
   StepConst cb = c;
   cb.block = (uint32_t)block;
   if (block % kWave) return hipErrorInvalidValue;  // waves must cover aligned 64-particle runs
+  if (!clear_ends(next, n)) return hipErrorInvalidValue;
   const ControlOut co = ctl ? *ctl : ControlOut{};
   const bool o32 = !(mode & kWideMode) && n <= (1u << 29) && c.cells <= (1u << 30);  // (launch_collide)
 #define DEM_CI_W(R, M, W, P, X)                                                                                    \
@@ -1750,6 +1755,7 @@ hipError_t launch_integrate_to(const StepConst& c, hipStream_t s, int block, con
   StepConst cb = c;
   cb.block = (uint32_t)block;
   if (block % kWave) return hipErrorInvalidValue;  // waves must cover aligned 64-particle runs
+  if (next && !clear_ends(*next, n)) return hipErrorInvalidValue;
   per = per_of(per);
   const dim3 grid = grid_for((n + (uint32_t)per - 1u) / (uint32_t)per, block);
   const NextKeys nk = next ? *next : NextKeys{};

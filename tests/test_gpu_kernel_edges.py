@@ -354,3 +354,45 @@ def test_contacts_at_the_ends_of_the_float_range(gpu_ctx, oracle):
     s.vel[4:8] *= np.float32(1e-25)
     s.omega[:] = 0.0
     check_one_step(gpu_ctx, oracle, s)
+
+
+@pytest.mark.parametrize("n,cells", [(1, 40), (300, 130), (300, 1000), (5000, 4000)])
+def test_sparse_grids_equal_radix(gpu_ctx, n, cells):
+    """Small states re-sort as a whole while their grid has at most 64 cells a
+    disc, and in place beyond."""
+    s = walkers(n, 11, cells, 30.0)
+    gpu_ctx.set_step_variant(fused=True, contact_lists=True)
+    a, b = api.Simulation(gpu_ctx, s), api.Simulation(gpu_ctx, s)
+    a.set_sort_mode(1)
+    b.set_sort_mode(2)
+    try:
+        for steps in (1, 1, 2, 5):
+            a.step(steps)
+            (b.step_graph if steps > 1 else b.step)(steps)
+            da, db = a.download(), b.download()
+            for k in FIELDS:
+                assert bits_equal(da[k], db[k]), (k, steps)
+    finally:
+        a.close()
+        b.close()
+
+
+def test_grid_of_nearly_2_to_the_32_cells(gpu_ctx):
+    """The largest grids: no kernel's cell index wraps (51 GB of cell arrays)."""
+    s = walkers(200000, 12, 700, 1.0)
+    s.instances = [sc.Instance(box=(7.2e2, 7.2e2), extent=(7.2e2, 7.2e2), grid=(65535, 65536))]
+    s.pos[:] = np.random.default_rng(12).uniform(1.0, 719.0, s.pos.shape).astype(np.float32)
+    out = []
+    for mode in (1, 2):
+        sim = api.Simulation(gpu_ctx, s)
+        try:
+            sim.set_sort_mode(mode)
+            sim.step(2)
+            sim.step_graph(4)
+            out.append(sim.download(extra=False))
+            movers = sim.mover_count()
+        finally:
+            sim.close()
+    assert movers > 0
+    for k in ("id", "type", "loc", "pos", "vel", "theta", "omega"):
+        assert bits_equal(out[0][k], out[1][k]), k
