@@ -617,6 +617,10 @@ void sim_free(dem_sim* m) {
 // can re-sort from them.
 namespace {
 
+// The small states' counters (dem::kWholeCounts words) of buffer b.
+uint32_t* whole_counts(dem_sim* m, int b) { return m->whole_count + b * (int)(kMoverLists * kMoverStride); }
+uint32_t* whole_listed(dem_sim* m, int b) { return m->whole_count + 2 * (int)(kMoverLists * kMoverStride) + b; }
+
 dem::ShiftState shift_state(dem_sim* m, int b) {
   dem::ShiftState st;
   st.pos = m->pos[b];
@@ -677,10 +681,10 @@ hipError_t sim_forces(dem_sim* m, hipStream_t s, hipEvent_t* ev, const StepHook*
   if (sim_whole(m)) {
     // the next step goes from buffer t to buffer o
     nk.list = m->whole_list[t];
-    nk.list_count = m->whole_count + t;
+    nk.list_count = whole_counts(m, t);
     nk.clear = m->cs[o];
     nk.clear_n = m->cells;
-    if (resorted) nk.listed = m->whole_count + 2 + t;  // (counted by this step's re-sort)
+    if (resorted) nk.listed = whole_listed(m, t);  // (counted by this step's re-sort)
     nk.host_listed = m->shift.host_listed;
   }
   m->next_list = sim_whole(m);
@@ -750,12 +754,12 @@ hipError_t sim_step_whole(dem_sim* m, hipStream_t s, hipEvent_t* ev, const StepH
     for (int k = 0; k < 2; ++k) (void)hipEventRecord(ev[k], s);
   dem::WholeMovers mv;
   mv.list = m->whole_list[o];
-  mv.count = m->whole_count + o;
+  mv.count = whole_counts(m, o);
   mv.bits = m->resort.bits;
   mv.key = m->key;
-  mv.next_count = m->whole_count + t;
-  mv.listed = m->whole_count + 2 + t;
-  mv.next_listed = m->whole_count + 2 + o;
+  mv.next_count = whole_counts(m, t);
+  mv.listed = whole_listed(m, t);
+  mv.next_listed = whole_listed(m, o);
   mv.host_count = m->resort.host_count;
   const hipError_t e = dem::launch_resort_whole(s, shift_state(m, o), shift_state(m, t), mv, m->sidx, m->cells, m->n);
   if (e != hipSuccess) return e;
@@ -800,7 +804,7 @@ hipError_t sim_step_on(dem_sim* m, hipStream_t s, hipEvent_t* ev, bool resort, c
     if (e != hipSuccess) return e;
     // this step's collide + integrate accumulates the next step's mover counts
     const uint32_t tiles = (n + dem::kResortTile - 1u) / dem::kResortTile;
-    e = sim_whole(m) ? dem::launch_fill(s, m->whole_count, 0u, 4)
+    e = sim_whole(m) ? dem::launch_fill(s, m->whole_count, 0u, kWholeCounts)
                      : dem::launch_fill(s, m->resort.tile_count, 0u, tiles);
     if (e != hipSuccess) return e;
     if (ev) (void)hipEventRecord(ev[1], s);
@@ -840,7 +844,7 @@ hipError_t sim_step_on(dem_sim* m, hipStream_t s, hipEvent_t* ev, bool resort, c
 // and 51 against 19 at 1,000; 65,536 discs 15.9 against 15.0 at 16 and 22.7
 // against 17.7 at 64 (and with movers the whole step is the faster: 54 against
 // 90 us at 16).  Hence kWholeSparse cells a disc and kWholeCells in all.
-constexpr uint32_t kWholeMax = 262144, kWholeSparse = 64, kWholeCells = 1u << 21;
+constexpr uint32_t kWholeSparse = 64, kWholeCells = 1u << 21;
 bool whole_fits(const dem_sim* m) {
   return m->n <= kWholeMax && m->cells <= kWholeCells && m->cells <= kWholeSparse * m->n;
 }
@@ -870,13 +874,22 @@ hipError_t sim_acc_complete(dem_sim* m, hipStream_t s) {
 // most n / kListedFrac particles.
 constexpr uint32_t kListedFrac = 4;
 
+// Whole re-sorts stay cheaper than radix-sorted steps up to about n / 8 movers
+// and this many (a step, whole against radix-sorted: 16,000 discs with 1,630
+// movers 35 against 42 us, with 6,289 63 against 62; 65,536 with 6,504 43
+// against 59, with 24,356 86 against 78; 262,144 with 4,201 65 against 72,
+// with 14,527 77 against 76, with 26,901 88 against 79).
+constexpr uint32_t kWholeMovers = 16384;
+
 bool sim_use_resort(dem_sim* m) {
   // (the movers must be listed as this step's re-sort reads them)
   if (!m->resort_ok || m->sort_mode == 1 || m->next_list != sim_whole(m)) return false;
   if (m->sort_mode == 2) return true;
-  // The radix sort and full reorder cost about the same every step.  The
-  // re-sort's movers step is one workgroup, fast up to a few thousand
-  // movers; in place, every particle it lists (its slot changed: each mover
+  // The radix sort and full reorder cost about the same every step.  A whole
+  // re-sort's cost grows slowly with its movers (kWholeMovers), and stays
+  // within twice a radix-sorted step's for any number of them, as the choice
+  // may come late.  In place and in the copy layout the movers step is one
+  // workgroup, fast up to a few thousand movers; in place, every particle it lists (its slot changed: each mover
   // shifts the particles between its old and new slot) has its state staged
   // and written back.  Past either limit the steps radix sort, and the
   // re-sort is tried again after 1, 2, 4 ... 64 radix-sorted steps (its
@@ -890,7 +903,7 @@ bool sim_use_resort(dem_sim* m) {
   const volatile uint32_t* h = m->h_count;
   const uint32_t movers = h[0], listed = h[1];
   const bool inplace = sim_inplace(m);
-  const uint32_t mover_limit = sim_whole(m) ? kWholeSorted : std::max(4096u, m->n / 64u);
+  const uint32_t mover_limit = sim_whole(m) ? std::min(m->n / 8u, kWholeMovers) : std::max(4096u, m->n / 64u);
   const uint32_t listed_limit = m->n / kListedFrac;
   const bool cheap = movers <= mover_limit && (!inplace || listed <= listed_limit);
   if (cheap) {
@@ -1033,8 +1046,8 @@ int dem_sim_create(dem_context* ctx, uint32_t n, uint32_t num_cells, int with_ra
   if (!r) r = sim_alloc(m, &m->shift.count, 4);
   if (!r) r = sim_alloc(m, &m->shift.tag, n);
   for (int b = 0; b < 2; ++b)
-    if (!r && whole_fits(m)) r = sim_alloc(m, &m->whole_list[b], std::max(n, dem::kWholeSorted));
-  if (!r) r = sim_alloc(m, &m->whole_count, 4);
+    if (!r && whole_fits(m)) r = sim_alloc(m, &m->whole_list[b], (size_t)dem::kMoverLists * dem::mover_list_cap(n));
+  if (!r) r = sim_alloc(m, &m->whole_count, dem::kWholeCounts);
   m->shift.pos = m->pos[kScratch];
   m->shift.vel = m->vel[kScratch];
   m->shift.theta = m->theta[kScratch];

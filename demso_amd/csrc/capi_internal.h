@@ -104,10 +104,10 @@ struct dem_sim {
   // (sim_acc_complete).
   uint32_t* quiet = nullptr;
   bool acc_lazy = false;
-  // Whole re-sort (dem::launch_resort_whole): the movers of the state in
-  // buffer b, their count and the particles the step from it listed
-  // (whole_count[0/1] and [2/3]); next_list says that the last step left them
-  // (rather than the mover counts per tile of the other re-sorts)
+  // Whole re-sort (dem::launch_resort_whole): the lists of movers of the state
+  // in buffer b and their counters (dem::kWholeCounts); next_list says that
+  // the last step left them (rather than the mover counts per tile of the
+  // other re-sorts)
   uint64_t* whole_list[2] = {};
   uint32_t* whole_count = nullptr;
   bool next_list = false;

@@ -180,15 +180,28 @@ hipError_t launch_resort_shift_apply(hipStream_t s, const ShiftState& st, const 
 // identity (only the listed slots are written).
 hipError_t launch_shift_index(hipStream_t s, const ShiftScratch& sh, uint32_t* index, uint32_t n,
                               bool identity_done = false);
-// Re-sort and reorder of a small state in one kernel, from its movers as
-// integrate listed them (NextKeys::list): every particle goes from its slot in
-// `from` (arrays in the order of from.skey) to its slot in `to`, with the
-// sorted keys and index, loc, and the cell ranges of reorderDataAndFindCell-
-// Start (to.cell_start all kEmpty before; cell_end is one array for both).
-// count movers are in list; next_count and next_listed are set to 0 for the
-// steps that follow, listed gains the particles whose slot or key changed.
+// Re-sort and reorder of a small state (at most kWholeMax particles) in one
+// kernel, from its movers as integrate listed them (NextKeys::list): every
+// particle goes from its slot in `from` (arrays in the order of from.skey) to
+// its slot in `to`, with the sorted keys and index, loc, and the cell ranges
+// of reorderDataAndFindCellStart (to.cell_start all kEmpty before; cell_end is
+// one array for both).  count movers are in list; next_count and next_listed
+// are set to 0 for the steps that follow, listed gains the particles whose
+// slot or key changed.
+// The movers are in kMoverLists lists of mover_list_cap(n) places each, wave w
+// appending to list w % kMoverLists, whose count is at count + kMoverStride *
+// (w % kMoverLists): one append a wave on one word, 4,096 of them at 262,144
+// discs, took 18 us a step where every wave has a mover.
+constexpr uint32_t kWholeMax = 262144;
+constexpr uint32_t kMoverLists = 4, kMoverStride = 32;
+inline __host__ __device__ uint32_t mover_list_cap(uint32_t n) {
+  return ((n + 63u) / 64u + kMoverLists - 1u) / kMoverLists * 64u;
+}
+// Counters of a state: for either buffer the movers' counts, then the
+// particles that the step from it listed.
+constexpr uint32_t kWholeCounts = 2u * kMoverLists * kMoverStride + 2u;
 struct WholeMovers {
-  const uint64_t* list = nullptr;  // at least kWholeSorted entries may be read
+  const uint64_t* list = nullptr;
   const uint32_t* count = nullptr;
   const uint32_t* bits = nullptr;  // the mover bits and keys (NextKeys)
   const uint32_t* key = nullptr;
@@ -197,9 +210,6 @@ struct WholeMovers {
   uint32_t* next_listed = nullptr;
   uint32_t* host_count = nullptr;
 };
-// Movers up to which their order is kept in LDS (more are counted through
-// one by one, for every particle).
-constexpr uint32_t kWholeSorted = 512;
 hipError_t launch_resort_whole(hipStream_t s, const ShiftState& from, const ShiftState& to, const WholeMovers& mv,
                                uint32_t* index, uint32_t num_cells, uint32_t n);
 hipError_t launch_reorder(hipStream_t s, int block, uint32_t* cell_start, uint32_t* cell_end,
@@ -233,9 +243,10 @@ struct NextKeys {
   uint32_t* bits = nullptr;
   uint32_t* tile_count = nullptr;
   // For launch_resort_whole, instead of tile_count: the movers' (key << 32 |
-  // slot), appended in any order to list from *list_count (zero before); the
-  // next step's cellStart, set to kEmpty here; and the last re-sort's count
-  // of listed particles, passed on to its host-mapped mirror (null: none).
+  // slot), appended in any order to the lists (WholeMovers; counts zero
+  // before); the next step's cellStart, set to kEmpty here; and the last
+  // re-sort's count of listed particles, passed on to its host-mapped mirror
+  // (null: none).
   uint64_t* list = nullptr;
   uint32_t* list_count = nullptr;
   uint32_t* clear = nullptr;

@@ -1307,6 +1307,7 @@ __device__ __forceinline__ void next_key(const StepConst& c, const NextKeys& nk,
   const bool mover = k != old;
   if (mover) nk.key[i] = k;  // a stayer's key is its sorted key
   const uint64_t moved = __ballot(mover);
+  const uint32_t list = kWhole ? i / (uint32_t)kWave % kMoverLists : 0u;
   uint32_t at = 0;
   if (__lane_id() == 0) {  // lane 0 holds the wave's first index, a multiple of 64
     const uint32_t w0 = i / 32u, nwords = (n + 31u) / 32u;
@@ -1314,13 +1315,14 @@ __device__ __forceinline__ void next_key(const StepConst& c, const NextKeys& nk,
     if (w0 + 1u < nwords) nk.bits[w0 + 1u] = (uint32_t)(moved >> 32);
     const uint32_t cnt = (uint32_t)__popcll(moved);
     if (cnt) {
-      if constexpr (kWhole) at = atomicAdd(nk.list_count, cnt);
+      if constexpr (kWhole) at = atomicAdd(nk.list_count + list * kMoverStride, cnt);
       else atomicAdd(&nk.tile_count[i / kResortTile], cnt);
     }
   }
   if (kWhole && moved) {
+    const uint32_t cap = mover_list_cap(n);
     at = __builtin_amdgcn_readfirstlane(at) + (uint32_t)__popcll(moved & ((1ull << __lane_id()) - 1ull));
-    if (mover && at < n) nk.list[at] = ((uint64_t)k << 32) | i;
+    if (mover && at < cap) nk.list[list * cap + at] = ((uint64_t)k << 32) | i;
   }
 }
 

@@ -825,113 +825,285 @@ __device__ __forceinline__ uint32_t insertion_point_start(uint32_t k, uint32_t p
   return first_above(prev_key, n, k);
 }
 
+// What a block of k_resort_whole works out from mover lists too long for LDS
+// (more than a wave's worth in one of them), in a bounded number of steps: its own particles'
+// pairs are sorted in LDS, the lists are read once (a mover among them adds
+// itself to the first of them above it, found by bisection), and prefix sums
+// over those counts give each particle the movers below it; prefix sums over
+// the mover bits give the movers before a position.  (Counting through the
+// list for every particle took 2.4 ms a step at 200,000 discs of which 3%
+// move; this takes 57 us, and 75 with 10%.)
+constexpr uint32_t kRunWords = 32;  // mover bits are summed by runs of 1,024
+constexpr uint32_t kRuns = kWholeMax / (32u * kRunWords);
+static_assert(kRuns == kPlaceThreads, "a thread per run");
+struct WholeRanks {
+  uint64_t part[kPlaceThreads];   // the block's movers' pairs (new key, position), then its stayers'
+  uint64_t pair[kPlaceThreads];   // ... sorted
+  uint64_t most[kPlaceThreads];   // the largest mover below each of those
+  uint32_t count[kPlaceThreads];  // the movers below each of those
+  uint32_t before[kRuns + 1];     // movers before each run
+  uint64_t wave_most[kPlaceThreads / kWave];
+  uint32_t wave_count[kPlaceThreads / kWave], wave_bits[kPlaceThreads / kWave], wave_movers[kPlaceThreads / kWave];
+};
+
+// Movers at positions below q.
+__device__ __forceinline__ uint32_t ranks_before(const WholeRanks& s, const uint32_t* __restrict__ bits, uint32_t q) {
+  const uint32_t w = q >> 5, run = w / kRunWords;
+  uint32_t c = s.before[run];
+#pragma unroll 4
+  for (uint32_t k = run * kRunWords; k < w; ++k) c += (uint32_t)__popc(bits[k]);
+  return c + (q & 31u ? (uint32_t)__popc(bits[w] & ((1u << (q & 31u)) - 1u)) : 0u);
+}
+
+// One past the last stayer below q (0: none).
+__device__ __forceinline__ uint32_t ranks_last_stayer(const WholeRanks& s, const uint32_t* __restrict__ bits, uint32_t q) {
+  while (q) {
+    const uint32_t w = (q - 1u) >> 5, in = ((q - 1u) & 31u) + 1u;  // the low `in` bits of word w
+    const uint32_t stay = ~bits[w] & (0xFFFFFFFFu >> (32u - in));
+    if (stay) return w * 32u + 32u - (uint32_t)__clz((int)stay);
+    q = w * 32u;
+    // whole runs of movers
+    for (uint32_t run = w / kRunWords; w % kRunWords == 0u && run; --run) {
+      if (s.before[run] - s.before[run - 1u] != kRunWords * 32u) break;
+      q -= kRunWords * 32u;
+    }
+  }
+  return 0u;
+}
+
+// Fills s for this block (x: each thread's pair, all ones past the end; list:
+// the wave's mover list, of count) and returns through below and pred the
+// movers below x and the largest of them.
+__device__ __forceinline__ void ranks_of(WholeRanks& s, const uint64_t* __restrict__ list, uint32_t count,
+                                         const uint32_t* __restrict__ bits, uint32_t n, uint64_t x, bool mover,
+                                         uint32_t& below, uint64_t& pred) {
+  const uint32_t tid = threadIdx.x, lane = __lane_id(), w = tid / (uint32_t)kWave;
+  const uint64_t movers = __ballot(mover);
+  if (lane == 0) s.wave_movers[w] = (uint32_t)__popcll(movers);
+  s.most[tid] = 0u;
+  s.count[tid] = 0u;
+  s.before[tid] = 0u;
+  __syncthreads();
+  // the runs' movers: four words a thread, eight threads a run
+  const uint32_t words = (n + 31u) / 32u;
+  for (uint32_t k = 4u * tid; k < (words + 31u) / 32u * 32u; k += 4u * kPlaceThreads) {
+    uint32_t c = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < 4u; ++u) c += k + u < words ? (uint32_t)__popc(bits[k + u]) : 0u;
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) c += (uint32_t)__shfl_xor((int)c, o);
+    if (lane % 8u == 0u) s.before[k / kRunWords] = c;
+  }
+  // the block's movers by themselves, and its stayers, whose pairs are in order
+  uint32_t mine = (uint32_t)__popcll(movers & ((1ull << lane) - 1ull)), own = 0;  // movers before this thread; in all
+#pragma unroll
+  for (uint32_t k = 0; k < kPlaceThreads / kWave; ++k) {
+    mine += k < w ? s.wave_movers[k] : 0u;
+    own += s.wave_movers[k];
+  }
+  s.part[mover ? mine : own + (tid - mine)] = x;
+  __syncthreads();
+  uint32_t rank = tid - mine;  // stayers below x, then also movers
+  if (mover) {
+    uint32_t lo = own, hi = kPlaceThreads;
+    while (lo < hi) {
+      const uint32_t mid = (lo + hi) >> 1;
+      if (s.part[mid] < x) lo = mid + 1u;
+      else hi = mid;
+    }
+    rank = lo - own;
+  }
+  for (uint32_t j = 0; j < own; ++j) rank += s.part[j] < x ? 1u : 0u;
+  s.pair[rank] = x;
+  __syncthreads();
+  // (four movers a thread at once, as a bisection is eight dependent reads;
+  // most movers are below or above all of the block's pairs)
+  constexpr uint32_t kAtOnce = 4;
+  const uint64_t first = s.pair[0], last = s.pair[kPlaceThreads - 1];
+  uint32_t first_count = 0;
+  uint64_t first_most = 0;
+  for (uint32_t j = lane; j < count; j += kAtOnce * (uint32_t)kWave) {
+    uint64_t y[kAtOnce];
+    bool among = false;
+#pragma unroll
+    for (uint32_t u = 0; u < kAtOnce; ++u) {
+      y[u] = j + u * kWave < count ? list[j + u * kWave] : ~0ull;  // (not below any)
+      first_count += y[u] < first ? 1u : 0u;
+      first_most = y[u] < first && y[u] > first_most ? y[u] : first_most;
+      among |= y[u] >= first && y[u] < last;
+    }
+    if (!among) continue;
+    uint32_t at[kAtOnce];  // the block's pairs at or below y (at most 255)
+#pragma unroll
+    for (uint32_t u = 0; u < kAtOnce; ++u) at[u] = 0;
+#pragma unroll
+    for (uint32_t step = kPlaceThreads / 2u; step; step >>= 1)
+#pragma unroll
+      for (uint32_t u = 0; u < kAtOnce; ++u)
+        if (s.pair[at[u] + step - 1u] <= y[u]) at[u] += step;
+#pragma unroll
+    for (uint32_t u = 0; u < kAtOnce; ++u)
+      if (y[u] >= first && y[u] < last) {
+        atomicAdd(&s.count[at[u]], 1u);
+        atomicMax((unsigned long long*)&s.most[at[u]], (unsigned long long)y[u]);
+      }
+  }
+  if (first_count) {
+    atomicAdd(&s.count[0], first_count);
+    atomicMax((unsigned long long*)&s.most[0], (unsigned long long)first_most);
+  }
+  // inclusive prefixes over the particles (counts, largest) and the runs
+  const uint32_t run = s.before[tid];
+  uint32_t r = wave_inclusive_scan(run);
+  if (lane == kWave - 1) s.wave_bits[w] = r;
+  __syncthreads();
+  uint32_t c = wave_inclusive_scan(s.count[tid]);
+  uint64_t b = s.most[tid];
+#pragma unroll
+  for (uint32_t o = 1; o < (uint32_t)kWave; o <<= 1) {
+    const uint64_t y = __shfl_up((unsigned long long)b, o);
+    b = lane >= o && y > b ? y : b;
+  }
+  if (lane == kWave - 1) {
+    s.wave_count[w] = c;
+    s.wave_most[w] = b;
+  }
+  __syncthreads();
+  for (uint32_t k = 0; k < w; ++k) {
+    r += s.wave_bits[k];
+    c += s.wave_count[k];
+    b = s.wave_most[k] > b ? s.wave_most[k] : b;
+  }
+  s.before[tid] = r - run;
+  if (tid == kPlaceThreads - 1) s.before[kRuns] = r;
+  s.count[tid] = c;
+  s.most[tid] = b;
+  __syncthreads();
+  below = s.count[rank];
+  pred = s.most[rank];
+}
+
+static_assert(kMoverLists == kPlaceThreads / kWave, "a list a wave");
+
 template <bool kRadius>
 __global__ __launch_bounds__(kPlaceThreads) void k_resort_whole(ShiftState from, ShiftState to, WholeMovers mv,
                                                                 uint32_t* __restrict__ index, uint32_t num_cells,
                                                                 uint32_t n) {
-  constexpr uint32_t kEach = kWholeSorted / kPlaceThreads;
-  __shared__ uint64_t s_raw[kWholeSorted];   // as listed
-  __shared__ uint64_t s_pair[kWholeSorted];  // by (new key, position)
-  __shared__ uint32_t s_pos[kWholeSorted];   // by position
-  __shared__ uint32_t s_key[kWholeSorted];   // the new keys, by position
+  struct Sorted {
+    uint64_t raw[kPlaceThreads];   // as listed
+    uint64_t pair[kPlaceThreads];  // by (new key, position)
+    uint32_t pos[kPlaceThreads];   // by position
+    uint32_t key[kPlaceThreads];   // the new keys, by position
+  };
+  __shared__ union {
+    Sorted few;
+    WholeRanks many;
+  } sh;
+  __shared__ uint32_t s_changed[kPlaceThreads / kWave];
+  Sorted& s = sh.few;
   const uint32_t tid = threadIdx.x, i = blockIdx.x * kPlaceThreads + tid;
   const bool ok = i < n;
   const uint32_t ii = ok ? i : 0u;
-  const uint32_t m = *mv.count;
-  uint64_t raw[kEach];
+  // (a wave takes a list; its first places may be read whatever the count)
+  const uint32_t cap = mover_list_cap(n), w = tid / (uint32_t)kWave, lane = __lane_id();
+  uint32_t count[kMoverLists];
 #pragma unroll
-  for (uint32_t e = 0; e < kEach; ++e) raw[e] = mv.list[e * kPlaceThreads + tid];
+  for (uint32_t l = 0; l < kMoverLists; ++l) count[l] = mv.count[l * kMoverStride];
+  const uint64_t raw = mv.list[w * cap + lane];
   const uint32_t old = from.skey[ii], before_key = from.skey[ii ? ii - 1u : 0u];
   const float2 pos = from.pos[ii], vel = from.vel[ii];
   const float theta = from.theta[ii], omega = from.omega[ii], radius = kRadius ? from.radius[ii] : 0.0f;
   const uint32_t id = from.id[ii], type = from.type[ii];
+  uint32_t m = 0, ahead = 0, own = 0;  // movers; in the lists before this wave's; in its own
+  bool few = true;
+#pragma unroll
+  for (uint32_t l = 0; l < kMoverLists; ++l) {
+    count[l] = min(count[l], cap);
+    m += count[l];
+    ahead += l < w ? count[l] : 0u;
+    own = l == w ? count[l] : own;
+    few = few && count[l] <= (uint32_t)kWave;
+  }
+  if (i < kMoverLists) mv.next_count[i * kMoverStride] = 0u;
   if (i == 0) {
-    *mv.next_count = 0u;
     *mv.next_listed = 0u;
     if (mv.host_count) *mv.host_count = m;
   }
-  const bool sorted = m <= kWholeSorted;
-  if (sorted && m) {
-#pragma unroll
-    for (uint32_t e = 0; e < kEach; ++e) s_raw[e * kPlaceThreads + tid] = raw[e];
-    __syncthreads();
-#pragma unroll
-    for (uint32_t e = 0; e < kEach; ++e) {
-      if (e * kPlaceThreads + tid >= m) continue;
-      const uint64_t x = raw[e];
-      uint32_t by_pair = 0, by_pos = 0;  // the positions differ, so both ranks are unique
-      for (uint32_t j = 0; j < m; ++j) {
-        const uint64_t y = s_raw[j];
-        by_pair += y < x ? 1u : 0u;
-        by_pos += (uint32_t)y < (uint32_t)x ? 1u : 0u;
+  bool mover = false;
+  uint32_t key = old;
+  uint32_t below = 0;       // movers whose pair is below this one's,
+  uint64_t mover_pred = 0;  // ... and the largest of them (below == 0: none)
+  uint32_t at = ii;         // the stayers before it are those at positions below at,
+  uint32_t gone = 0;        // of which these are movers
+  uint32_t q = 0;           // one past the last stayer below at
+  // Each block ranks the movers one by one while there are few (at most a
+  // wave's worth in each list: 131,072 discs with 278 movers take 45 us a step
+  // so, 38 by ranks_of; 65,536 with 178 28 against 31).
+  if (few) {
+    if (m) {
+      if (lane < own) s.raw[ahead + lane] = raw;
+      __syncthreads();
+      if (lane < own) {
+        uint32_t by_pair = 0, by_pos = 0;  // the positions differ, so both ranks are unique
+        for (uint32_t j = 0; j < m; ++j) {
+          const uint64_t y = s.raw[j];
+          by_pair += y < raw ? 1u : 0u;
+          by_pos += (uint32_t)y < (uint32_t)raw ? 1u : 0u;
+        }
+        s.pair[by_pair] = raw;
+        s.pos[by_pos] = (uint32_t)raw;
+        s.key[by_pos] = (uint32_t)(raw >> 32);
       }
-      s_pair[by_pair] = x;
-      s_pos[by_pos] = (uint32_t)x;
-      s_key[by_pos] = (uint32_t)(x >> 32);
+      __syncthreads();
     }
-    __syncthreads();
-  }
-  // movers at positions below q
-  auto movers_before_pos = [&](uint32_t q) {
-    uint32_t lo = 0;
-    if (sorted) {
-      uint32_t hi = m;
+    // movers at positions below p
+    auto movers_before_pos = [&](uint32_t p) {
+      uint32_t lo = 0, hi = m;
       while (lo < hi) {
         const uint32_t mid = (lo + hi) >> 1;
-        if (s_pos[mid] < q) lo = mid + 1u;
+        if (s.pos[mid] < p) lo = mid + 1u;
         else hi = mid;
       }
-    } else {
-      for (uint32_t j = 0; j < m; ++j) lo += (uint32_t)mv.list[j] < q ? 1u : 0u;
-    }
-    return lo;
-  };
-  bool mover = false;
-  uint32_t key = old, own_rank = 0;
-  if (sorted) {
-    own_rank = movers_before_pos(ii);
-    mover = own_rank < m && s_pos[own_rank] == ii;
-    if (mover) key = s_key[own_rank];
-  } else {
-    mover = (mv.bits[ii >> 5] >> (ii & 31u)) & 1u;
-    if (mover) key = mv.key[ii];
-  }
-  // movers whose pair is below this one's, and the largest of them
-  const uint64_t x = composite(key, ii);
-  uint32_t below = 0;
-  uint64_t mover_pred = 0;  // (below == 0: none)
-  if (sorted) {
+      return lo;
+    };
+    gone = movers_before_pos(ii);
+    mover = gone < m && s.pos[gone] == ii;
+    if (mover) key = s.key[gone];
+    const uint64_t x = composite(key, ii);
     uint32_t hi = m;
     while (below < hi) {
       const uint32_t mid = (below + hi) >> 1;
-      if (s_pair[mid] < x) below = mid + 1u;
+      if (s.pair[mid] < x) below = mid + 1u;
       else hi = mid;
     }
-    if (below) mover_pred = s_pair[below - 1u];
+    if (below) mover_pred = s.pair[below - 1u];
+    if (mover) {
+      at = insertion_point_start(key, ii, from.skey, from.cell_start, num_cells, n);
+      gone = movers_before_pos(at);
+    }
+    q = at;
+    for (uint32_t g = gone; q && g && s.pos[g - 1u] == q - 1u; --g) --q;
   } else {
-    for (uint32_t j = 0; j < m; ++j) {
-      const uint64_t y = mv.list[j];
-      if (y < x) {
-        ++below;
-        mover_pred = y > mover_pred ? y : mover_pred;
-      }
+    mover = ok && ((mv.bits[ii >> 5] >> (ii & 31u)) & 1u);
+    if (mover) key = mv.key[ii];
+    ranks_of(sh.many, mv.list + w * cap, own, mv.bits, n, ok ? composite(key, ii) : ~0ull, mover, below, mover_pred);
+    if (mover) at = insertion_point_start(key, ii, from.skey, from.cell_start, num_cells, n);
+    gone = ranks_before(sh.many, mv.bits, at);
+    q = ranks_last_stayer(sh.many, mv.bits, at);
+  }
+  const uint32_t slot = below + at - gone;
+  if (m) {
+    // (one atomic a block: one a wave, 4,096 on one word, took 18 us)
+    const uint64_t lanes = __ballot(ok && (mover || slot != i));
+    if (lane == 0) s_changed[w] = (uint32_t)__popcll(lanes);
+    __syncthreads();
+    if (tid == 0) {
+      uint32_t changed = 0;
+#pragma unroll
+      for (uint32_t k = 0; k < kPlaceThreads / kWave; ++k) changed += s_changed[k];
+      if (changed) atomicAdd(mv.listed, changed);
     }
   }
-  // the stayers before it: those at positions below at
-  uint32_t at = ii, gone = own_rank;
-  if (mover) at = insertion_point_start(key, ii, from.skey, from.cell_start, num_cells, n);
-  if (mover || !sorted) gone = movers_before_pos(at);
-  const uint32_t slot = below + at - gone;
-  // the last stayer below at
-  uint32_t q = at;
-  if (sorted) {
-    for (uint32_t g = gone; q && g && s_pos[g - 1u] == q - 1u; --g) --q;
-  } else {
-    while (q && ((mv.bits[(q - 1u) >> 5] >> ((q - 1u) & 31u)) & 1u)) --q;
-  }
-  const bool changed = ok && (mover || slot != i);
-  const uint64_t lanes = __ballot(changed);
-  if (lanes && __lane_id() == 0) atomicAdd(mv.listed, (uint32_t)__popcll(lanes));
   if (!ok || slot >= n) return;  // (always below n for a consistent input)
   // the key before this one in the new order
   uint32_t pred = mover_pred ? (uint32_t)(mover_pred >> 32) : 0u;
@@ -1029,6 +1201,7 @@ hipError_t launch_shift_index(hipStream_t s, const ShiftScratch& sh, uint32_t* i
 hipError_t launch_resort_whole(hipStream_t s, const ShiftState& from, const ShiftState& to, const WholeMovers& mv,
                                uint32_t* index, uint32_t num_cells, uint32_t n) {
   if (n == 0) return hipSuccess;
+  if (n > kWholeMax) return hipErrorInvalidValue;
   for (const ShiftState* st : {&from, &to})
     if (!st->pos || !st->vel || !st->theta || !st->omega || !st->id || !st->type || !st->loc || !st->skey ||
         !st->cell_start || !st->cell_end)

@@ -396,3 +396,63 @@ def test_grid_of_nearly_2_to_the_32_cells(gpu_ctx):
     assert movers > 0
     for k in ("id", "type", "loc", "pos", "vel", "theta", "omega"):
         assert bits_equal(out[0][k], out[1][k]), k
+
+
+def hoppers(n, slots):
+    """n discs a cell apart, of which those at the given sorted slots hop to
+    the free cell on their right or above in the first step."""
+    cols = int(np.ceil(np.sqrt(n)))
+    s = sc.column_collapse(seed=1, cols=cols, n=n, box=((2 * cols + 4) * 0.011, (2 * cols + 4) * 0.011), dt=1e-4)
+    k = np.arange(n)
+    g = s.instances[0]
+    cell = np.array(g.extent) / np.array(g.grid)
+    s.pos[:] = ((np.stack([k % cols, k // cols], 1) * 2 + 0.5) * cell).astype(np.float32)
+    s.radius[:] = 0.0045
+    s.vel[slots, np.asarray(slots) % 2] = 110.0
+    return s
+
+
+# the small states' mover lists (a list takes every fourth wave's): one list
+# exactly full for the ranking of few, one over, all four full, one over; whole
+# runs of 1,024 movers; every disc
+HOPS = {
+    "one_list_64": (4099, np.arange(64)),
+    "one_list_65": (4099, np.r_[np.arange(64), 256]),
+    "lists_full": (4099, np.arange(256)),
+    "lists_full_and_1": (4099, np.arange(257)),
+    "first_and_last": (4099, np.array([0, 4098])),
+    "random_1000": (20037, np.random.default_rng(0).choice(20037, 1000, replace=False)),
+    "runs": (70001, np.r_[np.arange(1000, 5200), np.arange(66000, 70001)]),
+    "all_300": (300, np.arange(300)),
+    "all_5000": (5000, np.arange(5000)),
+    "random_20000": (262143, np.random.default_rng(1).choice(262143, 20000, replace=False)),
+    "all_262144": (262144, np.arange(262144)),
+}
+
+
+@pytest.mark.parametrize("name", list(HOPS))
+@pytest.mark.parametrize("fused", [False, True])
+def test_mover_lists_equal_radix(gpu_ctx, name, fused):
+    n, slots = HOPS[name]
+    s = hoppers(n, slots)
+    gpu_ctx.set_step_variant(fused=fused, contact_lists=True)
+    a, b = api.Simulation(gpu_ctx, s), api.Simulation(gpu_ctx, s)
+    a.set_sort_mode(1)
+    b.set_sort_mode(2)
+    try:
+        for k in range(4):
+            a.step(1)
+            b.step(1)
+            da, db = a.download(), b.download()
+            if k == 1:
+                assert b.mover_count() == len(slots)
+            for f in FIELDS:
+                assert bits_equal(da[f], db[f]), (f, k)
+        a.step(4)
+        b.step_graph(4)
+        da, db = a.download(), b.download()
+        for f in FIELDS:
+            assert bits_equal(da[f], db[f]), f
+    finally:
+        a.close()
+        b.close()
