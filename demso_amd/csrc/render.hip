@@ -109,19 +109,26 @@ __global__ __launch_bounds__(256) void k_plot_claim(RenderConst rc, const Render
                                                     const float* __restrict__ radius, uint32_t* __restrict__ owner,
                                                     uint32_t n) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  bool beyond = false;
+  uint32_t top = 0;  // the last of the disc's pixels
   if (i < n) {
     const Disc d = disc_of(rc, tt, pos[i], type[i], radius, i);
     const float pr2 = d.pr * d.pr;
-    for (int x = -d.h; x < d.h; ++x)
-      for (int y = -d.h; y < d.h; ++y)
-        if ((float)(x * x + y * y) < pr2) {
-          const uint32_t gx = (uint32_t)(d.cx + x), gy = (uint32_t)(d.cy + y);
-          const uint32_t pixel = gx + gy * (uint32_t)rc.dimx;
-          if (pixel < rc.npix) atomicMax(&owner[pixel], i + 1u);
-          else beyond = true;
-        }
+    // (both loops step x x + y y and the pixel instead of multiplying: the
+    // test against the image costs the loop no time then)
+    for (int x = -d.h; x < d.h; ++x) {
+      int r2 = x * x + d.h * d.h, odd = 1 - 2 * d.h;
+      uint32_t pixel = (uint32_t)d.cx + (uint32_t)x + ((uint32_t)d.cy - (uint32_t)d.h) * (uint32_t)rc.dimx;
+      for (int y = -d.h; y < d.h; ++y) {
+        const bool in = (float)r2 < pr2;
+        top = max(top, in ? pixel : 0u);
+        if (in & (pixel < rc.npix)) atomicMax(&owner[pixel], i + 1u);
+        r2 += odd;
+        odd += 2;
+        pixel += (uint32_t)rc.dimx;
+      }
+    }
   }
+  const bool beyond = top >= rc.npix;
   const uint64_t lanes = __ballot(beyond);
   if (beyond && (lanes >> __lane_id()) == 1ull) atomicMax(&owner[rc.npix - 1u], i + 1u);
 }
@@ -357,7 +364,9 @@ int dem_update_pressure_scale(dem_context* ctx, const float* pressure, uint32_t 
   hipStream_t s = ctx->stream;
   hipLaunchKernelGGL(k_zero_word, dim3(1), dim3(1), 0, s, ctx->d_scalar);
   if (numParticles) {
-    const uint32_t blocks = std::min<uint32_t>((numParticles + 1023u) / 1024u, 1024u);
+    // a value a thread up to 65,536, then more a thread up to 1,024 blocks
+    const uint32_t blocks = std::min(std::max((numParticles + 1023u) / 1024u, std::min((numParticles + 255u) / 256u, 256u)),
+                                     1024u);
     hipLaunchKernelGGL(k_max_key, dim3(blocks), dim3(256), 0, s, pressure, numParticles, ctx->d_scalar);
   }
   uint32_t key = 0;
