@@ -1569,17 +1569,19 @@ inline int mat_kind(const StepConst& c) {
       else MACRO(false, kManyMat, MODE, X);                              \
     }                                                                    \
   } while (0)
-// (the controlled particle needs a single instance: launches with one are
-// refused for an ensemble)
+// (a controlled particle is set for a single instance; an ensemble that the
+// context is given afterwards meets it in every instance, one candidate at a
+// time)
 #define DEM_DISPATCH_CTL(MACRO, MODE)                                    \
   do {                                                                   \
     const int mk_ = mat_kind(c);                                         \
-    if (mk_ == kInstances) return hipErrorInvalidValue;                  \
     if (radius) {                                                        \
-      if (mk_ == kOneMat) MACRO(true, kOneMat, MODE, true);              \
+      if (mk_ == kInstances) MACRO(true, kInstances, kPlain, true);      \
+      else if (mk_ == kOneMat) MACRO(true, kOneMat, MODE, true);         \
       else MACRO(true, kManyMat, MODE, true);                            \
     } else {                                                             \
-      if (mk_ == kOneMat) MACRO(false, kOneMat, MODE, true);             \
+      if (mk_ == kInstances) MACRO(false, kInstances, kPlain, true);     \
+      else if (mk_ == kOneMat) MACRO(false, kOneMat, MODE, true);        \
       else MACRO(false, kManyMat, MODE, true);                           \
     }                                                                    \
   } while (0)

@@ -142,3 +142,35 @@ def test_controlled_particle_wraps_and_is_refused_by_the_adjoint(oracle):
     sim.step(1)
     sim.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("variant", [dict(), dict(fused=True, contact_lists=True), dict(contact_lists=True),
+                                     dict(copy=True, fused=True)])
+def test_ensemble_loaded_after_the_controlled_particle(oracle, variant):
+    """A context whose controlled particle was set for a single instance and
+    that is then given an ensemble: every instance meets the particle."""
+    one = sc.column_collapse(cols=8, rows=8)
+    s = sc.ensemble(instances=3, counts=[300, 130, 77], seed=6)
+    ctx = api.Context(0)
+    ctx.load_scene(one)
+    kw = dict(pos=(0.02, 0.021), type=0, move=(1e-4, -5e-5))
+    ctx.set_controlled(**kw)
+    sim = api.Simulation(ctx, s)
+    ctx.set_step_variant(**variant)
+    ref = oracle.Sim(s, "f32")
+    ref.set_control(oracle.control(kw["pos"], 0, move=kw["move"], wrap_below_y=-1.0,
+                                   wrap_above_x=float(np.float32(one.instances[0].box[0])) + 0.5, reset_x=-0.5,
+                                   reset_y=10.5))
+    sim.step(3)
+    sim.step_graph(8)
+    ref.step(11)
+    g, o = sim.download(), ref.state()
+    state, reaction = ctx.controlled()
+    cs, red = ref.control()
+    for k in ("hash", "index", "pos", "vel", "theta", "omega", "acc", "alpha", "pressure"):
+        assert bits_equal(g[k], o[k]), k
+    assert state["pos"].tolist() == list(cs.pos)
+    assert bits_equal(reaction, red.astype(np.float32)) and np.abs(red).max() > 0
+    ref.close()
+    sim.close()
+    ctx.close()
