@@ -775,6 +775,9 @@ hipError_t sim_step_whole(dem_sim* m, hipStream_t s, hipEvent_t* ev, const StepH
 hipError_t sim_step_on(dem_sim* m, hipStream_t s, hipEvent_t* ev, bool resort, const StepHook* hook) {
   dem_context* ctx = m->ctx;
   const StepConst& c = ctx->c;
+  // A step that fails half-way leaves movers, counts and cells of two steps:
+  // the next one sorts from scratch (the callers set this again after a step).
+  m->resort_ok = false;
   if (resort && sim_whole(m)) return sim_step_whole(m, s, ev, hook);
   if (resort && sim_inplace(m)) return sim_step_inplace(m, s, ev, hook);
   // The state is in buffer o and the step writes buffer t.  Two layouts:
@@ -943,6 +946,7 @@ int sim_graph(dem_sim* m, bool resort, hipGraphExec_t* exec) {
       DEM_HIP(ctx, hipStreamCreateWithFlags(&m->cap_stream, hipStreamNonBlocking), "hipStreamCreate");
     const int saved = m->cur;
     const bool saved_flip = m->flipped, saved_list = m->perm_list, saved_lazy = m->acc_lazy;
+    const bool saved_ok = m->resort_ok, saved_next = m->next_list;
     uint32_t* const saved_key = m->sorted_key;
     uint32_t* const saved_idx = m->sorted_idx;
     hipGraph_t g = nullptr;
@@ -957,6 +961,8 @@ int sim_graph(dem_sim* m, bool resort, hipGraphExec_t* exec) {
     m->sorted_idx = saved_idx;
     m->perm_list = saved_list;
     m->acc_lazy = saved_lazy;
+    m->resort_ok = saved_ok;  // (no step has run)
+    m->next_list = saved_next;
     if (e1 != hipSuccess) {
       if (g) (void)hipGraphDestroy(g);
       return hip_fail(ctx, e1, "capturing the step");
