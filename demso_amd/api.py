@@ -110,13 +110,27 @@ class Context:
         self.device = device
         self.box = None  # (Lx, Ly) of the last scene loaded
         # simulations made on this context: destroyed before it, so that no
-        # sim outlives the C context it points to
+        # sim outlives the C context it points to.  The C handles too (each
+        # sim's, with its adjoints'): a garbage-collected cycle finalizes its
+        # objects in any order, with the weak references already cleared.
         self._sims = weakref.WeakSet()
+        self._open = {}
+
+    def _destroy_sim(self, handle) -> None:
+        """Destroys a sim and its adjoints, unless that has been done."""
+        adjoints = self._open.pop(handle, None)
+        if adjoints is None:
+            return
+        for adj in adjoints:
+            self.lib.dem_adj_destroy(adj)
+        self.lib.dem_sim_destroy(handle)
 
     def close(self) -> None:
         if self.handle:
             for sim in list(self._sims):
                 sim.close()
+            for handle in list(self._open):
+                self._destroy_sim(handle)
             self.lib.dem_destroy(self.handle)
             self.handle = None
 
@@ -467,13 +481,14 @@ class Simulation:
         self.handle = h.value
         self._adjoints = weakref.WeakSet()  # destroyed before this sim
         ctx._sims.add(self)
+        ctx._open[self.handle] = set()
         self.upload(scene)
 
     def close(self) -> None:
         if getattr(self, "handle", None):
             for adj in list(getattr(self, "_adjoints", ())):
                 adj.close()
-            self.lib.dem_sim_destroy(self.handle)
+            self.ctx._destroy_sim(self.handle)
             self.handle = None
 
     def __del__(self):
@@ -595,10 +610,14 @@ class Adjoint:
         sim.ctx._check(self.lib.dem_adj_create(sim.handle, checkpoint_every, byref(h)))
         self.handle = h.value
         sim._adjoints.add(self)
+        sim.ctx._open[sim.handle].add(self.handle)
 
     def close(self) -> None:
         if getattr(self, "handle", None):
-            self.lib.dem_adj_destroy(self.handle)
+            mine = self.sim.ctx._open.get(self.sim.handle, ())
+            if self.handle in mine:  # (not destroyed with its sim)
+                mine.remove(self.handle)
+                self.lib.dem_adj_destroy(self.handle)
             self.handle = None
 
     def __del__(self):
