@@ -162,19 +162,22 @@ class Context:
             self.set_materials(particle_props(scene, single_instance=False))
 
     def set_step_variant(self, fused: bool = False, prefetch: bool = False, batch: bool = False,
-                         copy: bool = False, wide: bool = False, contact_lists: bool = False,
+                         copy: bool = False, wide: bool = False, contact_lists: Optional[bool] = None,
                          per_lane: Optional[dict] = None) -> None:
         """Owned simulations: collide + integrate as one kernel or two, and
-        how collide loads its candidates: one at a time, one ahead
-        (prefetch) or the first of every row at once (batch); copy
+        how collide loads its candidates: one ahead (prefetch), the first of
+        every row at once (batch), by contact lists (contact_lists: the
+        candidates that may touch are marked before the contact law runs over
+        them; None, the default, takes them unless prefetch or batch is asked
+        for, as a new context does), or one at a time (False); copy
         makes re-sorted steps reorder the whole state into the other buffer
         instead of moving only the particles whose slot changes; wide
         makes collide use 64-bit addresses (as states over 2^29 particles
-        or 2^30 cells do); contact_lists makes collide mark the candidates that may
-        touch before running the contact law over them (contact-dense
-        states); per_lane gives the particles a lane (1, 2 or 4) of "hash",
+        or 2^30 cells do); per_lane gives the particles a lane (1, 2 or 4) of "hash",
         "reorder" and "integrate".  The results are the same in every
         combination."""
+        if contact_lists is None:
+            contact_lists = not (prefetch or batch)
         flags = (int(bool(fused)) | (2 if prefetch else 0) | (4 if batch else 0) | (8 if copy else 0)
                  | (16 if wide else 0) | (32 if contact_lists else 0))
         lg = {1: 0, 2: 1, 4: 2}

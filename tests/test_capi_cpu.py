@@ -112,3 +112,25 @@ def test_torch_extension_loads():
 
     mod = torch_ext.load()
     assert hasattr(mod, "trajectory")
+
+
+def test_step_variant_defaults():
+    """A caller who sets one knob keeps a new context's contact lists, unless
+    another candidate mode is asked for."""
+    from demso_amd import api
+
+    class Lib:
+        def dem_set_step_variant(self, handle, flags):
+            self.flags = flags
+            return 0
+
+        def dem_destroy(self, handle):
+            return 0
+
+    ctx = api.Context.__new__(api.Context)
+    ctx.lib, ctx.handle = Lib(), None
+    for kw, flags in (({}, 0x20), (dict(per_lane={"hash": 2}), 0x120), (dict(fused=True), 0x21),
+                      (dict(prefetch=True), 0x2), (dict(batch=True), 0x4), (dict(contact_lists=False), 0),
+                      (dict(contact_lists=True, copy=True), 0x28)):
+        ctx.set_step_variant(**kw)
+        assert ctx.lib.flags == flags, kw

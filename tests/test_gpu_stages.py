@@ -347,3 +347,20 @@ def test_step_variant_errors(gpu_ctx):
         gpu_ctx.set_step_variant(per_lane={"hash": 3})
     gpu_ctx.set_step_variant(contact_lists=True, per_lane={"hash": 4, "reorder": 2, "integrate": 4})
     gpu_ctx.set_step_variant()
+
+
+@pytest.mark.parametrize("name", list(SCENES))
+def test_collide_one_candidate_at_a_time(gpu_ctx, oracle, name):
+    """The plain mode, which a caller asks for by contact_lists=False."""
+    s = SCENES[name]
+    gpu_ctx.load_scene(s)
+    system, h, i, hs, is_, cs, ce, st = oracle_sorted(oracle, s)
+    n = s.n
+    acc, alpha, pres = dev(np.zeros((n, 2), np.float32)), dev(np.zeros(n, np.float32)), dev(np.full(n, 7.0, np.float32))
+    for wide in (False, True):
+        gpu_ctx.set_step_variant(contact_lists=False, wide=wide)
+        api.collide(gpu_ctx, dev(st["pos"]), dev(st["vel"]), acc, dev(st["omega"]), alpha, dev(st["type"]), dev(cs),
+                    dev(ce), n, s.total_cells, pres, radius=dev(st["radius"]) if st["radius"] is not None else None)
+        gpu_ctx.synchronize()
+        for got, want in zip((acc, alpha, pres), oracle.collide(system, st, cs, ce)):
+            assert bits_equal(host(got), want), wide
