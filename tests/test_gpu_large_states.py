@@ -3,8 +3,9 @@ batches of many small instances."""
 import numpy as np
 import pytest
 
+from demso_amd import api
 from demso_amd import scene as sc
-from helpers import batch_of, bits_equal
+from helpers import batch_of, bits_equal, mixed_pack
 from test_gpu_adjoint import gpu_grads
 
 pytestmark = pytest.mark.gpu
@@ -47,3 +48,69 @@ def test_checkpoint_interval_of_large_states(gpu_ctx, fused):
         assert bits_equal(finalk, final), K
         assert bits_equal(gpk, gp) and bits_equal(gvk, gv), K
         assert np.allclose(park, par, rtol=0, atol=1e-9 * np.abs(par).max(axis=0)), K
+
+
+def squeezed_batch(counts, seed):
+    s = sc.ensemble(seed=seed, instances=len(counts), counts=counts)
+    rng = np.random.default_rng(seed)
+    s.pos[:] *= np.float32(0.86)
+    s.vel[:] = (rng.normal(size=s.vel.shape) * 0.1).astype(np.float32)
+    s.omega[:] = (rng.normal(size=s.n) * 10.0).astype(np.float32)
+    return s
+
+
+def type_radii(s):
+    """The same discs with their material's radius, mass and inertia (the
+    generator's materials have none)."""
+    for m, r in zip(s.materials, np.random.default_rng(5).uniform(0.0048, 0.0054, len(s.materials))):
+        m.radius = float(r)
+        m.mass = m.areal * m.radius ** 2
+        m.inertia = 0.4 * m.mass * m.radius ** 2
+    s.radius = None
+    return s
+
+
+# waves inside one instance, waves across two or more (the last wave not
+# full), and several materials in a wave of one instance; radii of the discs
+# or of their materials
+STATES = {
+    "aligned": lambda: squeezed_batch([4416] * 60, 1),
+    "ragged": lambda: squeezed_batch(np.random.default_rng(3).integers(1000, 5000, 90).tolist(), 3),
+    "straddling": lambda: squeezed_batch(np.random.default_rng(2).integers(180, 420, 900).tolist(), 2),
+    "straddling_type_radii": lambda: type_radii(squeezed_batch([299] * 900, 4)),
+    "materials": lambda: mixed_pack(cols=521, rows=505),
+}
+FIELDS = ("hash", "index", "cellStart", "id", "type", "loc", "pos", "vel", "theta", "omega", "acc", "alpha", "pressure")
+
+
+@pytest.mark.parametrize("name", list(STATES))
+def test_large_states_step_alike_in_every_layout(oracle, name):
+    """Past 262,144 discs: contact lists, split and fused, re-sorted in place,
+    against the plain mode with the radix sort, and all against the oracle
+    after one step."""
+    s = STATES[name]()
+    assert s.n > 262144
+    ref = oracle.Sim(s, "f32")
+    ref.step(1)
+    want = ref.state()
+    ref.close()
+    assert np.count_nonzero(want["acc"]) > s.n // 4
+    base = None
+    for variant, mode in ((dict(contact_lists=False), 1), (dict(contact_lists=True), 2),
+                          (dict(contact_lists=True, fused=True), 2)):
+        ctx = api.Context(0)
+        sim = api.Simulation(ctx, s)
+        ctx.set_step_variant(**variant)
+        sim.set_sort_mode(mode)
+        sim.step(1)
+        got = sim.download()
+        for k in ("hash", "index", "pos", "vel", "theta", "omega", "acc", "alpha", "pressure"):
+            assert bits_equal(got[k], want[k]), (variant, k)
+        sim.step(2)
+        sim.step_graph(6)
+        got = sim.download()
+        base = base or got
+        for k in FIELDS:
+            assert bits_equal(got[k], base[k]), (variant, k)
+        sim.close()
+        ctx.close()
