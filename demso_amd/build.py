@@ -63,6 +63,22 @@ def build_library(verbose: bool = False) -> Path:
     return LIB
 
 
+CHECK = ROOT / "tests" / "contact_math_check.so"
+
+
+def build_check(verbose: bool = False) -> Path:
+    """Compile the GPU tests' check of csrc/contact_math.h, with the library's flags."""
+    tmp = CHECK.with_suffix(".so.tmp")
+    cmd = [hipcc(), *HIP_FLAGS, f"-I{CSRC}", "-o", str(tmp), str(CHECK.with_suffix(".hip"))]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"hipcc failed ({res.returncode}):\n{res.stderr}")
+    os.replace(tmp, CHECK)
+    return CHECK
+
+
 DRIVER = PKG / "demso_run"
 DRIVER_SOURCES = ["xml.cpp", "dsml.cpp", "prepare.cpp", "demso_run.cpp"]
 
@@ -100,5 +116,6 @@ def build_oracle(verbose: bool = False) -> Path:
 
 if __name__ == "__main__":
     print(build_library(verbose=True))
+    print(build_check(verbose=True))
     print(build_driver(verbose=True))
     print(build_oracle(verbose=True))
