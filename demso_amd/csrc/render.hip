@@ -364,9 +364,10 @@ int dem_update_pressure_scale(dem_context* ctx, const float* pressure, uint32_t 
   hipStream_t s = ctx->stream;
   hipLaunchKernelGGL(k_zero_word, dim3(1), dim3(1), 0, s, ctx->d_scalar);
   if (numParticles) {
-    // a value a thread up to 65,536, then more a thread up to 1,024 blocks
-    const uint32_t blocks = std::min(std::max((numParticles + 1023u) / 1024u, std::min((numParticles + 255u) / 256u, 256u)),
-                                     1024u);
+    // a value a thread up to 64 blocks (their atomics queue on one word: 256
+    // take 1 us more than 64), then four up to 1,024 blocks, then more
+    const uint32_t blocks =
+        std::min(std::max((numParticles + 1023u) / 1024u, std::min((numParticles + 255u) / 256u, 64u)), 1024u);
     hipLaunchKernelGGL(k_max_key, dim3(blocks), dim3(256), 0, s, pressure, numParticles, ctx->d_scalar);
   }
   uint32_t key = 0;
