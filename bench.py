@@ -520,7 +520,7 @@ def main() -> int:
     # a multi-kernel stage (3 kernels per radix pass) and is reported apart
     stages = sim.stage_times(max(5, min(args.steps, 50)))
     fused = bool(tuned and tuned.get("fused"))
-    layout = "copy" if tuned and tuned.get("copy") else ("whole" if n <= 262144 else "inplace")
+    layout = "copy" if tuned and tuned.get("copy") else ("whole" if n <= 262144 and cells <= min(64 * n, 1 << 21) else "inplace")
     if fused:
         layout += "_fused"
     acct = dict(layout=layout, radius=scene.radius is not None, typed=len(scene.materials) > 1)

@@ -890,11 +890,11 @@ bool sim_use_resort(dem_sim* m) {
   if (m->sort_mode == 2) return true;
   // The radix sort and full reorder cost about the same every step.  A whole
   // re-sort's cost grows slowly with its movers (kWholeMovers), and stays
-  // within twice a radix-sorted step's for any number of them, as the choice
-  // may come late.  In place and in the copy layout the movers step is one
-  // workgroup, fast up to a few thousand movers; in place, every particle it lists (its slot changed: each mover
-  // shifts the particles between its old and new slot) has its state staged
-  // and written back.  Past either limit the steps radix sort, and the
+  // within about twice a radix-sorted step's for any number of them, as the
+  // choice may come late.  In place and in the copy layout the movers step is
+  // one workgroup, fast up to a few thousand movers; in place, every particle
+  // it lists (its slot changed: each mover shifts the particles between its
+  // old and new slot) has its state staged and written back.  Past either limit the steps radix sort, and the
   // re-sort is tried again after 1, 2, 4 ... 64 radix-sorted steps (its
   // counts are only measured by a re-sort), or after 8, 16 ... 64 when the
   // counts were at twice a limit or more.  The counts are the latest the

@@ -600,11 +600,12 @@ __device__ __forceinline__ void shift_in(uint32_t (&w)[3], const float (&x)[3], 
 // (585 lookups a wave at 4M settling discs, where it was busy 93% of the
 // kernel's time) bound the kernel: with the windows it took 50 us there
 // (59), 150 us on the 4M dense pack (172), 136 us on the 8.2M-disc ensemble
-// (149).  Now vector instructions bound it (397 a wave there, 78% of the time
-// issuing): with one word of marks, the rows' ranges by minimum and maximum
-// and the short roots, quotients and cells, 53 us there (54, the same hour), 128
-// us on the dense pack (151), 143 us on the ensemble (152).  Three rows of kWindow entries, then
-// kWindowSlack more, as a lane with few candidates reads on past its row's.
+// (149).  Now vector instructions bound it: with one word of marks, the rows'
+// ranges by minimum and maximum and the short roots, quotients and cells, 53
+// us there (54 before, on the same machine) with 381 instructions a wave, 128
+// us on the dense pack (151) with 1,435, 143 us on the ensemble (152) with 478.
+// Three rows of kWindow entries, then kWindowSlack more, as a lane with few
+// candidates reads on past its row's.
 // An entry's three words lie together, so a lane's walk has one address a row
 // (and no bank conflict, a wave's lanes being 3 words apart).  Eight waves a
 // SIMD fit (32 x 5,120 bytes of 160 KB).

@@ -784,8 +784,8 @@ __global__ __launch_bounds__(256) void k_shift_apply(ShiftState st, ShiftScratch
 // and by position), each thread has its particle's state in flight meanwhile
 // and then knows its slot, and from the two orders also the pair before it
 // in the new order, which gives the cell ranges.  Only a mover waits for a
-// second round of loads, to find its new neighbours.  5.3 us at 65,536 discs
-// (a step 25 -> 13 us), 4.0 at 4,096.
+// second round of loads, to find its new neighbours.  6 us at 65,536 settled
+// discs (a step 25 -> 13 us), 3.5 at 4,096.
 
 // The first slot of the previous order whose key is above k, for a key that
 // is followed by no cell of cell_start's next kNextCells: 15 probes at once.

@@ -275,12 +275,14 @@ int dem_sim_autotune(dem_sim* sim, uint32_t* block);
 /* Sort method of the sim's steps.  After a step the state is in the sorted
  * order of its keys, so the next step can re-sort: only particles whose cell
  * changed are sorted and merged with the rest (same result as the radix
- * sort, bit for bit).  mode 0 (default): re-sort while the last re-sort's
- * counts (dem_sim_resort_counts) stay small (movers at most max(4096, n/64);
- * in place, at most n/4 particles listed), else radix sort and try the
- * re-sort again after 1, 2, 4 ... 64 radix-sorted steps (8, 16 ... 64 when a
- * count was twice its limit or more); 1: radix sort every
- * step; 2: re-sort whenever the state allows it.  The first step after
+ * sort, bit for bit).  Small states (at most 262,144 particles, 64 cells a
+ * particle and 2^21 cells) go into the other buffer whole, in one kernel;
+ * larger ones are re-sorted in place.  mode 0 (default): re-sort while the
+ * last re-sort's counts (dem_sim_resort_counts) stay small (movers at most
+ * min(n/8, 16384) as a whole, else max(4096, n/64); in place, at most n/4
+ * particles listed), else radix sort and try the re-sort again after 1, 2,
+ * 4 ... 64 radix-sorted steps (8, 16 ... 64 when a count was twice its limit
+ * or more); 1: radix sort every step; 2: re-sort whenever the state allows it.  The first step after
  * dem_sim_upload, dem_sim_set_by_id (positions), dem_sim_autotune or
  * dem_adj_backward always radix sorts. */
 int dem_sim_set_sort_mode(dem_sim* sim, int mode);
@@ -288,30 +290,35 @@ int dem_sim_set_sort_mode(dem_sim* sim, int mode);
  * stream is synchronized). */
 int dem_sim_mover_count(dem_sim* sim, uint32_t* count);
 /* The last re-sort's counts (exact once the stream is synchronized): movers
- * as dem_sim_mover_count, and listed, the particles the last in-place
- * re-sort moved to another slot or gave a new key (the movers plus the
- * particles their moves shift), whose state it staged and wrote back.  No
+ * as dem_sim_mover_count, and listed, the particles the last re-sort (in
+ * place or as a whole) moved to another slot or gave a new key: the movers
+ * plus the particles their moves shift, whose state an in-place one staged
+ * and wrote back.  No
  * counterpart in the reference (its steps always radix sort); for callers
  * that choose the sort mode themselves. */
 int dem_sim_resort_counts(dem_sim* sim, uint32_t* movers, uint32_t* listed);
 /* Kernel variants of the owned simulations of ctx (dem_sim_autotune sets
  * the fastest): DEM_STEP_FUSED runs collide and integrate as one kernel,
- * DEM_STEP_PREFETCH makes collide fetch each neighbour candidate one
+ * which takes contact lists whatever candidate mode is set (one candidate at
+ * a time with 64-bit addresses); as two, collide loads its candidates one at
+ * a time, DEM_STEP_PREFETCH makes it fetch each neighbour candidate one
  * iteration ahead, DEM_STEP_BATCH makes it load the first candidate of all
- * three neighbour rows at once (not together with PREFETCH; the fused
- * kernel loads one at a time instead).  Results are the same bit for bit. */
+ * three neighbour rows at once (not together with PREFETCH), and
+ * DEM_STEP_LIST takes contact lists.  Results are the same bit for bit. */
 #define DEM_STEP_FUSED 0x1
 #define DEM_STEP_PREFETCH 0x2
 #define DEM_STEP_BATCH 0x4
-/* Re-sorted steps of the split layout normally keep the state in its buffer
- * and move only the particles whose sorted slot changes (plus the cell
- * ranges around them); DEM_STEP_COPY makes them reorder the whole state
- * into the other buffer instead, as radix-sorted steps do.  Same results. */
+/* Re-sorted steps of large states normally keep the state in its buffer and
+ * move only the particles whose sorted slot changes (plus the cell ranges
+ * around them), those of small ones sort and reorder it into the other buffer
+ * in one kernel (dem_sim_set_sort_mode); DEM_STEP_COPY makes them reorder the
+ * whole state into the other buffer instead, as radix-sorted steps do.  Same
+ * results. */
 #define DEM_STEP_COPY 0x8
 /* Collide normally addresses its arrays by 32-bit offsets while they stay
  * under 4 GiB (up to 2^29 particles and 2^30 cells) and with 64-bit
- * addresses and one candidate at a time beyond; DEM_STEP_WIDE makes it use
- * the latter at every size.  Same results. */
+ * addresses beyond; DEM_STEP_WIDE makes it use the latter at every size.
+ * Same results. */
 #define DEM_STEP_WIDE 0x10
 /* DEM_STEP_LIST makes collide first mark, row by row, the candidates that
  * may touch (position and radius only) and then run the contact law over
