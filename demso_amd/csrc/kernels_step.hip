@@ -812,19 +812,20 @@ __device__ __forceinline__ void collide_particle(const StepConst& c, uint32_t i,
         // compiler's order)
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       }
-      // the window entry of candidate j of row y
-      auto entry = [&](int y, uint32_t j) { return j - w0[y] + (uint32_t)y * kWindow; };
-      // The candidates of the rows' parts (m of them from f, at most 31 a
-      // lane together) marked into w, left-aligned: the first one at bit 31.
+      // candidate j of row y has the window entry j - base[y]
+      const uint32_t base[3] = {w0[0], w0[1] - kWindow, w0[2] - 2u * kWindow};
+      // The candidates of three parts of rows (m of them from f, with
+      // window entries from f - b0, at most 31 each) marked into w, left-aligned: the first one at bit 31.
       // Lanes with shorter parts walk on (WaveWindow's slack) as long as any
       // has candidates: the loop is the wave's.
-      auto mark = [&](auto attract, const uint32_t (&f)[3], const uint32_t (&m)[3], uint32_t (&w)[3]) {
+      auto mark = [&](auto attract, const uint32_t (&f)[3], const uint32_t (&m)[3], const uint32_t (&b0)[3],
+                      uint32_t (&w)[3]) {
         const uint32_t L = max(m[0], max(m[1], m[2]));
         uint32_t k = 0;
         if (in_win) {
           const WindowEntry* e[3];
 #pragma unroll
-          for (int y = 0; y < 3; ++y) e[y] = win->at + (m[y] ? entry(y, f[y]) : (uint32_t)y * kWindow);
+          for (int y = 0; y < 3; ++y) e[y] = win->at + (m[y] ? f[y] - b0[y] : 0u);
           // two candidates a row at a time
           for (; __ballot(k < L); k += 2u) {
             WindowEntry b[3][2];
@@ -858,6 +859,13 @@ __device__ __forceinline__ void collide_particle(const StepConst& c, uint32_t i,
 #pragma unroll
         for (int y = 0; y < 3; ++y) w[y] = k ? w[y] << (32u - k) : 0u;
       };
+      auto clear_marks = [&](const uint32_t (&f)[3], const uint32_t (&m)[3], uint32_t (&w)[3]) {
+#pragma unroll
+        for (int y = 0; y < 3; ++y) {
+          w[y] &= ~(~0u >> m[y]);                         // past the part's end
+          w[y] &= ~(0x80000000u >> min(i - f[y], 31u));  // the particle itself (there is no 32nd candidate)
+        }
+      };
       // candidate j (entry e of the windows), as the law reads it
       auto listed = [&](uint32_t j, uint32_t e) {
         Cand b;
@@ -889,17 +897,12 @@ __device__ __forceinline__ void collide_particle(const StepConst& c, uint32_t i,
         using W = decltype(word);
         constexpr uint32_t kUp = 8u * sizeof(W) - 32u;
         uint32_t w[3] = {0u, 0u, 0u};
-        if (c.attract) mark(std::true_type{}, f, m, w);
-        else mark(std::false_type{}, f, m, w);
-#pragma unroll
-        for (int y = 0; y < 3; ++y) {
-          w[y] &= ~(~0u >> m[y]);                         // past the part's end
-          w[y] &= ~(0x80000000u >> min(i - f[y], 31u));  // the particle itself (there is no 32nd candidate)
-        }
+        if (c.attract) mark(std::true_type{}, f, m, base, w);
+        else mark(std::false_type{}, f, m, base, w);
+        clear_marks(f, m, w);
         return (W)w[0] << kUp | (W)w[1] << kUp >> m[0] | (W)w[2] << kUp >> (m[0] + m[1]);
       };
-      // The law over the marked candidates; returns how many cells had begun
-      // at the last one.
+      // The law over the marked candidates of the rows, which are the parts.
       auto contacts = [&](auto h, decltype(h) cells, const uint32_t (&f)[3], const uint32_t (&m)[3]) {
         using W = decltype(h);
         const uint32_t l1 = m[0], l2 = m[0] + m[1], f1 = f[1] - l1, f2 = f[2] - l2;
@@ -921,7 +924,6 @@ __device__ __forceinline__ void collide_particle(const StepConst& c, uint32_t i,
           }
           listed_pair(c, q, listed(j, e), cfx, cfy, moment, pres);
         }
-        return cell;
       };
       // every row in one pass
       auto whole = [&](auto word) {
@@ -941,7 +943,7 @@ __device__ __forceinline__ void collide_particle(const StepConst& c, uint32_t i,
             cells |= len[y] ? b | b >> (cut[y] & 0xFFFFu) | b >> (cut[y] >> 16) : (W)0;
             at += len[y];
           }
-          (void)contacts(h, cells, rs, len);
+          contacts(h, cells, rs, len);
           flush();
         }
       };
@@ -951,27 +953,68 @@ __device__ __forceinline__ void collide_particle(const StepConst& c, uint32_t i,
       } else if (__builtin_expect_with_probability(__ballot(total > 63u || L > 31u) == 0, 1, 0.9999)) {
         whole((uint64_t)0);
       } else {
-        // passes over 31 of each lane's candidates at a time
-        constexpr uint32_t kPass = 31u;
+        // Crowded neighbourhoods: a row's candidates up to 93 at a time, as
+        // three parts of equal length walked together: 300,304 dense discs
+        // with 72, 144, 324 and 900 candidates take 31, 37, 92 and 205 us a
+        // collide (38, 59, 205 and 539 in passes over 31 candidates of which
+        // two rows waited, 56, 73, 129 and 260 one at a time).  In a loop over
+        // the rows, whose ranges are found again: a rare path, kept from
+        // deciding how many registers the kernels take.
         if (!have_dyn) load_own_dyn();
         q.rden = 1.0 / q.den;
-        for (uint32_t done = 0; __ballot(done < total); done += kPass) {
-          uint32_t f[3], m[3], cells = 0, at = 0, before = 0;
+        float2 pc = q.p;
+        asm("" : "+v"(pc.x), "+v"(pc.y));
+        uint32_t tc = own.t;
+        if constexpr (kMulti && !kUni) asm("" : "+v"(tc));
+        const Instance in = kMulti ? c.inst[clamp_idx(c.mat[tc].inst, c.num_instances)] : c.inst0;
+        const int G0 = (int)in.grid[0], G1 = (int)in.grid[1];
+        int gx, gy;
+        grid_pos(in, pc, gx, gy);
+        if (clamp) clamp_cell(in, gx, gy);
+#pragma unroll 1
+        for (uint32_t y = 0; y < 3u; ++y) {
+          const int iy = gy + (int)y - 1;
+          const bool ok = !clamp || (iy >= 0 && iy < G1);
+          const uint32_t at1 = in.cell_base + (clamp ? (uint32_t)(ok ? iy : gy) : (uint32_t)iy & ((uint32_t)G1 - 1u)) * (uint32_t)G0 +
+                               (clamp ? (uint32_t)gx : (uint32_t)gx & ((uint32_t)G0 - 1u));
+          const uint32_t at0 = clamp && gx == 0 ? at1 : at1 - 1u, at2 = clamp && gx == G0 - 1 ? at1 : at1 + 1u;
+          const uint32_t s0 = ld<kO>(cell_start, at0), s1 = ld<kO>(cell_start, at1), s2 = ld<kO>(cell_start, at2);
+          const uint32_t e0 = s0 != kEmpty ? ld<kO>(cell_end, at0) : 0u, e1 = s1 != kEmpty ? ld<kO>(cell_end, at1) : 0u,
+                         e2 = s2 != kEmpty ? ld<kO>(cell_end, at2) : 0u;
+          const uint32_t last = ok ? min(max(max(e0, e1), e2), n) : 0u, first = min(min(min(s0, s1), s2), last);
+          const uint32_t count = last - first, c1 = max(e0, first) - first, c2 = max(e1 - first, c1);
+          const uint32_t wy = y == 0u ? w0[0] : (y == 1u ? w0[1] - kWindow : w0[2] - 2u * kWindow);
+          const uint32_t rows[3] = {wy, wy, wy};
+          uint32_t cell = 0u;
+          for (uint32_t done = 0; __ballot(done < count); done += 93u) {
+            const uint32_t left = done < count ? min(count - done, 93u) : 0u, part = (left + 2u) / 3u;
+            uint32_t f[3], m[3], w[3] = {0u, 0u, 0u};
 #pragma unroll
-          for (int y = 0; y < 3; ++y) {
-            const uint32_t lo = min(max(done, before) - before, len[y]);
-            f[y] = rs[y] + lo;
-            m[y] = min(max(done + kPass, before) - before, len[y]) - lo;
-            before += len[y];
-            // the cells that begin in this part
-            for (uint32_t b : {0u, cut[y] & 0xFFFFu, cut[y] >> 16})
-              cells |= b >= lo && b - lo < m[y] ? 0x80000000u >> (at + (b - lo)) : 0u;
-            at += m[y];
+            for (uint32_t s = 0; s < 3u; ++s) {
+              f[s] = first + done + s * part;
+              m[s] = left > s * part ? min(part, left - s * part) : 0u;
+            }
+            if (c.attract) mark(std::true_type{}, f, m, rows, w);
+            else mark(std::false_type{}, f, m, rows, w);
+            clear_marks(f, m, w);
+            uint32_t h0 = w[0], h1 = w[1], h2 = w[2];
+            while (h0 | h1 | h2) {
+              const bool in0 = h0 != 0u, in1 = h1 != 0u;
+              const uint32_t k = (uint32_t)__builtin_clz(in0 ? h0 : (in1 ? h1 : h2)), rest = ~(0x80000000u >> k);
+              h2 = in0 || in1 ? h2 : h2 & rest;
+              h1 = in0 ? h1 : h1 & rest;
+              h0 &= rest;
+              const uint32_t at = done + k + (in0 ? 0u : (in1 ? part : 2u * part));
+              const uint32_t in_cell = (at >= c1 ? 1u : 0u) + (at >= c2 ? 1u : 0u);
+              if (in_cell != cell) {
+                flush();
+                cell = in_cell;
+              }
+              listed_pair(c, q, listed(first + at, first + at - rows[0]), cfx, cfy, moment, pres);
+            }
           }
-          // (the next pass may go on with the last contact's cell)
-          if (contacts(marks(0u, f, m), cells, f, m) != (uint32_t)__popc(cells)) flush();
+          flush();
         }
-        flush();
       }
     } else if (kMode == kList) {
       by_cell = true;
@@ -1145,7 +1188,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMode == kL
 }
 
 // The list mode is held to 72 VGPRs, 7 waves a SIMD: what spills then is the
-// walk of crowded neighbourhoods in passes.  (8 waves, 64 VGPRs and 78 SGPRs,
+// walk of crowded neighbourhoods.  (8 waves, 64 VGPRs and 78 SGPRs,
 // spill on the common path: 131 us against 128 on the 4M dense pack, 159
 // against 143 on the 8.2M-disc ensemble.)
 // The one-material batched mode needed 65 VGPRs with 64-bit addresses; held to 64 (8

@@ -456,3 +456,26 @@ def test_mover_lists_equal_radix(gpu_ctx, name, fused):
     finally:
         a.close()
         b.close()
+
+
+@pytest.mark.parametrize("wrap", [False, True])
+@pytest.mark.parametrize("m", [66, 100, 282, 600, 1500])
+def test_crowded_rows(gpu_ctx, oracle, m, wrap):
+    """Rows of 22 to 500 candidates (one to six chunks of 93, in parts of up
+    to 31): a crowd inside the grid, one at its corner and one in a single
+    cell, whose rows above and below are empty; clamped and wrapping."""
+    from demso_amd import _lib
+
+    rng = np.random.default_rng(m)
+    s = sc.column_collapse(seed=m, cols=3 * m, n=3 * m, box=(0.352, 0.352))
+    s.instances = [sc.Instance(box=(0.352, 0.352), extent=(0.352, 0.352), grid=(32, 32))]
+    if wrap:
+        s.flags &= ~_lib.DEM_GRID_CLAMP
+    cell = 0.011
+    s.pos[:m] = (rng.uniform(0.05, 2.95, (m, 2)) + 8.0) * cell
+    s.pos[m:2 * m] = (rng.uniform(0.05, 2.95, (m, 2)) + (0.0 if not wrap else 29.0)) * cell
+    s.pos[2 * m:] = (rng.uniform(0.05, 0.95, (m, 2)) + np.array([20.0, 25.0])) * cell
+    s.radius[:] = rng.uniform(0.0005, 0.0055, s.n).astype(np.float32)
+    s.vel[:] = (rng.normal(size=s.vel.shape) * 0.2).astype(np.float32)
+    s.omega[:] = (rng.normal(size=s.n) * 30.0).astype(np.float32)
+    check_one_step(gpu_ctx, oracle, s)
