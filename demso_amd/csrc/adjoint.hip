@@ -45,9 +45,13 @@ constexpr int kParams = 4;  // kn, kt, cn, mu
 // state); beyond it, only the listed slots are saved and put back.
 constexpr uint32_t kScatterMax = 262144;
 // Up to this many particles the walk over the candidates and the reverse of
-// the pair law are one kernel (65,536 discs in contact: 8.7 us, against 4.8 +
-// 11.2 in two); beyond, where most of a settling state has no contact, two.
-constexpr uint32_t kMarkMin = 262144;
+// the pair law are one kernel, beyond two (a whole reversed step, one against
+// two: settled columns, whose discs all touch, of 300,304 discs 50 against 53
+// us, of 1,000,000 105 against 111, of 2,099,601 216 against 185; batches
+// without contacts of 522,733 77 against 77, of 2,162,994 244 against 184, of
+// 4,732,842 502 against 355.  A column without contacts gains earlier, 168
+// against 117 at 1,000,000).
+constexpr uint32_t kMarkMin = 1048576;
 
 // Threads a workgroup of every kernel here (a constant: a kernel that asks the
 // runtime begins with a vector load and a wait for it).

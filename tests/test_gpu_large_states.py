@@ -7,6 +7,7 @@ from demso_amd import api
 from demso_amd import scene as sc
 from helpers import batch_of, bits_equal, mixed_pack
 from test_gpu_adjoint import gpu_grads
+from test_gpu_kernel_edges import packed_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -48,6 +49,29 @@ def test_checkpoint_interval_of_large_states(gpu_ctx, fused):
         assert bits_equal(finalk, final), K
         assert bits_equal(gpk, gp) and bits_equal(gvk, gv), K
         assert np.allclose(park, par, rtol=0, atol=1e-9 * np.abs(par).max(axis=0)), K
+
+
+def test_adjoint_past_a_million_discs_lists_contacts(gpu_ctx):
+    """Past 1,048,576 discs the adjoint lists the discs with contacts first: a
+    batch of copies of one system (free, touching and heaped discs; rows of
+    more than 64 candidates) against the system alone, which takes the
+    one-kernel path: gradients of the state bit for bit, of the parameters to
+    the order of their sums (some 4,000 terms)."""
+    one = packed_rows(3001, seed=9)
+    one.pos[1000:2000, 0] *= np.float32(1.02)
+    one.pos[1000:2000, 1] += np.float32(0.2)  # (free discs)
+    copies = 350
+    many = batch_of(one, copies)
+    assert many.n > 1048576
+    rng = np.random.default_rng(0)
+    W, V = rng.normal(size=(one.n, 2)), rng.normal(size=(one.n, 2))
+    (gp1, gv1, par1), _ = gpu_grads(gpu_ctx, one, 3, W, V, K=2)
+    (gpm, gvm, parm), _ = gpu_grads(gpu_ctx, many, 3, np.tile(W, (copies, 1)), np.tile(V, (copies, 1)), K=2)
+    assert np.count_nonzero(par1) >= 3
+    for k in (0, 1, 171, copies - 1):
+        at = slice(k * one.n, (k + 1) * one.n)
+        assert bits_equal(gpm[at], gp1) and bits_equal(gvm[at], gv1), k
+    assert np.all(np.abs(parm - par1) <= 1e-9 * np.maximum(np.abs(par1), 1e-3 * np.abs(par1).max()))
 
 
 def squeezed_batch(counts, seed):
