@@ -1043,16 +1043,17 @@ __global__ __launch_bounds__(kPlaceThreads) void k_resort_whole(ShiftState from,
     if (m) {
       if (lane < own) s.raw[ahead + lane] = raw;
       __syncthreads();
-      if (lane < own) {
+      if (tid < m) {
+        const uint64_t mine = s.raw[tid];
         uint32_t by_pair = 0, by_pos = 0;  // the positions differ, so both ranks are unique
         for (uint32_t j = 0; j < m; ++j) {
           const uint64_t y = s.raw[j];
-          by_pair += y < raw ? 1u : 0u;
-          by_pos += (uint32_t)y < (uint32_t)raw ? 1u : 0u;
+          by_pair += y < mine ? 1u : 0u;
+          by_pos += (uint32_t)y < (uint32_t)mine ? 1u : 0u;
         }
-        s.pair[by_pair] = raw;
-        s.pos[by_pos] = (uint32_t)raw;
-        s.key[by_pos] = (uint32_t)(raw >> 32);
+        s.pair[by_pair] = mine;
+        s.pos[by_pos] = (uint32_t)mine;
+        s.key[by_pos] = (uint32_t)(mine >> 32);
       }
       __syncthreads();
     }
