@@ -62,7 +62,8 @@ METRIC = "particle-steps/s @4M discs; batched-ensemble and fwd+adjoint vs plain 
 # Fused (collide + integrate in one kernel, in place): it reads pos 8, vel 8,
 #   omega 4, theta 4, radius 4, type 4 and writes acc 8, alpha 4, pressure 4,
 #   pos 8, vel 8, theta 4, omega 4 (+ 8 per cell), reported under collide.
-# Whole (up to 262,144 particles; the fused kernel or the two of in place):
+# Whole (up to 262,144 particles, 64 cells a particle and 2^21 cells; the fused
+#   kernel or the two of in place):
 #   re-sort and reorder in one kernel, reported under sort: R key 4, pos 8,
 #   vel 8, theta 4, omega 4, id 4, type 4, radius 4, W the same, loc 4 and
 #   index 4, + the next cellStart 4 per cell.
